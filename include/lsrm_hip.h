@@ -200,6 +200,17 @@ int lsrm_sel_attn_validate(const int32_t* topk_idx, int64_t hkv, int64_t n_q,
                            const int32_t* cu_seqlens_k, int64_t batch,
                            int64_t n_k, int32_t* flags, void* stream);
 
+/* lsrm_sel_attn_validate and the count of row changes in one pass over the
+ * selection: info[0] = the metadata bits, info[1] = number of (kv head,
+ * query i > 0) whose row differs from query i - 1's (entries compared as
+ * they are), from which the caller decides between plan kinds. */
+int lsrm_sel_attn_inspect(const int32_t* topk_idx, int64_t hkv, int64_t n_q,
+                          int64_t topk, const int32_t* cu_seqblocks,
+                          const int32_t* cu_block_tokens, int64_t n_blocks,
+                          const int32_t* cu_seqlens_q,
+                          const int32_t* cu_seqlens_k, int64_t batch,
+                          int64_t n_k, int64_t* info, void* stream);
+
 /* ------------------------------------------------------------------------
  * Selected-block attention, forward.
  *   q [n_q, hq, head_dim], k/v [n_k, hkv, head_dim] of dtype (F16 or BF16)

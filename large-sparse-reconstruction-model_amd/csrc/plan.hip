@@ -215,13 +215,26 @@ __global__ __launch_bounds__(256) void breaks_vec_kernel(
   if (live) brk[(int64_t)h * nq + i] = (i == 0 || start || diff) ? 1 : 0;
 }
 
+// Row flags from lane flags where P neighbouring lanes hold one row: bit r * P
+// is set when any bit of lanes r * P .. r * P + P - 1 is (scalar work).
+template <int P>
+constexpr uint64_t ROW_LSB = ROW_LSB<2 * P> * (1ull | (1ull << P));
+template <>
+constexpr uint64_t ROW_LSB<64> = 1ull;
+template <int P>
+__device__ inline uint64_t row_or(uint64_t m) {
+#pragma unroll
+  for (int o = 1; o < P; o <<= 1) m |= m >> o;
+  return m & ROW_LSB<P>;
+}
+
 // Same for rows of P 16-byte pieces (k = 4 P), P a power of two <= 64: lane
-// (row i, piece p) holds piece p of row i, so a wave reads 64 / P whole rows
-// as one contiguous run per load; piece p of row i - 1 is the lane P below
-// (the last row of the previous group, or a load for the wave's first row),
-// and the P lanes of a row OR their differences.  A wave covers BRK_G such
-// groups with all their loads in flight, and looks its batch element up once
-// when its rows lie inside one (else row by row).
+// (row i, piece p) holds piece p of row i and of row i - 1, so a wave reads
+// 64 / P whole rows as one contiguous run per load (the second read of a line
+// is served by the cache), and the P lanes of a row are combined in scalar
+// registers.  A wave covers BRK_G such groups with all their loads in flight,
+// and looks its batch element up once when its rows lie inside one (else row
+// by row).
 constexpr int BRK_G = 8;
 template <int P>
 __global__ __launch_bounds__(256) void breaks_rows_kernel(
@@ -236,14 +249,13 @@ __global__ __launch_bounds__(256) void breaks_rows_kernel(
   if (i0 >= nq) return;  // whole waves
   const int p = lane % P, rl = lane / P;
   const u32x4* rows = reinterpret_cast<const u32x4*>(topk + (int64_t)h * nq * (4 * P));
-  u32x4 cur[BRK_G];
+  u32x4 cur[BRK_G], prev[BRK_G];
 #pragma unroll
   for (int g = 0; g < BRK_G; ++g) {
-    const int64_t i = i0 + g * RPW + rl;
-    cur[g] = rows[(i < nq ? i : nq - 1) * P + p];
+    const int64_t i = i0 + g * RPW + rl < nq ? i0 + g * RPW + rl : nq - 1;
+    cur[g] = rows[i * P + p];
+    prev[g] = rows[(i > 0 ? i - 1 : 0) * P + p];
   }
-  u32x4 first_prev = cur[0];
-  if (lane < P && i0 > 0) first_prev = rows[(i0 - 1) * P + p];
   const int64_t i_last = i0 + RPW * BRK_G - 1 < nq ? i0 + RPW * BRK_G - 1 : nq - 1;
   int b0 = 0, bs0 = 0, nbb0 = 0;
   bool st0 = true;
@@ -253,27 +265,18 @@ __global__ __launch_bounds__(256) void breaks_rows_kernel(
 #pragma unroll
   for (int g = 0; g < BRK_G; ++g) {
     const int64_t i = i0 + g * RPW + rl;
-    u32x4 prev;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int up = __shfl_up((int)cur[g][e], P);
-      const int last = g > 0 ? __shfl((int)cur[g > 0 ? g - 1 : 0][e], (RPW - 1) * P + p)
-                             : (int)first_prev[e];
-      prev[e] = (uint32_t)(lane >= P ? up : last);
-    }
     int nbb = nbb0;
     bool start = i == qs0;
     if (!one && i < nq) {
       int b, bs;
       query_batch(cu_q, batch, cu_sb, i, &b, &bs, &nbb, &start);
     }
-    int diff = 0;
+    bool diff = i == 0 || start;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      diff |= norm_entry((int)cur[g][e], nbb) != norm_entry((int)prev[e], nbb) ? 1 : 0;
-#pragma unroll
-    for (int o = 1; o < P; o <<= 1) diff |= __shfl_xor(diff, o);
-    if (i < nq && p == 0) brk[(int64_t)h * nq + i] = (i == 0 || start || diff) ? 1 : 0;
+      diff |= norm_entry((int)cur[g][e], nbb) != norm_entry((int)prev[g][e], nbb);
+    const uint64_t brks = row_or<P>(__ballot(diff));
+    if (i < nq && p == 0) brk[(int64_t)h * nq + i] = (uint8_t)((brks >> lane) & 1);
   }
 }
 
@@ -1340,30 +1343,154 @@ __global__ __launch_bounds__(256) void validate_meta_kernel(
   if (f) atomicOr(flags, f);
 }
 
-__global__ __launch_bounds__(256) void validate_topk_kernel(
+// Row checks of a selection in one read of it: the metadata bits of every row
+// (LSRM_META_TOPK_*) and, with `changes`, the number of rows whose entries
+// differ from the previous row's of the same head (raw entries, whatever the
+// batch element: what a host comparison of neighbouring rows counts).
+//
+// One row per thread, any k.
+__global__ __launch_bounds__(256) void inspect_rows_kernel(
     const int32_t* __restrict__ topk, int64_t nq, int k,
     const int32_t* __restrict__ cu_q, int64_t batch,
-    const int32_t* __restrict__ cu_sb, int32_t* flags) {
+    const int32_t* __restrict__ cu_sb, int32_t* flags,
+    unsigned long long* __restrict__ changes) {
+  __shared__ int s_changes, s_flags;
   const int h = blockIdx.y;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nq) return;
-  int b, bs, nbb;
-  bool start;
-  query_batch(cu_q, batch, cu_sb, i, &b, &bs, &nbb, &start);
-  const int32_t* row = topk + ((int64_t)h * nq + i) * k;
-  bool seen_invalid = false, any = false;
-  int f = 0;
-  for (int j = 0; j < k; ++j) {
-    const bool valid = norm_entry(row[j], nbb) >= 0;
-    if (valid) {
-      any = true;
-      if (seen_invalid) f |= LSRM_META_TOPK_NOT_PREFIX;
-    } else {
-      seen_invalid = true;
+  if (threadIdx.x == 0) s_changes = s_flags = 0;
+  __syncthreads();
+  if (i < nq) {
+    int b, bs, nbb;
+    bool start;
+    query_batch(cu_q, batch, cu_sb, i, &b, &bs, &nbb, &start);
+    const int32_t* row = topk + ((int64_t)h * nq + i) * k;
+    const int32_t* up = i > 0 ? row - k : row;
+    bool seen_invalid = false, any = false, diff = false;
+    int f = 0;
+    for (int j = 0; j < k; ++j) {
+      const int v = row[j];
+      const bool valid = norm_entry(v, nbb) >= 0;
+      if (valid) {
+        any = true;
+        if (seen_invalid) f |= LSRM_META_TOPK_NOT_PREFIX;
+      } else {
+        seen_invalid = true;
+      }
+      if (changes) diff |= v != up[j];
+    }
+    if (!any) f |= LSRM_META_TOPK_EMPTY_ROW;
+    if (f) atomicOr(&s_flags, f);
+    if (diff) atomicAdd(&s_changes, 1);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0 && s_flags) atomicOr(flags, s_flags);
+  if (changes && threadIdx.x == 0 && s_changes)
+    atomicAdd(changes, (unsigned long long)s_changes);
+}
+
+// The same for rows of P 16-byte pieces (k = 4 P, P a power of two <= 64,
+// 16-byte-aligned rows), in the lane layout of breaks_rows_kernel: bound by
+// the one read of the rows.  One row per thread fetches a line again for each
+// 16-byte column of a wave's 64 rows: 268 MB of top-32 rows took 1194 us
+// without the count of changed rows (torch: another 485 us), this form takes
+// 75 us with it (3.6 TB/s); 201 MB of top-16 rows 112 + 370 -> 56 us.
+template <int P>
+__global__ __launch_bounds__(256) void inspect_pieces_kernel(
+    const int32_t* __restrict__ topk, int64_t nq, const int32_t* __restrict__ cu_q,
+    int64_t batch, const int32_t* __restrict__ cu_sb, int32_t* flags,
+    unsigned long long* __restrict__ changes) {
+  static_assert(P >= 1 && P <= 64 && (P & (P - 1)) == 0, "rows must tile a wave");
+  constexpr int RPW = 64 / P;  // rows per group
+  __shared__ int s_changes, s_flags;
+  const int h = blockIdx.y;
+  const int lane = threadIdx.x & 63;
+  const int p = lane % P, rl = lane / P;
+  const u32x4* rows = reinterpret_cast<const u32x4*>(topk + (int64_t)h * nq * (4 * P));
+  if (threadIdx.x == 0) s_changes = s_flags = 0;
+  __syncthreads();
+  int f = 0, n_diff = 0;
+  const int64_t step = (int64_t)gridDim.x * (blockDim.x / 64) * (RPW * BRK_G);
+  for (int64_t i0 =
+           ((int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)) * (RPW * BRK_G);
+       i0 < nq; i0 += step) {  // whole waves
+    // the row and the row above it (the same lines, served by the cache)
+    u32x4 cur[BRK_G], prev[BRK_G];
+#pragma unroll
+    for (int g = 0; g < BRK_G; ++g) {
+      const int64_t i = i0 + g * RPW + rl < nq ? i0 + g * RPW + rl : nq - 1;
+      cur[g] = rows[i * P + p];
+      prev[g] = rows[(i > 0 ? i - 1 : 0) * P + p];  // row 0 compares with itself
+    }
+    const int64_t i_last = i0 + RPW * BRK_G - 1 < nq ? i0 + RPW * BRK_G - 1 : nq - 1;
+    int b0 = 0, bs0 = 0, nbb0 = 0;
+    bool st0 = true;
+    query_batch(cu_q, batch, cu_sb, i0, &b0, &bs0, &nbb0, &st0);
+    const bool one = b0 >= 0 && i_last < (int64_t)cu_q[b0 + 1];
+#pragma unroll
+    for (int g = 0; g < BRK_G; ++g) {
+      const int64_t i = i0 + g * RPW + rl;
+      int nbb = nbb0;
+      if (!one && i < nq) {
+        int b, bs;
+        bool start;
+        query_batch(cu_q, batch, cu_sb, i, &b, &bs, &nbb, &start);
+      }
+      const bool live = i < nq;  // a lane past the rows raises no flag
+      bool diff = false, any = !live, valid[4], gap = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        diff |= cur[g][e] != prev[g][e];
+        valid[e] = live && norm_entry((int)cur[g][e], nbb) >= 0;
+        any |= valid[e];
+        if (e > 0) gap |= valid[e] && !valid[e - 1];
+      }
+      n_diff += __popcll(row_or<P>(__ballot(live && diff)));
+      if (row_or<P>(__ballot(any)) != ROW_LSB<P>) f |= LSRM_META_TOPK_EMPTY_ROW;
+      // an entry 0 of a piece follows entry 3 of the row's piece before it
+      const uint64_t before = (__ballot(valid[3]) << 1) | ROW_LSB<P>;
+      if (__ballot(gap) | (__ballot(valid[0]) & ~before)) f |= LSRM_META_TOPK_NOT_PREFIX;
     }
   }
-  if (!any) f |= LSRM_META_TOPK_EMPTY_ROW;
-  if (f) atomicOr(flags, f);
+  if (lane == 0 && f) atomicOr(&s_flags, f);
+  if (lane == 0 && n_diff) atomicAdd(&s_changes, n_diff);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_flags) atomicOr(flags, s_flags);
+  if (changes && threadIdx.x == 0 && s_changes)
+    atomicAdd(changes, (unsigned long long)s_changes);
+}
+
+constexpr int64_t INSPECT_GROUPS = 1536;  // six workgroups per CU
+
+// Launches the row checks: the piece form where the rows allow it (as
+// build_tile_plan's row comparison), else one row per thread.
+int launch_inspect_rows(const int32_t* topk, int64_t hkv, int64_t nq, int64_t topk_n,
+                        const int32_t* cu_q, int64_t batch, const int32_t* cu_sb,
+                        int32_t* flags, unsigned long long* changes, hipStream_t st) {
+  if (nq <= 0) return LSRM_OK;
+  const int64_t pieces = topk_n / 4;
+  if (topk_n % 4 == 0 && ((uintptr_t)topk % 16) == 0 && pieces <= 64 &&
+      (pieces & (pieces - 1)) == 0) {
+    // A bounded grid: every workgroup that saw a change adds to one word
+    // (about 6 ns each: 8192 of them took half of the kernel's time).
+    const int64_t need = ceil_div(ceil_div(nq, (64 / pieces) * BRK_G), 4);
+    const dim3 grid((unsigned)std::min<int64_t>(need, ceil_div(INSPECT_GROUPS, hkv)),
+                    (unsigned)hkv);
+#define LSRM_INSPECT(P)                                                                   \
+  case P:                                                                                 \
+    hipLaunchKernelGGL(inspect_pieces_kernel<P>, grid, dim3(256), 0, st, topk, nq, cu_q,  \
+                       batch, cu_sb, flags, changes);                                     \
+    break;
+    switch (pieces) {
+      LSRM_INSPECT(1) LSRM_INSPECT(2) LSRM_INSPECT(4) LSRM_INSPECT(8)
+      LSRM_INSPECT(16) LSRM_INSPECT(32) LSRM_INSPECT(64)
+    }
+#undef LSRM_INSPECT
+  } else {
+    hipLaunchKernelGGL(inspect_rows_kernel, dim3(ceil_div(nq, 256), (unsigned)hkv), dim3(256), 0,
+                       st, topk, nq, (int)topk_n, cu_q, batch, cu_sb, flags, changes);
+  }
+  LSRM_CHECK_LAUNCH();
+  return LSRM_OK;
 }
 
 // ----------------------------------------------------------- block ids --
@@ -1387,31 +1514,50 @@ __global__ __launch_bounds__(256) void block_ids_kernel(
 
 using namespace lsrm;
 
-extern "C" int lsrm_sel_attn_validate(
-    const int32_t* topk_idx, int64_t hkv, int64_t n_q, int64_t topk,
-    const int32_t* cu_seqblocks, const int32_t* cu_block_tokens,
-    int64_t n_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
-    int64_t batch, int64_t n_k, int32_t* flags, void* stream) {
+namespace {
+
+// lsrm_sel_attn_validate, and with `changes` lsrm_sel_attn_inspect.
+int inspect_impl(const int32_t* topk_idx, int64_t hkv, int64_t n_q, int64_t topk,
+                 const int32_t* cu_seqblocks, const int32_t* cu_block_tokens, int64_t n_blocks,
+                 const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, int64_t batch,
+                 int64_t n_k, int32_t* flags, unsigned long long* changes, hipStream_t st) {
   if (hkv <= 0 || n_q < 0 || topk <= 0 || n_blocks < 0 || batch <= 0 ||
       n_k < 0 || !flags || !cu_seqblocks || !cu_block_tokens || !cu_seqlens_q ||
       !cu_seqlens_k || (n_q > 0 && !topk_idx))
     return LSRM_ERR_INVALID_ARG;
-  hipStream_t st = (hipStream_t)stream;
-  int rc = launch_zero_i32(flags, 1, st);
+  // the count's word follows the flags' in lsrm_sel_attn_inspect's result
+  int rc = launch_zero_i32(flags, changes ? 4 : 1, st);
   if (rc) return rc;
   const int64_t m = n_blocks > batch ? n_blocks : batch;
   hipLaunchKernelGGL(validate_meta_kernel, dim3(ceil_div(m > 0 ? m : 1, 256)),
                      dim3(256), 0, st, cu_seqblocks, cu_block_tokens, n_blocks,
                      cu_seqlens_q, cu_seqlens_k, batch, n_q, n_k, flags);
   LSRM_CHECK_LAUNCH();
-  if (n_q > 0) {
-    dim3 grid(ceil_div(n_q, 256), (unsigned)hkv);
-    hipLaunchKernelGGL(validate_topk_kernel, grid, dim3(256), 0, st, topk_idx,
-                       n_q, (int)topk, cu_seqlens_q, batch, cu_seqblocks,
-                       flags);
-    LSRM_CHECK_LAUNCH();
-  }
-  return LSRM_OK;
+  return launch_inspect_rows(topk_idx, hkv, n_q, topk, cu_seqlens_q, batch, cu_seqblocks, flags,
+                             changes, st);
+}
+
+}  // namespace
+
+extern "C" int lsrm_sel_attn_validate(
+    const int32_t* topk_idx, int64_t hkv, int64_t n_q, int64_t topk,
+    const int32_t* cu_seqblocks, const int32_t* cu_block_tokens,
+    int64_t n_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    int64_t batch, int64_t n_k, int32_t* flags, void* stream) {
+  return inspect_impl(topk_idx, hkv, n_q, topk, cu_seqblocks, cu_block_tokens, n_blocks,
+                      cu_seqlens_q, cu_seqlens_k, batch, n_k, flags, nullptr,
+                      (hipStream_t)stream);
+}
+
+extern "C" int lsrm_sel_attn_inspect(
+    const int32_t* topk_idx, int64_t hkv, int64_t n_q, int64_t topk,
+    const int32_t* cu_seqblocks, const int32_t* cu_block_tokens,
+    int64_t n_blocks, const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k,
+    int64_t batch, int64_t n_k, int64_t* info, void* stream) {
+  if (!info) return LSRM_ERR_INVALID_ARG;
+  return inspect_impl(topk_idx, hkv, n_q, topk, cu_seqblocks, cu_block_tokens, n_blocks,
+                      cu_seqlens_q, cu_seqlens_k, batch, n_k, reinterpret_cast<int32_t*>(info),
+                      reinterpret_cast<unsigned long long*>(info + 1), (hipStream_t)stream);
 }
 
 extern "C" size_t lsrm_reverse_query_map_workspace_size(int64_t n_q,

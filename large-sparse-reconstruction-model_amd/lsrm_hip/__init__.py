@@ -63,6 +63,8 @@ _SIGNATURES = {
     ),
     "lsrm_sel_attn_validate": (
         _I, [_P, _I64, _I64, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P]),
+    "lsrm_sel_attn_inspect": (
+        _I, [_P, _I64, _I64, _I64, _P, _P, _I64, _P, _P, _I64, _I64, _P, _P]),
     "lsrm_sel_attn_workspace_size": (_SZ, [_I64, _I64, _I64, _I64, _I64, _I64, _I]),
     "lsrm_sel_attn_fwd": (
         _I,
@@ -366,6 +368,25 @@ def validate(topk_idx: torch.Tensor, cu_seqblocks: torch.Tensor,
             _ptr(_i32(cu_seqlens_q)), _ptr(_i32(cu_seqlens_k)), cu_seqlens_q.numel() - 1,
             n_k, _ptr(flags), _stream(dev)), "lsrm_sel_attn_validate")
     return int(flags.item())
+
+
+def inspect_selection(topk_idx: torch.Tensor, cu_seqblocks: torch.Tensor,
+                      cu_block_tokens: torch.Tensor, cu_seqlens_q: torch.Tensor,
+                      cu_seqlens_k: torch.Tensor, n_k: int):
+    """validate and the number of (kv head, query) rows that differ from the
+    row before them, in one read of the selection and one host read."""
+    dev = _dev_check(topk_idx, cu_seqblocks, cu_block_tokens, cu_seqlens_q, cu_seqlens_k)
+    topk_idx = _i32(topk_idx)
+    hkv, nq, k = topk_idx.shape
+    info = torch.empty(2, dtype=torch.int64, device=dev)
+    with torch.cuda.device(dev):
+        _check(lib().lsrm_sel_attn_inspect(
+            _ptr(topk_idx), hkv, nq, k, _ptr(_i32(cu_seqblocks)),
+            _ptr(_i32(cu_block_tokens)), cu_block_tokens.numel() - 1,
+            _ptr(_i32(cu_seqlens_q)), _ptr(_i32(cu_seqlens_k)), cu_seqlens_q.numel() - 1,
+            n_k, _ptr(info), _stream(dev)), "lsrm_sel_attn_inspect")
+    bits, changes = info.tolist()
+    return bits, changes
 
 
 def describe_meta_error(bits: int) -> str:

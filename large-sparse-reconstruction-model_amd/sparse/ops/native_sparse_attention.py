@@ -52,25 +52,37 @@ def set_key_centric(enabled) -> None:
     _key_centric = enabled if enabled == "auto" else bool(enabled)
 
 
-def _use_key_centric(q, k, topk_idx) -> bool:
-    """The key-centric choice for this selection (see set_key_centric)."""
+def _counts_row_changes(topk_idx) -> bool:
+    """Whether the key-centric choice reads this selection's rows.  Under graph
+    capture or compilation the count cannot be read back (and a key-centric
+    plan is not built under capture): the grouped-tile plan."""
+    return _key_centric == "auto" and topk_idx.shape[1] >= 2 and \
+        not torch.compiler.is_compiling() and \
+        not (topk_idx.is_cuda and torch.cuda.is_current_stream_capturing())
+
+
+def _use_key_centric(q, k, topk_idx, changes=None) -> bool:
+    """The key-centric choice for this selection (see set_key_centric).
+    changes: the number of rows that differ from the row before them, when
+    it has been counted."""
     if _key_centric != "auto":
         return bool(_key_centric)
-    # Under graph capture or compilation the count cannot be read back (and a
-    # key-centric plan is not built under capture): the grouped-tile plan.
-    if topk_idx.shape[1] < 2 or torch.compiler.is_compiling() or \
-            (topk_idx.is_cuda and torch.cuda.is_current_stream_capturing()):
+    if not _counts_row_changes(topk_idx):
         return False
     # The plan groups runs shorter than a quarter of a 128-row tile's
     # queries; the key-centric part pays off when such runs dominate.
     short = max(1, (128 // (q.shape[1] // k.shape[1])) // 4)
-    changes = int((topk_idx[:, 1:] != topk_idx[:, :-1]).any(-1).sum())
+    if changes is None:
+        changes = int((topk_idx[:, 1:] != topk_idx[:, :-1]).any(-1).sum())
     runs = changes + topk_idx.shape[0]
     return runs * short > topk_idx.shape[0] * topk_idx.shape[1]
 
 
 def _check_meta(q, k, topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlens_q,
-                cu_seqlens_k) -> None:
+                cu_seqlens_k):
+    """Checks the metadata; returns the selection's row changes when the
+    key-centric choice needs them (one device pass and one host read serve
+    both), else None."""
     if topk_idx.dim() != 3 or topk_idx.shape[0] != k.shape[1] or topk_idx.shape[1] != q.shape[0]:
         raise ValueError(
             f"topk_idx must be [num_kv_heads, total_q, topk]; got {tuple(topk_idx.shape)} for "
@@ -79,13 +91,20 @@ def _check_meta(q, k, topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlen
         raise ValueError("num_q_heads must be a multiple of num_kv_heads")
     if cu_seqlens_q.numel() != cu_seqblocks.numel():
         raise ValueError("cu_seqlens_q and cu_seqblocks must both have batch_size + 1 entries")
-    if not _validate:
-        return
-    bits = _hip.validate(topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlens_q,
-                         cu_seqlens_k, k.shape[0])
+    bits, changes = 0, None
+    if _counts_row_changes(topk_idx):
+        # the metadata bits count only with validation on, and then alone
+        # cu_seqlens_k is read
+        bits, changes = _hip.inspect_selection(
+            topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlens_q,
+            cu_seqlens_k if _validate else cu_seqlens_q, k.shape[0])
+    elif _validate:
+        bits = _hip.validate(topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlens_q,
+                             cu_seqlens_k, k.shape[0])
     bits &= ~_hip.META_TOPK_EMPTY_ROW   # empty rows are defined: output 0
-    if bits:
+    if _validate and bits:
         raise ValueError(f"invalid sparse-attention metadata: {_hip.describe_meta_error(bits)}")
+    return changes
 
 
 class NSA(torch.autograd.Function):
@@ -112,9 +131,9 @@ class NSA(torch.autograd.Function):
         if softmax_scale is None:
             softmax_scale = 1.0 / math.sqrt(q.shape[-1])
 
-        _check_meta(q, k, topk_idx, cu_seqblocks, cu_block_include_tokens, cu_seqlens_q,
-                    cu_seqlens_k)
-        key_centric = _use_key_centric(q, k, topk_idx)
+        changes = _check_meta(q, k, topk_idx, cu_seqblocks, cu_block_include_tokens,
+                              cu_seqlens_q, cu_seqlens_k)
+        key_centric = _use_key_centric(q, k, topk_idx, changes)
         if any(t.requires_grad for t in (q, k, v)) and q.is_cuda and q.shape[0] > 0 and \
                 not torch.compiler.is_compiling():
             # One plan per selection: built here with its backward part, it
