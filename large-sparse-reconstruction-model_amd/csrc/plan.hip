@@ -6,11 +6,9 @@
 // _scatter_queries_kernel / host-looped segmented sort
 // (sparse/ops/triton_native_sparse_attention_impl_kvcentric.py:494-684),
 // all on the device and without host synchronisation: for rows that are
-// queries, one stable radix sort of (head * n_blocks + block, listing) pairs
-// generated in (head, query, slot) order; for rows that are run tiles,
-// count -> scan -> atomic scatter -> per-segment sort.
+// queries, a stable counting sort over chunks of queries; for rows that are
+// run tiles, count -> scan -> atomic scatter -> per-segment sort.
 #include <algorithm>
-#include <rocprim/device/device_radix_sort.hpp>
 
 #include "plan.h"
 
@@ -573,24 +571,15 @@ int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
 
 // --------------------------------------------------------- reverse map --
 
-// Row source: row r of head h reads the selection of query `query(h, r)`;
-// rows that `skip` are not entered.
+// Rows that are run tiles: row r of head h reads the selection of its tile's
+// first query.
 struct RowSrc {
-  const int2* tiles;      // null: rows are queries
-  const int32_t* count;   // rows per head (tiles) or null
+  const int2* tiles;
+  const int32_t* count;  // tiles per head
   int64_t nq;
-  const uint8_t* only;    // rows are queries: [hkv, nq] mask, or null (all)
-  int enc;                // > 0: a listing stores row * enc + slot (enc = topk)
-  __device__ int64_t n_rows(int h) const {
-    return tiles ? (int64_t)count[h] : nq;
-  }
-  // Range of the stored values (the counting sort's key range).
-  __device__ int64_t n_values(int h) const { return n_rows(h) * (enc > 0 ? enc : 1); }
+  __device__ int64_t n_rows(int h) const { return (int64_t)count[h]; }
   __device__ int64_t query(int h, int64_t r) const {
-    return tiles ? (int64_t)tiles[(int64_t)h * nq + r].x : r;
-  }
-  __device__ bool skip(int h, int64_t r) const {
-    return !tiles && only && !only[(int64_t)h * nq + r];
+    return (int64_t)tiles[(int64_t)h * nq + r].x;
   }
 };
 
@@ -601,7 +590,7 @@ __global__ __launch_bounds__(256) void rev_count_kernel(
     int32_t* __restrict__ counts) {
   const int h = blockIdx.y;
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows.n_rows(h) || rows.skip(h, r)) return;
+  if (r >= rows.n_rows(h)) return;
   const int64_t q = rows.query(h, r);
   int b, bs, nbb;
   bool start;
@@ -622,7 +611,7 @@ __global__ __launch_bounds__(256) void rev_scatter_kernel(
     int32_t* __restrict__ rev, int64_t cap) {
   const int h = blockIdx.y;
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows.n_rows(h) || rows.skip(h, r)) return;
+  if (r >= rows.n_rows(h)) return;
   const int64_t q = rows.query(h, r);
   int b, bs, nbb;
   bool start;
@@ -635,7 +624,7 @@ __global__ __launch_bounds__(256) void rev_scatter_kernel(
       const int64_t pos =
           cu_rev[(int64_t)h * (nb + 1) + c] +
           atomicAdd(&fill[(int64_t)h * nb + c], 1);
-      if (pos < cap) rev[(int64_t)h * cap + pos] = (int32_t)(rows.enc > 0 ? r * rows.enc + j : r);
+      if (pos < cap) rev[(int64_t)h * cap + pos] = (int32_t)r;
     }
   }
 }
@@ -660,7 +649,7 @@ __global__ __launch_bounds__(256) void rev_count_lds_kernel(
   for (int i = threadIdx.x; i < nb; i += blockDim.x) hist[i] = 0;
   __syncthreads();
   const int64_t r = r0 + threadIdx.x;
-  if (r < rows.n_rows(h) && !rows.skip(h, r)) {
+  if (r < rows.n_rows(h)) {
     const int64_t q = rows.query(h, r);
     int b, bs, nbb;
     bool start;
@@ -693,7 +682,7 @@ __global__ __launch_bounds__(256) void rev_scatter_lds_kernel(
   }
   __syncthreads();
   const int64_t r = r0 + threadIdx.x;
-  const bool on = r < rows.n_rows(h) && !rows.skip(h, r);
+  const bool on = r < rows.n_rows(h);
   int bs = 0, nbb = 0;
   const int32_t* row = topk;
   if (on) {
@@ -717,7 +706,7 @@ __global__ __launch_bounds__(256) void rev_scatter_lds_kernel(
       if (v >= 0 && v < nbb && (int64_t)bs + v < nb) {
         const int64_t c = bs + v;
         const int64_t pos = cu_rev[(int64_t)h * (nb + 1) + c] + cnt[c] + atomicAdd(&local[c], 1);
-        if (pos < cap) rev[(int64_t)h * cap + pos] = (int32_t)(rows.enc > 0 ? r * rows.enc + j : r);
+        if (pos < cap) rev[(int64_t)h * cap + pos] = (int32_t)r;
       }
     }
   }
@@ -784,10 +773,9 @@ __global__ __launch_bounds__(256) void rev_sort_kernel(
     for (int i = threadIdx.x; i < len; i += blockDim.x) seg[i] = s[i];
     return;
   }
-  // Windowed counting sort: values are row ids in [0, n_rows) (or encoded
-  // listings in [0, n_rows * enc)).
+  // Windowed counting sort: values are row ids in [0, n_rows).
   int32_t* out = aux + (int64_t)h * cap + s0;
-  const int64_t range = rows.n_values(h);
+  const int64_t range = rows.n_rows(h);
   __shared__ int s_base;
   if (threadIdx.x == 0) s_base = 0;
   __syncthreads();
@@ -824,138 +812,257 @@ __global__ __launch_bounds__(256) void rev_sort_kernel(
   for (int64_t i = threadIdx.x; i < len; i += blockDim.x) seg[i] = out[i];
 }
 
-// ------------------------------------- query rows: one stable radix sort --
+// --------------------------------- query rows: one stable counting sort --
+// Rows that are queries (all of them, or those marked in `only`): a head's
+// queries are cut into chunks, each chunk's listings counted per block in
+// LDS, the counts scanned in (block, chunk) order, and each chunk's listings
+// placed in (query, slot) order behind the chunk's offset in every block.
+// Two reads of the marked rows and one write of each listing: bound by LDS
+// atomics and the scattered 4-byte writes.  A chunk without marked queries
+// costs its mask bytes, so a plan over block rows (nothing marked) does no
+// sort at all.  A radix sort of (block, listing) pairs took, pairs and
+// placement included, 1240 us at 24 heads x 131072 per-token top-16 rows and
+// 1450 us at 4 x 524288 top-32 block rows with nothing marked.
+constexpr int REV_WIN = 4096;          // blocks per workgroup (48 KB of LDS)
+constexpr int64_t REV_WAVES = 4096;    // chunks over all heads: 16 waves per CU
+constexpr int64_t REV_COUNTS = 8 << 20;  // chunk counts over all heads, at most (32 MB)
 
-// Pair i = (h * nq + q) * k + j: key h * nb + block for a valid slot of a
-// marked query, else the sentinel hkv * nb; value the listing (q, or
-// q * k + j when encoding the slot).  Generated in (h, q, j) order, so the
-// stable sort leaves each block's listings ascending.  One thread per pair
-// (n = hkv * nq * k < 2^31, checked by the caller): the row reads and the
-// key / value writes are contiguous across the wave.
-__global__ __launch_bounds__(256) void rev_pairs_kernel(
-    const int32_t* __restrict__ topk, int64_t hkv, int64_t nq, int k,
-    const int32_t* __restrict__ cu_q, int64_t batch, const int32_t* __restrict__ cu_sb,
-    int64_t nb, const uint8_t* __restrict__ only, bool encode, uint32_t* __restrict__ keys,
-    int32_t* __restrict__ vals) {
-  // 32-bit index arithmetic (every index here is below 2^31); a grid-stride
-  // loop over a bounded grid
-  const uint32_t n = (uint32_t)(hkv * nq * k);
-  const uint32_t none = (uint32_t)(hkv * nb);
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t hq = i / (uint32_t)k;  // h * nq + q
-    const int j = (int)(i - hq * (uint32_t)k);
-    const int h = (int)(hq / (uint32_t)nq);
-    const int64_t q = (int64_t)(hq - (uint32_t)h * (uint32_t)nq);
-    const bool on = !only || only[hq];
-    int b, bs, nbb;
-    bool start;
-    query_batch(cu_q, batch, cu_sb, q, &b, &bs, &nbb, &start);
-    const int v = topk[i];
-    const bool ok = on && v >= 0 && v < nbb && (int64_t)bs + v < nb;
-    keys[i] = ok ? (uint32_t)(h * nb + bs + v) : none;
-    vals[i] = encode ? (int32_t)(q * k + j) : (int32_t)q;
+struct RevChunks {
+  int64_t len, n;  // queries per chunk (a multiple of 64), chunks per head
+};
+inline RevChunks rev_chunks(int64_t hkv, int64_t nq, int64_t nb) {
+  int64_t n = std::min<int64_t>(ceil_div(REV_WAVES, hkv), REV_COUNTS / (hkv * (nb > 0 ? nb : 1)));
+  n = std::max<int64_t>(1, std::min<int64_t>(n, (nq + 63) / 64));
+  RevChunks c;
+  c.len = (((nq + n - 1) / n) + 63) / 64 * 64;
+  if (c.len < 64) c.len = 64;
+  c.n = std::max<int64_t>(1, (nq + c.len - 1) / c.len);
+  return c;
+}
+
+struct RevQueries {
+  const int32_t* topk;
+  int64_t nq;
+  int k;
+  const int32_t* cu_q;
+  int64_t batch;
+  const int32_t* cu_sb;
+  int64_t nb;
+  const uint8_t* only;  // [hkv, nq], or null: every query
+  int64_t chunk_len;
+  int n_chunks;
+};
+
+// The queries q0 .. q0 + 63 of head h that are listed (bit i: q0 + i).
+__device__ inline uint64_t rev_marked(const RevQueries& a, int h, int64_t q0, int lane) {
+  const int64_t q = q0 + lane;
+  return __ballot(q < a.nq && (!a.only || a.only[(int64_t)h * a.nq + q]));
+}
+
+// Calls f(r, j, c) for every listed id of queries q0 .. q0 + 63 whose global
+// block lies in [w0, w1): r the query's index in the group, j the slot, c the
+// block.  U ids per load (4: rows of whole, aligned 16-byte pieces).  One
+// wave; consecutive lanes hold consecutive ids.
+template <int U, class F>
+__device__ inline void rev_listings(const RevQueries& a, int h, int64_t q0, uint64_t marked,
+                                    int lane, int64_t w0, int64_t w1, F f) {
+  int b, bs0, nbb0;
+  bool st;
+  query_batch(a.cu_q, a.batch, a.cu_sb, q0, &b, &bs0, &nbb0, &st);
+  const bool one = b >= 0 && q0 + 63 < (int64_t)a.cu_q[b + 1];  // one batch element
+  const int units = a.k / U;  // per row
+  const int32_t* rows = a.topk + ((int64_t)h * a.nq + q0) * a.k;
+  for (int i = lane; i < 64 * units; i += 64) {
+    const int r = i / units;
+    if (!((marked >> r) & 1ull)) continue;
+    int32_t v[U];
+    if constexpr (U == 4) {
+      const u32x4 x = reinterpret_cast<const u32x4*>(rows)[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = (int32_t)x[e];
+    } else {
+      v[0] = rows[i];
+    }
+    int bs = bs0, nbb = nbb0;
+    if (!one) query_batch(a.cu_q, a.batch, a.cu_sb, q0 + r, &b, &bs, &nbb, &st);
+#pragma unroll
+    for (int e = 0; e < U; ++e) {
+      const int64_t c = (int64_t)bs + v[e];
+      if (v[e] >= 0 && v[e] < nbb && c >= w0 && c < w1) f(r, (i - r * units) * U + e, c);
+    }
   }
 }
 
-// seg[s] = first sorted position whose key is >= s, for s = 0 .. hkv * nb:
-// one thread per s, a binary search over the sorted keys (the work does not
-// depend on how the keys are spread; with every key the sentinel, a walk
-// between neighbouring keys would leave one thread writing all of seg).
-__global__ __launch_bounds__(256) void rev_bounds_kernel(const uint32_t* __restrict__ keys,
-                                                         int64_t n, int64_t n_seg,
-                                                         int32_t* __restrict__ seg) {
-  const int64_t sgi = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (sgi > n_seg) return;
-  int64_t lo = 0, hi = n;  // answer in [lo, hi]
-  while (lo < hi) {
-    const int64_t mid = (lo + hi) >> 1;
-    if ((int64_t)keys[mid] < sgi)
-      lo = mid + 1;
-    else
-      hi = mid;
+template <int U>
+__global__ __launch_bounds__(256) void rev_chunk_count_kernel(RevQueries a,
+                                                              int32_t* __restrict__ counts) {
+  extern __shared__ int hist[];
+  const int h = blockIdx.y, chunk = blockIdx.x;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int64_t w0 = (int64_t)blockIdx.z * REV_WIN;
+  const int64_t w1 = w0 + REV_WIN < a.nb ? w0 + REV_WIN : a.nb;
+  for (int i = threadIdx.x; i < w1 - w0; i += blockDim.x) hist[i] = 0;
+  __syncthreads();
+  const int64_t c0 = chunk * a.chunk_len;
+  const int64_t c1 = c0 + a.chunk_len < a.nq ? c0 + a.chunk_len : a.nq;
+  for (int64_t q0 = c0 + wv * 64; q0 < c1; q0 += 256) {
+    const uint64_t m = rev_marked(a, h, q0, lane);
+    if (m)
+      rev_listings<U>(a, h, q0, m, lane, w0, w1,
+                      [&](int, int, int64_t c) { atomicAdd(&hist[c - w0], 1); });
   }
-  seg[sgi] = (int32_t)lo;
+  __syncthreads();
+  for (int i = threadIdx.x; i < w1 - w0; i += blockDim.x)
+    counts[((int64_t)h * a.nb + w0 + i) * a.n_chunks + chunk] = hist[i];
 }
 
-// Per-head CSR offsets and totals from the segment starts.
-__global__ __launch_bounds__(256) void rev_offsets_kernel(const int32_t* __restrict__ seg,
-                                                          int64_t hkv, int64_t nb,
-                                                          int32_t* __restrict__ cu_rev,
-                                                          int32_t* __restrict__ totals) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= hkv * (nb + 1)) return;
-  const int64_t h = t / (nb + 1), c = t - h * (nb + 1);
-  const int32_t base = seg[h * nb];
-  cu_rev[t] = seg[h * nb + c] - base;
-  if (c == nb) totals[h] = seg[h * nb + nb] - base;
-}
-
-// rev[h * cap + pos] = the sorted listings of head h (the first seg[n_seg]
-// sorted pairs are the valid ones).
-__global__ __launch_bounds__(256) void rev_place_kernel(const uint32_t* __restrict__ keys,
-                                                        const int32_t* __restrict__ vals,
-                                                        const int32_t* __restrict__ seg,
-                                                        int64_t nb, int64_t n_seg, int64_t cap,
-                                                        int32_t* __restrict__ rev) {
-  const int64_t n = seg[n_seg];
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t h = keys[i] / (uint32_t)nb;  // keys and nb below 2^31: 32-bit divide
-    rev[h * cap + (i - seg[h * nb])] = vals[i];
+// Chunk counts in (block, chunk) order -> offsets in place, and the CSR
+// offsets of the blocks.
+struct ChunkCountF {
+  const int32_t* counts;
+  int64_t per_head;  // nb * n_chunks
+  __device__ int64_t limit(int, int64_t n) const { return n; }
+  __device__ int operator()(int h, int64_t i) const { return counts[(int64_t)h * per_head + i]; }
+};
+struct ChunkOffW {
+  int32_t* counts;
+  int64_t per_head;
+  int n_chunks;
+  int32_t* cu_rev;
+  int64_t nb;
+  __device__ void operator()(int h, int64_t i, int ex, int v, int64_t lim) const {
+    counts[(int64_t)h * per_head + i] = ex;
+    const int32_t c = (int32_t)i / n_chunks;  // i < REV_COUNTS + nb
+    int32_t* p = cu_rev + (int64_t)h * (nb + 1);
+    if (c * n_chunks == (int32_t)i) p[c] = ex;
+    if (i == lim - 1) p[nb] = ex + v;
   }
-}
+};
 
-size_t rev_sort_temp_bytes(int64_t n, unsigned bits) {
-  size_t bytes = 0;
-  (void)rocprim::radix_sort_pairs(nullptr, bytes, (const uint32_t*)nullptr,
-                                  (uint32_t*)nullptr, (const int32_t*)nullptr,
-                                  (int32_t*)nullptr, (unsigned)(n > 0 ? n : 1), 0, bits,
-                                  (hipStream_t)0);
-  return bytes;
+// One wave per chunk, 64 queries at a time: every listed block collects the
+// group's queries in a 64-bit mask, so that a listing's place is the block's
+// offset plus the queries below its own in the mask.  A group in which a row
+// lists a block twice takes its listings 64 at a time in order instead.
+template <int U>
+__global__ __launch_bounds__(64) void rev_chunk_place_kernel(RevQueries a,
+                                                             const int32_t* __restrict__ offs,
+                                                             int32_t* __restrict__ rev,
+                                                             int64_t cap, bool encode) {
+  extern __shared__ unsigned long long masks[];  // [blocks], then the offsets
+  const int h = blockIdx.y, chunk = blockIdx.x, lane = threadIdx.x;
+  const int64_t w0 = (int64_t)blockIdx.z * REV_WIN;
+  const int64_t w1 = w0 + REV_WIN < a.nb ? w0 + REV_WIN : a.nb;
+  const int nw = (int)(w1 - w0);
+  int* next = reinterpret_cast<int*>(masks + nw);
+  const int64_t c0 = chunk * a.chunk_len;
+  const int64_t c1 = c0 + a.chunk_len < a.nq ? c0 + a.chunk_len : a.nq;
+  int32_t* out = rev + (int64_t)h * cap;
+  bool ready = false;
+  for (int64_t q0 = c0; q0 < c1; q0 += 64) {
+    const uint64_t m = rev_marked(a, h, q0, lane);
+    if (!m) continue;
+    if (!ready) {  // the first marked group of the chunk
+      for (int i = lane; i < nw; i += 64) {
+        masks[i] = 0ull;
+        next[i] = offs[((int64_t)h * a.nb + w0 + i) * a.n_chunks + chunk];
+      }
+      ready = true;
+    }
+    __syncthreads();
+    bool twice = false;
+    rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int, int64_t c) {
+      twice |= (atomicOr(&masks[c - w0], 1ull << r) >> r) & 1ull;
+    });
+    __syncthreads();
+    if (!__ballot(twice)) {
+      rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int j, int64_t c) {
+        const int64_t pos =
+            next[c - w0] + __popcll(masks[c - w0] & ((1ull << r) - 1ull));
+        if (pos < cap) out[pos] = (int32_t)(encode ? (q0 + r) * a.k + j : q0 + r);
+      });
+      __syncthreads();
+      // the block's first listing moves its offset past the group
+      rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int, int64_t c) {
+        const unsigned long long mm = masks[c - w0];
+        if (mm && __ffsll(mm) - 1 == r) {
+          next[c - w0] += __popcll(mm);
+          masks[c - w0] = 0ull;
+        }
+      });
+    } else {
+      rev_listings<1>(a, h, q0, m, lane, w0, w1,
+                      [&](int, int, int64_t c) { masks[c - w0] = 0ull; });
+      const int32_t* rows = a.topk + ((int64_t)h * a.nq + q0) * a.k;
+      for (int i0 = 0; i0 < 64 * a.k; i0 += 64) {  // 64 listings in order
+        const int r = (i0 + lane) / a.k;
+        int c = -1;  // this lane's block within the window
+        if ((m >> r) & 1ull) {
+          int b, bs, nbb;
+          bool st;
+          query_batch(a.cu_q, a.batch, a.cu_sb, q0 + r, &b, &bs, &nbb, &st);
+          const int v = rows[i0 + lane];
+          const int64_t cg = (int64_t)bs + v;
+          if (v >= 0 && v < nbb && cg >= w0 && cg < w1) c = (int)(cg - w0);
+        }
+        uint64_t pend = __ballot(c >= 0);
+        while (pend) {  // one block's listings at a time (wave-uniform)
+          const int l = __builtin_ctzll(pend);
+          const int cl = __builtin_amdgcn_readlane(c, l);
+          const uint64_t same = __ballot(c == cl);
+          int base = 0;
+          if (lane == l) base = atomicAdd(&next[cl], __popcll(same));
+          base = __builtin_amdgcn_readlane(base, l);
+          const int64_t pos = base + __popcll(same & ((1ull << lane) - 1ull));
+          if (c == cl && pos < cap) {
+            const int64_t q = q0 + r;
+            out[pos] = (int32_t)(encode ? q * a.k + (i0 + lane - r * a.k) : q);
+          }
+          pend &= ~same;
+        }
+      }
+    }
+    __syncthreads();
+  }
 }
 
 int build_query_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq, int64_t topk_n,
                             const int32_t* cu_q, int64_t batch, const int32_t* cu_sb,
                             int64_t nb, Carver& ws, RevMap& map, hipStream_t st,
                             const uint8_t* only, bool encode_slot) {
-  const int64_t n = hkv * nq * topk_n;
-  const int64_t n_seg = hkv * nb;
-  uint32_t* keys = ws.take<uint32_t>((size_t)(n > 0 ? n : 1));
-  uint32_t* keys_out = ws.take<uint32_t>((size_t)(n > 0 ? n : 1));
-  int32_t* vals = ws.take<int32_t>((size_t)(n > 0 ? n : 1));
-  int32_t* vals_out = ws.take<int32_t>((size_t)(n > 0 ? n : 1));
-  int32_t* seg = ws.take<int32_t>((size_t)(n_seg + 1));
-  unsigned bits = 1;  // key bits: keys are <= n_seg
-  while (bits < 32 && (1ull << bits) <= (unsigned long long)n_seg) ++bits;
-  const size_t tb = rev_sort_temp_bytes(n, bits);
-  char* temp = ws.take<char>(tb);
+  const RevChunks ch = rev_chunks(hkv, nq, nb);
+  const int64_t per_head = (nb > 0 ? nb : 1) * ch.n;
+  int32_t* counts = ws.take<int32_t>((size_t)(hkv * per_head));
+  int32_t* sums = ws.take<int32_t>((size_t)scan_sums_size(per_head, hkv));
   if (!map.cu_rev) map.cu_rev = ws.take<int32_t>((size_t)(hkv * (nb + 1)));
   if (!map.rev) map.rev = ws.take<int32_t>((size_t)(hkv * (map.cap > 0 ? map.cap : 1)));
   if (!map.totals) map.totals = ws.take<int32_t>((size_t)hkv);
   if (!ws.base || ws.dry) return LSRM_OK;
   if (!ws.ok()) return LSRM_ERR_WORKSPACE;
-  if (nb == 0 || n == 0) {
+  if (nb == 0 || nq == 0) {
     int rc = launch_zero_i32(map.cu_rev, hkv * (nb + 1), st);
     if (rc) return rc;
     return launch_zero_i32(map.totals, hkv, st);
   }
-  const int64_t grid = std::min<int64_t>(ceil_div(n + 1, 256), 16384);
-  hipLaunchKernelGGL(rev_pairs_kernel, dim3(grid), dim3(256), 0, st, topk,
-                     hkv, nq, (int)topk_n, cu_q, batch, cu_sb, nb, only, encode_slot, keys,
-                     vals);
+  const RevQueries a{topk, nq,   (int)topk_n, cu_q, batch,
+                     cu_sb, nb, only,        ch.len, (int)ch.n};
+  const dim3 grid((unsigned)ch.n, (unsigned)hkv, (unsigned)ceil_div(nb, REV_WIN));
+  const size_t win = (size_t)std::min<int64_t>(nb, REV_WIN);
+  const bool vec = topk_n % 4 == 0 && ((uintptr_t)topk % 16) == 0;
+  if (vec)
+    hipLaunchKernelGGL(rev_chunk_count_kernel<4>, grid, dim3(256), win * 4, st, a, counts);
+  else
+    hipLaunchKernelGGL(rev_chunk_count_kernel<1>, grid, dim3(256), win * 4, st, a, counts);
   LSRM_CHECK_LAUNCH();
-  size_t tbv = tb;
-  if (rocprim::radix_sort_pairs(temp, tbv, keys, keys_out, vals, vals_out, (unsigned)n, 0,
-                                bits, st) != hipSuccess)
-    return LSRM_ERR_LAUNCH;
-  hipLaunchKernelGGL(rev_bounds_kernel, dim3(ceil_div(n_seg + 1, 256)), dim3(256), 0, st,
-                     keys_out, n, n_seg, seg);
-  LSRM_CHECK_LAUNCH();
-  hipLaunchKernelGGL(rev_offsets_kernel, dim3(ceil_div(hkv * (nb + 1), 256)), dim3(256), 0, st,
-                     seg, hkv, nb, map.cu_rev, map.totals);
-  LSRM_CHECK_LAUNCH();
-  hipLaunchKernelGGL(rev_place_kernel, dim3(grid), dim3(256), 0, st, keys_out,
-                     vals_out, seg, nb, n_seg, map.cap, map.rev);
+  const int rc = run_scan(ChunkCountF{counts, per_head},
+                          ChunkOffW{counts, per_head, (int)ch.n, map.cu_rev, nb}, per_head,
+                          (int)hkv, sums, map.totals, st);
+  if (rc) return rc;
+  if (vec)
+    hipLaunchKernelGGL(rev_chunk_place_kernel<4>, grid, dim3(64), win * 12, st, a, counts,
+                       map.rev, map.cap, encode_slot);
+  else
+    hipLaunchKernelGGL(rev_chunk_place_kernel<1>, grid, dim3(64), win * 12, st, a, counts,
+                       map.rev, map.cap, encode_slot);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }
@@ -965,8 +1072,7 @@ int build_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq,
                       const int32_t* cu_sb, int64_t nb, bool rows_are_tiles,
                       const TilePlan* plan, Carver& ws, RevMap& map,
                       hipStream_t st, const uint8_t* only, bool encode_slot) {
-  if (!rows_are_tiles && hkv * nq * topk_n < (int64_t{1} << 31) &&
-      hkv * nb < (int64_t{1} << 31))
+  if (!rows_are_tiles)
     return build_query_reverse_map(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, nb, ws, map, st,
                                    only, encode_slot);
   int32_t* counts = ws.take<int32_t>((size_t)(hkv * (nb > 0 ? nb : 1)));
@@ -979,10 +1085,7 @@ int build_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq,
   if (!ws.base || ws.dry) return LSRM_OK;
   if (!ws.ok()) return LSRM_ERR_WORKSPACE;
 
-  RowSrc rows{rows_are_tiles ? plan->tiles : nullptr,
-              rows_are_tiles ? plan->tile_count : nullptr, nq,
-              rows_are_tiles ? nullptr : only,
-              (!rows_are_tiles && encode_slot) ? (int)topk_n : 0};
+  RowSrc rows{plan->tiles, plan->tile_count, nq};
   int rc = launch_zero_i32(counts, hkv * nb, st);
   if (rc) return rc;
   rc = launch_zero_i32(fill, hkv * nb, st);

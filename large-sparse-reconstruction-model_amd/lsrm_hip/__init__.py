@@ -196,12 +196,11 @@ def _attn_check(q, k, v, topk_idx, do=None, o=None, lse=None) -> torch.device:
 
 
 def _no_capture(what: str) -> None:
-    """Backward and key-centric plans sort with rocPRIM, whose radix sort
-    clears its state with hipMemsetAsync: such plans are not built under HIP
-    graph capture (a memset node has given wrong results on graph replays)."""
+    """Backward and key-centric plans are not built under HIP graph capture:
+    replays of their construction are not covered by a check."""
     if torch.cuda.is_current_stream_capturing():
-        raise RuntimeError(f"{what} cannot be built under HIP graph capture (its sort "
-                           "issues memsets); build the plan before capturing")
+        raise RuntimeError(f"{what} cannot be built under HIP graph capture; build the plan "
+                           "before capturing")
 
 
 def _i32(t: torch.Tensor) -> torch.Tensor:
@@ -457,8 +456,8 @@ def plan_for(q_shape, k_shape, topk_idx, cu_seqblocks, cu_block_tokens, cu_seqle
     global plan_builds
     capturing = torch.cuda.is_current_stream_capturing()
     if capturing and not backward:
-        # the key-centric part sorts with rocPRIM (memsets): a captured
-        # forward takes the grouped-tile plan, which captures
+        # key-centric plans are not built under capture: a captured forward
+        # takes the grouped-tile plan
         key_centric = False
     key = None if capturing else _plan_key(q_shape, k_shape, topk_idx, cu_seqblocks,
                                            cu_block_tokens, cu_seqlens_q, key_centric)
