@@ -1040,7 +1040,8 @@ sel_attn_dkdv_kernel(AttnArgs a) {
     __syncthreads();
   }
   };
-  if (uniform(a.plan.ghead_off[a.hkv]) > 0)
+  // (a key-centric plan may list queries of run tiles too)
+  if (a.kc.fitems || uniform(a.plan.ghead_off[a.hkv]) > 0)
     items_loop(Phase<1>{});
   else
     items_loop(Phase<0>{});

@@ -105,16 +105,19 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
               hipStream_t st) {
   const bool backward = (flags & LSRM_PLAN_BACKWARD) != 0;
   const int tq = ROWS / g;
+  bool derive = false;  // the backward's query map comes from the key-centric one
   int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, ws,
                            w.plan, st, true);
   if (rc) return rc;
   if (backward) {
     // dK/dV rows: the run tiles that selected a block, then the queries of
-    // grouped tiles that selected it.
+    // grouped tiles (and of packed run tiles) that selected it.
+    const int packed_q = dkdv_packed_q((flags & LSRM_PLAN_KEY_CENTRIC) != 0, tq);
+    derive = (flags & LSRM_PLAN_KEY_CENTRIC) != 0 && packed_q == 0;
     w.rev = RevMap{};
     w.rev.cap = nq * topk_n;
     rc = build_reverse_map(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, nb, true,
-                           &w.plan, ws, w.rev, st);
+                           &w.plan, ws, w.rev, st, nullptr, false, packed_q);
     if (rc) return rc;
     uint8_t* grouped = reinterpret_cast<uint8_t*>(
         ws.take<int32_t>((size_t)((hkv * nq + 3) / 4 > 0 ? (hkv * nq + 3) / 4 : 1)));
@@ -122,10 +125,12 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
       if (!ws.ok()) return LSRM_ERR_WORKSPACE;
       rc = mark_grouped_queries(w.plan, hkv, nq, grouped, st);
       if (rc) return rc;
+      rc = mark_short_tiles(w.plan, hkv, nq, packed_q, grouped, st);
+      if (rc) return rc;
     }
     w.qrev = RevMap{};
     w.qrev.cap = nq * topk_n;
-    if (flags & LSRM_PLAN_KEY_CENTRIC) {
+    if (derive) {
       // The key-centric part lists the same queries per block (slot-encoded,
       // in the same order): the map is carved here and derived from that one
       // once it is built.
@@ -165,7 +170,7 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
     rc = build_kc_items(kc.grev, cu_blk, nk, hkv, nb, tq, head_dim, topk_n, ws, kc,
                         w.plan.counter, kc_plan_marker(flags, (int)head_dim), st);
     if (rc) return rc;
-    if (backward && ws.base && !ws.dry) {
+    if (derive && ws.base && !ws.dry) {
       rc = derive_query_map(kc.grev, w.qrev, hkv, nb, topk_n, st);
       if (rc) return rc;
     }

@@ -52,16 +52,35 @@ int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
 // with `only` (a [hkv, nq] byte mask) only the queries it marks.
 // encode_slot (rows are queries): a listing stores q * topk_n + j, j the
 // slot of the row that lists the block (ascending order is unchanged).
+// skip_q (rows are tiles): tiles of at most skip_q queries are left out.
 int build_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq,
                       int64_t topk_n, const int32_t* cu_q, int64_t batch,
                       const int32_t* cu_sb, int64_t nb, bool rows_are_tiles,
                       const TilePlan* plan, Carver& ws, RevMap& map,
                       hipStream_t st, const uint8_t* only = nullptr,
-                      bool encode_slot = false);
+                      bool encode_slot = false, int skip_q = 0);
 
 // flags[h, q] = 1 for the queries of the grouped tiles of `plan`, else 0.
 int mark_grouped_queries(const TilePlan& plan, int64_t hkv, int64_t nq,
                          uint8_t* flags, hipStream_t st);
+
+// flags[h, q] = 1 too for the queries of the run tiles of at most short_q
+// queries.
+int mark_short_tiles(const TilePlan& plan, int64_t hkv, int64_t nq, int short_q,
+                     uint8_t* flags, hipStream_t st);
+
+// Longest run tile whose queries dK/dV takes one by one from the query map
+// (128 / g of them packed into a step) instead of one tile per step, in a
+// backward plan of the given flags; 0: none.  Only key-centric plans with
+// tiles of at most 16 queries (8 or more query heads per kv head): there a
+// run of a few equal per-token rows is not short enough to be grouped, yet
+// fills a quarter of a step.  3D-aware rows of 122880 tokens at 32 / 2 heads:
+// 26600 run tiles per kv head, 2.0 of 8 queries on average; dK/dV 9.28 ->
+// 6.13 ms.  With larger tiles such runs are grouped anyway, and the map is
+// derived from the key-centric one.
+inline int dkdv_packed_q(bool key_centric, int tq) {
+  return key_centric && tq <= 16 ? tq / 2 : 0;
+}
 
 // Key-centric part of a plan (plan flag LSRM_PLAN_KEY_CENTRIC): the grouped
 // tiles are taken out of the grouped-tile kernels (which a key-centric plan

@@ -572,12 +572,16 @@ int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
 // --------------------------------------------------------- reverse map --
 
 // Rows that are run tiles: row r of head h reads the selection of its tile's
-// first query.
+// first query; tiles of at most `skip_q` queries are not entered.
 struct RowSrc {
   const int2* tiles;
   const int32_t* count;  // tiles per head
   int64_t nq;
+  int skip_q;
   __device__ int64_t n_rows(int h) const { return (int64_t)count[h]; }
+  __device__ bool skip(int h, int64_t r) const {
+    return skip_q > 0 && tiles[(int64_t)h * nq + r].y <= skip_q;
+  }
   __device__ int64_t query(int h, int64_t r) const {
     return (int64_t)tiles[(int64_t)h * nq + r].x;
   }
@@ -590,7 +594,7 @@ __global__ __launch_bounds__(256) void rev_count_kernel(
     int32_t* __restrict__ counts) {
   const int h = blockIdx.y;
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows.n_rows(h)) return;
+  if (r >= rows.n_rows(h) || rows.skip(h, r)) return;
   const int64_t q = rows.query(h, r);
   int b, bs, nbb;
   bool start;
@@ -611,7 +615,7 @@ __global__ __launch_bounds__(256) void rev_scatter_kernel(
     int32_t* __restrict__ rev, int64_t cap) {
   const int h = blockIdx.y;
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows.n_rows(h)) return;
+  if (r >= rows.n_rows(h) || rows.skip(h, r)) return;
   const int64_t q = rows.query(h, r);
   int b, bs, nbb;
   bool start;
@@ -649,7 +653,7 @@ __global__ __launch_bounds__(256) void rev_count_lds_kernel(
   for (int i = threadIdx.x; i < nb; i += blockDim.x) hist[i] = 0;
   __syncthreads();
   const int64_t r = r0 + threadIdx.x;
-  if (r < rows.n_rows(h)) {
+  if (r < rows.n_rows(h) && !rows.skip(h, r)) {
     const int64_t q = rows.query(h, r);
     int b, bs, nbb;
     bool start;
@@ -682,7 +686,7 @@ __global__ __launch_bounds__(256) void rev_scatter_lds_kernel(
   }
   __syncthreads();
   const int64_t r = r0 + threadIdx.x;
-  const bool on = r < rows.n_rows(h);
+  const bool on = r < rows.n_rows(h) && !rows.skip(h, r);
   int bs = 0, nbb = 0;
   const int32_t* row = topk;
   if (on) {
@@ -1071,7 +1075,7 @@ int build_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq,
                       int64_t topk_n, const int32_t* cu_q, int64_t batch,
                       const int32_t* cu_sb, int64_t nb, bool rows_are_tiles,
                       const TilePlan* plan, Carver& ws, RevMap& map,
-                      hipStream_t st, const uint8_t* only, bool encode_slot) {
+                      hipStream_t st, const uint8_t* only, bool encode_slot, int skip_q) {
   if (!rows_are_tiles)
     return build_query_reverse_map(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, nb, ws, map, st,
                                    only, encode_slot);
@@ -1085,7 +1089,7 @@ int build_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq,
   if (!ws.base || ws.dry) return LSRM_OK;
   if (!ws.ok()) return LSRM_ERR_WORKSPACE;
 
-  RowSrc rows{plan->tiles, plan->tile_count, nq};
+  RowSrc rows{plan->tiles, plan->tile_count, nq, skip_q};
   int rc = launch_zero_i32(counts, hkv * nb, st);
   if (rc) return rc;
   rc = launch_zero_i32(fill, hkv * nb, st);
@@ -1137,6 +1141,27 @@ __global__ __launch_bounds__(256) void mark_grouped_kernel(const int2* __restric
   if (t >= gcount[h]) return;
   const int2 g = gtiles[(int64_t)h * nq + t];
   for (int i = 0; i < g.y; ++i) flags[(int64_t)h * nq + g.x + i] = 1;
+}
+
+__global__ __launch_bounds__(256) void mark_short_kernel(const int2* __restrict__ tiles,
+                                                         const int32_t* __restrict__ count,
+                                                         int64_t nq, int short_q,
+                                                         uint8_t* __restrict__ flags) {
+  const int h = blockIdx.y;
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= count[h]) return;
+  const int2 r = tiles[(int64_t)h * nq + t];
+  if (r.y > short_q) return;
+  for (int i = 0; i < r.y; ++i) flags[(int64_t)h * nq + r.x + i] = 1;
+}
+
+int mark_short_tiles(const TilePlan& plan, int64_t hkv, int64_t nq, int short_q,
+                     uint8_t* flags, hipStream_t st) {
+  if (nq <= 0 || short_q <= 0) return LSRM_OK;
+  hipLaunchKernelGGL(mark_short_kernel, dim3(ceil_div(nq, 256), (unsigned)hkv), dim3(256), 0, st,
+                     plan.tiles, plan.tile_count, nq, short_q, flags);
+  LSRM_CHECK_LAUNCH();
+  return LSRM_OK;
 }
 
 int mark_grouped_queries(const TilePlan& plan, int64_t hkv, int64_t nq,
