@@ -676,4 +676,71 @@ __device__ inline uint32_t group_offset(const SelLds& s, GroupCursor& c, int P,
   return (uint32_t)tok * row_bytes + chunk_byte;
 }
 
+// ------------------------------------------------------- narrow run tiles --
+// Run tiles of at most NARROW_ROWS rows (short runs of per-token rows at many
+// query heads per kv head) would leave two or three of a workgroup's four
+// waves idle for the tile's whole key stream.  They are split over the keys
+// instead: the waves of one 32-row block (four for up to 32 rows, two for up
+// to 64) take the stream's 32-key blocks in turn, each at its own pace.  A
+// block's K and V rows belong to one wave, so they go straight into its
+// registers (two blocks ahead, no barrier); only the operand that is needed
+// transposed passes through a wave's own piece of LDS.  The waves' fp32 sums
+// are added in LDS in a fixed order at the end.
+//
+// Bound by L2 requests for the gathered rows (3D-aware rows of 122880 tokens
+// at 32 / 2 heads of 32: 26600 tiles per kv head, 480 M requests of 64 bytes,
+// 8.7 of 16 per clock and XCD): forward 3.69 -> 3.28 ms, dQ 5.11 -> 3.34 ms;
+// with the stream staged in LDS for all four waves, one barrier per 128 keys
+// and three steps in flight, 3.62 and 3.50 ms.  At head dim 64 a run tile's K
+// and V traffic sets its time whatever its rows, and the run-tile kernels move
+// it with wider requests: 454 blocks of 32..512 queries at 24 heads took 9.1 ms
+// as run tiles, 10.3 ms split by width (9.2 with the stream in LDS).
+constexpr bool narrow_split(int d) { return d <= 32; }
+
+// One wave's walk over its 32-key blocks of a narrow tile's stream.
+template <int D>
+struct NarrowBlocks {
+  static constexpr int NS = D / 16;
+  GroupCursor cur;
+  const SelLds* sel;
+  const int* map;
+  const char *kbase, *vbase;
+  uint32_t row_bytes, lane_off, chunk;
+  int nkeys, t_safe, lane_row;
+
+  __device__ inline void init(const AttnArgs& a, int h, const SelLds& s, const int* tokmap,
+                              int nk, int lane) {
+    sel = &s;
+    map = tokmap;
+    nkeys = nk;
+    t_safe = uniform(s.n > 0 ? s.tok[0] : 0);
+    row_bytes = (uint32_t)a.hkv * D * 2;
+    kbase = reinterpret_cast<const char*>(a.k + (int64_t)h * D);
+    vbase = reinterpret_cast<const char*>(a.v + (int64_t)h * D);
+    lane_row = lane & 31;
+    chunk = (uint32_t)(lane >> 5) * 16;
+    lane_off = (uint32_t)lane_row * row_bytes + chunk;
+    group_init(s, cur, tokmap != nullptr);
+  }
+  // K and V of block b (a wave's blocks ascend; positions past the stream
+  // load a resident token): lane (hb, row) holds chunks 2 s + hb of its row.
+  __device__ inline __attribute__((always_inline)) void load(int b, u32x4* k, u32x4* v) {
+    const uint32_t off = group_offset<32>(*sel, cur, b * 32, nkeys, t_safe, row_bytes, lane_row,
+                                          lane_off, chunk, map);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      k[s] = *reinterpret_cast<const u32x4*>(kbase + (uint64_t)off + s * 32);
+      v[s] = *reinterpret_cast<const u32x4*>(vbase + (uint64_t)off + s * 32);
+    }
+  }
+};
+
+// Orders a wave's own LDS writes before its later reads of other lanes' data
+// (one wave's LDS operations execute in order; this holds the compiler to it).
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace lsrm

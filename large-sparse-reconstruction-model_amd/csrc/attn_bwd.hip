@@ -33,7 +33,186 @@ namespace lsrm {
 
 // ------------------------------------------------------------------- dQ --
 
-// MODE 0 (DQ_RUN): the run tiles of the plan.  MODE 1 (DQ_UNION): the
+// dQ of a narrow run tile (see attn.h): every wave sums dS K over its own keys,
+// and the waves of one row block are added in LDS.
+template <int DT, int D>
+__device__ inline __attribute__((always_inline)) void narrow_dq(
+    const AttnArgs& a, int h, int q0, int rows, const SelLds& sel, const int* map, int nkeys,
+    char* lds, int wv, int lane) {
+  using G = KvTile<D>;
+  constexpr int NS = D / 16, ND = D / 32;
+  const int hb = lane >> 5, l32 = lane & 31;
+  // waves over the keys of one row block, this wave's row block and turn
+  const int nkw = rows <= 32 ? 4 : 2;
+  const int rb = rows <= 32 ? 0 : (wv & 1), kq = rows <= 32 ? wv : (wv >> 1);
+  const int r = rb * 32 + l32;
+  const bool row_ok = r < rows;
+  const int64_t qi = q0 + (row_ok ? r / a.g : 0);
+  const int hh = h * a.g + (row_ok ? r % a.g : 0);
+  NarrowBlocks<D> blocks;
+  blocks.init(a, h, sel, map, nkeys, lane);
+  const int nblk = (nkeys + 31) / 32;
+  u32x4 kb[2][NS], vb[2][NS];
+  if (kq < nblk) blocks.load(kq, kb[0], vb[0]);
+  if (kq + nkw < nblk) blocks.load(kq + nkw, kb[1], vb[1]);
+  u32x4 qb[NS], dob[NS];
+  float dpart = 0.0f;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    if (row_ok) {
+      const int64_t off = (qi * a.hq + hh) * D + s * 16 + hb * 8;
+      qb[s] = *reinterpret_cast<const u32x4*>(a.q + off);
+      dob[s] = *reinterpret_cast<const u32x4*>(a.dout + off);
+      const u32x4 ob = *reinterpret_cast<const u32x4*>(a.o + off);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        dpart += to_f32<DT>((uint16_t)(ob[i] & 0xffffu)) *
+                 to_f32<DT>((uint16_t)(dob[s][i] & 0xffffu));
+        dpart += to_f32<DT>((uint16_t)(ob[i] >> 16)) * to_f32<DT>((uint16_t)(dob[s][i] >> 16));
+      }
+    } else {
+      qb[s] = dob[s] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  const float delta = dpart + __shfl_xor(dpart, 32);
+  // exponent bias -lse; -inf (P = 0) for rows past the tile and rows that
+  // attend nothing
+  float bias = -__builtin_inf();
+  if (row_ok) {
+    const float l = a.lse_in[(int64_t)hh * a.nq + qi];
+    if (l > -__builtin_inf()) bias = -l;
+    if (hb == 0 && kq == 0) a.lse[(int64_t)hh * a.nq + qi] = delta;
+  }
+  char* sk = lds + wv * (32 * D * 2);
+  uint32_t vl_off[ND][2];
+  {
+    const int gi = lane & 15, dh = (lane >> 4) & 1;
+#pragma unroll
+    for (int db = 0; db < ND; ++db) {
+      const int dcol = db * 32 + dh * 16 + (gi & 3) * 4;
+      const int k0 = hb * 4 + (gi >> 2);
+      const int cb = dcol >> 3, half = (dcol & 4) * 2;
+      vl_off[db][0] = (uint32_t)(G::off(k0, cb) + half);
+      vl_off[db][1] = (uint32_t)(G::off(k0 + 8, cb) + half);
+    }
+  }
+  f32x16 dqacc[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dqacc[i][v] = 0.0f;
+  auto block = [&](int b, u32x4* kr, u32x4* vr) __attribute__((always_inline)) {
+    f32x16 sc, dp;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = dp[v] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      sc = mfma32<DT>(kr[s], qb[s], sc);
+      dp = mfma32<DT>(vr[s], dob[s], dp);
+    }
+    wave_lds_order();  // the block before this one has been read
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      *reinterpret_cast<u32x4*>(sk + G::off(l32, 2 * s + hb)) = kr[s];
+    wave_lds_order();
+    if (b + 2 * nkw < nblk) blocks.load(b + 2 * nkw, kr, vr);
+    if (b * 32 + 32 > nkeys) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (b * 32 + acc_row(v, hb) >= nkeys) sc[v] = -__builtin_inf();
+    }
+    u32x4 ds[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int v0 = c * 8 + 2 * e;
+        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[v0], a.scale_log2, bias));
+        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[v0 + 1], a.scale_log2, bias));
+        ds[c][e] = pack2<DT>(p0 * (dp[v0] - delta), p1 * (dp[v0 + 1] - delta));
+      }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int db = 0; db < ND; ++db) {
+        const int o = c * 16 * (D * 2);
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4*)(sk + o + vl_off[db][0])));
+        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4*)(sk + o + vl_off[db][1])));
+        dqacc[db] = mfma32<DT>(u32x4{lo[0], lo[1], hi[0], hi[1]}, ds[c], dqacc[db]);
+      }
+  };
+  if (rb * 32 < rows) {  // wave-uniform
+    for (int b = kq; b < nblk; b += 2 * nkw) {
+      block(b, kb[0], vb[0]);
+      if (b + nkw < nblk) block(b + nkw, kb[1], vb[1]);
+    }
+  }
+  __syncthreads();  // every wave has left its blocks
+  constexpr int RED = ND * 16;  // words per lane
+  float* red = reinterpret_cast<float*>(lds) + lane;
+  if (kq > 0) {
+    float* mine = red + (rb * (nkw - 1) + kq - 1) * RED * 64;
+#pragma unroll
+    for (int db = 0; db < ND; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mine[(db * 16 + v) * 64] = dqacc[db][v];
+  }
+  __syncthreads();
+  if (kq > 0 || !row_ok) return;
+  const float* others = red + rb * (nkw - 1) * RED * 64;
+  for (int w = 0; w < nkw - 1; ++w)
+#pragma unroll
+    for (int db = 0; db < ND; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) dqacc[db][v] += others[(w * RED + db * 16 + v) * 64];
+  uint16_t* drow = a.out + (qi * a.hq + hh) * D;
+#pragma unroll
+  for (int db = 0; db < ND; ++db)
+#pragma unroll
+    for (int gi = 0; gi < 4; ++gi) {
+      const int v = gi * 4;
+      // dS was kept unscaled: dQ = scale * (dS' K)
+      *reinterpret_cast<u32x2*>(drow + db * 32 + gi * 8 + hb * 4) =
+          u32x2{pack2<DT>(a.scale * dqacc[db][v], a.scale * dqacc[db][v + 1]),
+                pack2<DT>(a.scale * dqacc[db][v + 2], a.scale * dqacc[db][v + 3])};
+    }
+}
+
+template <int DT, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4))) void
+narrow_dq_kernel(AttnArgs a) {
+  constexpr int RED_BYTES = 3 * (D / 2) * 64 * 4, K_BYTES = 4 * 32 * D * 2;
+  __shared__ __align__(1024) char s_lds[RED_BYTES > K_BYTES ? RED_BYTES : K_BYTES];
+  __shared__ SelLds sel;
+  __shared__ int s_tokmap[KMAP_KEYS];
+  __shared__ int s_slot;
+  const int lane = threadIdx.x & 63, wv = uniform(threadIdx.x >> 6);
+  // A plan built without its backward part: nothing here is valid to read.
+  if (a.plan.counter[PLAN_BWD_SLOT] != PLAN_BWD_MAGIC) return;
+  const int32_t* off = a.plan.narrow_off;
+  const int total = off[a.hkv];
+  if (total == 0) return;
+  int32_t* queue = a.plan.counter + NARROW_QUEUE_SLOT;
+  for (;;) {
+    const int w = uniform(fetch_work(queue, &s_slot));
+    if (w >= total) break;
+    const int h = head_of(off, a.hkv, w);
+    const int2 tile = a.plan.by_width[(int64_t)h * a.nq + (a.nq - 1 - (w - off[h]))];
+    load_selection(a, h, tile.x, sel);
+    const int nkeys = uniform(sel.cum[sel.n]), rows = uniform(tile.y) * a.g;
+    const int* map = nullptr;
+    if (nkeys <= KMAP_KEYS) {
+      build_token_map(sel, s_tokmap, wv, lane);
+      map = s_tokmap;
+    }
+    narrow_dq<DT, D>(a, h, tile.x, rows, sel, map, nkeys, s_lds, wv, lane);
+  }
+  leave_queue(queue, queue + NARROW_EXIT_SLOT - NARROW_QUEUE_SLOT);
+}
+
+// MODE 0 (DQ_RUN): the run tiles of the plan (head dims up to 64: the wide ones).  MODE 1 (DQ_UNION): the
 // grouped tiles, run once over the union of their rows' blocks with per-row
 // key masks, or once per run of identical rows with the other rows' P forced
 // to zero (the passes of the forward's grouped tiles; no softmax state is
@@ -65,9 +244,12 @@ sel_attn_dq_kernel(AttnArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63, wv = uniform(tid >> 6);
   const int hb = lane >> 5, l32 = lane & 31;
+  // head dims with a narrow-tile kernel leave the narrow run tiles to it
+  constexpr bool WIDE = MODE == DQ_RUN && narrow_split(D);
   const int32_t* head_off =
-      GATHER ? a.kc.fitem_off : (UNION ? a.plan.ghead_off : a.plan.head_off);
-  const int2* tiles = UNION ? a.plan.gtiles : a.plan.tiles;
+      GATHER ? a.kc.fitem_off
+             : (UNION ? a.plan.ghead_off : (WIDE ? a.plan.wide_off : a.plan.head_off));
+  const int2* tiles = UNION ? a.plan.gtiles : (WIDE ? a.plan.by_width : a.plan.tiles);
   int32_t* queue = a.plan.counter + (GATHER ? KC_QUEUE_SLOT : (UNION ? 4 : 0));
   // A plan built without its backward part: nothing here is valid to read.
   if (a.plan.counter[PLAN_BWD_SLOT] != PLAN_BWD_MAGIC) return;
@@ -1474,6 +1656,13 @@ __global__ __launch_bounds__(256) void kc_dq_merge_kernel(AttnArgs a) {
 
 template <int DT, int D>
 int launch_bwd_t(const AttnArgs& a, hipStream_t st) {
+  if constexpr (narrow_split(D)) {
+    const int grid =
+        persistent_grid(reinterpret_cast<const void*>(&narrow_dq_kernel<DT, D>), 256, 0);
+    if (grid <= 0) return LSRM_ERR_LAUNCH;
+    hipLaunchKernelGGL((narrow_dq_kernel<DT, D>), dim3(grid), dim3(256), 0, st, a);
+    LSRM_CHECK_LAUNCH();
+  }
   {
     const void* fn = reinterpret_cast<const void*>(&sel_attn_dq_kernel<DT, D, DQ_RUN>);
     const int grid = persistent_grid(fn, 256, 0);

@@ -67,8 +67,209 @@ __device__ inline float row_max(const f32x16* sc) {
                                        __builtin_bit_cast(float, (unsigned)sw[1]));
 }
 
+// A narrow run tile (see attn.h): rows of queries q0 .. of kv head h over the
+// stream in `sel`.  The softmax runs online with lazy rescaling (p <= 2^8),
+// each wave over its own keys; at the end the waves of one row block are
+// merged in fp32: M = max m_w, O = sum 2^(m_w - M) O_w, l likewise.
+// `red` (LDS): a wave's V blocks while it runs, then the waves' sums.
+template <int DT, int D>
+__device__ inline __attribute__((always_inline)) void narrow_fwd(
+    const AttnArgs& a, int h, int q0, int rows, const SelLds& sel, const int* map, int nkeys,
+    char* lds, int wv, int lane) {
+  using G = KvTile<D>;
+  constexpr int NS = D / 16, ND = D / 32;
+  const int hb = lane >> 5, l32 = lane & 31;
+  // waves over the keys of one row block, this wave's row block and turn
+  const int nkw = rows <= 32 ? 4 : 2;
+  const int rb = rows <= 32 ? 0 : (wv & 1), kq = rows <= 32 ? wv : (wv >> 1);
+  const int r = rb * 32 + l32;
+  const bool row_ok = r < rows;
+  const int64_t qi = q0 + (row_ok ? r / a.g : 0);
+  const int hh = h * a.g + (row_ok ? r % a.g : 0);
+  NarrowBlocks<D> blocks;
+  blocks.init(a, h, sel, map, nkeys, lane);
+  const int nblk = (nkeys + 31) / 32;
+  u32x4 kb[2][NS], vb[2][NS];
+  if (kq < nblk) blocks.load(kq, kb[0], vb[0]);
+  if (kq + nkw < nblk) blocks.load(kq + nkw, kb[1], vb[1]);
+  u32x4 qb[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s)
+    qb[s] = row_ok ? *reinterpret_cast<const u32x4*>(a.q + (qi * a.hq + hh) * D + s * 16 + hb * 8)
+                   : u32x4{0u, 0u, 0u, 0u};
+  char* sv = lds + wv * (32 * D * 2);
+  uint32_t vl_off[ND][2];
+  {
+    const int gi = lane & 15, dh = (lane >> 4) & 1;
+#pragma unroll
+    for (int db = 0; db < ND; ++db) {
+      const int dcol = db * 32 + dh * 16 + (gi & 3) * 4;
+      const int k0 = hb * 4 + (gi >> 2);
+      const int cb = dcol >> 3, half = (dcol & 4) * 2;
+      vl_off[db][0] = (uint32_t)(G::off(k0, cb) + half);
+      vl_off[db][1] = (uint32_t)(G::off(k0 + 8, cb) + half);
+    }
+  }
+  f32x16 oacc[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[i][v] = 0.0f;
+  float m_run = -__builtin_inf(), l_run = 0.0f;
+  auto block = [&](int b, u32x4* kr, u32x4* vr) __attribute__((always_inline)) {
+    f32x16 sc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sc = mfma32<DT>(kr[s], qb[s], sc);
+    wave_lds_order();  // the block before this one has been read
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      *reinterpret_cast<u32x4*>(sv + G::off(l32, 2 * s + hb)) = vr[s];
+    wave_lds_order();
+    if (b + 2 * nkw < nblk) blocks.load(b + 2 * nkw, kr, vr);
+    if (b * 32 + 32 > nkeys) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (b * 32 + acc_row(v, hb) >= nkeys) sc[v] = -__builtin_inf();
+    }
+    const float m3 = max3f(max3f(sc[0], sc[1], sc[2]), max3f(sc[3], sc[4], sc[5]),
+                           max3f(sc[6], sc[7], sc[8]));
+    const float mx = max3f(m3, max3f(sc[9], sc[10], sc[11]),
+                           max3f(sc[12], sc[13], max3f(sc[14], sc[15], sc[15])));
+    const auto sw = __builtin_amdgcn_permlane32_swap(
+        __builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
+    const float m_tile =
+        __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)sw[0]),
+                                      __builtin_bit_cast(float, (unsigned)sw[1])) *
+        a.scale_log2;
+    if (__builtin_amdgcn_ballot_w64(m_tile > m_run + RESCALE_LOG2) != 0) {
+      const float m_new = __builtin_elementwise_maximum(m_run, m_tile);
+      const float alpha =
+          m_new == -__builtin_inf() ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < ND; ++db)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) oacc[db][v] *= alpha;
+    }
+    const float negm = m_run == -__builtin_inf() ? 0.0f : -m_run;
+    u32x4 pb[2];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int v0 = c * 8 + 2 * e;
+        pb[c][e] =
+            pack2<DT>(__builtin_amdgcn_exp2f(__builtin_fmaf(sc[v0], a.scale_log2, negm)),
+                      __builtin_amdgcn_exp2f(__builtin_fmaf(sc[v0 + 1], a.scale_log2, negm)));
+        l_run = sum2<DT>(pb[c][e], l_run);
+      }
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int db = 0; db < ND; ++db) {
+        const int o = c * 16 * (D * 2);
+        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4*)(sv + o + vl_off[db][0])));
+        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_s16x4*)(sv + o + vl_off[db][1])));
+        oacc[db] = mfma32<DT>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb[c], oacc[db]);
+      }
+  };
+  if (rb * 32 < rows) {  // wave-uniform
+    for (int b = kq; b < nblk; b += 2 * nkw) {
+      block(b, kb[0], vb[0]);
+      if (b + nkw < nblk) block(b + nkw, kb[1], vb[1]);
+    }
+  }
+  __syncthreads();  // every wave has left its blocks
+  constexpr int RED = ND * 16 + 2;  // words per lane
+  float* red = reinterpret_cast<float*>(lds) + lane;
+  if (kq > 0) {
+    float* mine = red + (rb * (nkw - 1) + kq - 1) * RED * 64;
+#pragma unroll
+    for (int db = 0; db < ND; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) mine[(db * 16 + v) * 64] = oacc[db][v];
+    mine[ND * 16 * 64] = m_run;
+    mine[(ND * 16 + 1) * 64] = l_run;
+  }
+  __syncthreads();
+  if (kq > 0 || rb * 32 >= rows) return;
+  const float* others = red + rb * (nkw - 1) * RED * 64;
+  float m = m_run;
+  for (int w = 0; w < nkw - 1; ++w)
+    m = __builtin_elementwise_maximum(m, others[(w * RED + ND * 16) * 64]);
+  auto weight = [&](float mw) {
+    return mw == -__builtin_inf() ? 0.0f : __builtin_amdgcn_exp2f(mw - m);
+  };
+  const float f0 = weight(m_run);
+  l_run *= f0;
+#pragma unroll
+  for (int db = 0; db < ND; ++db)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) oacc[db][v] *= f0;
+  for (int w = 0; w < nkw - 1; ++w) {
+    const float* o = others + w * RED * 64;
+    const float f = weight(o[ND * 16 * 64]);
+    l_run = __builtin_fmaf(f, o[(ND * 16 + 1) * 64], l_run);
+#pragma unroll
+    for (int db = 0; db < ND; ++db)
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        oacc[db][v] = __builtin_fmaf(f, o[(db * 16 + v) * 64], oacc[db][v]);
+  }
+  const float l_tot = l_run + __shfl_xor(l_run, 32);
+  if (!row_ok) return;
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  uint16_t* orow = a.out + (qi * a.hq + hh) * D;
+#pragma unroll
+  for (int db = 0; db < ND; ++db)
+#pragma unroll
+    for (int gi = 0; gi < 4; ++gi) {
+      const int v = gi * 4;
+      *reinterpret_cast<u32x2*>(orow + db * 32 + gi * 8 + hb * 4) =
+          u32x2{pack2<DT>(oacc[db][v] * inv, oacc[db][v + 1] * inv),
+                pack2<DT>(oacc[db][v + 2] * inv, oacc[db][v + 3] * inv)};
+    }
+  if (hb == 0)
+    a.lse[(int64_t)hh * a.nq + qi] = l_tot > 0.0f ? m + log2f(l_tot) : -__builtin_inf();
+}
+
+template <int DT, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 4))) void
+narrow_fwd_kernel(AttnArgs a) {
+  constexpr int RED_BYTES = 3 * (D / 2 + 2) * 64 * 4, V_BYTES = 4 * 32 * D * 2;
+  __shared__ __align__(1024) char s_lds[RED_BYTES > V_BYTES ? RED_BYTES : V_BYTES];
+  __shared__ SelLds sel;
+  __shared__ int s_tokmap[KMAP_KEYS];
+  __shared__ int s_slot;
+  const int lane = threadIdx.x & 63, wv = uniform(threadIdx.x >> 6);
+  const int32_t* off = a.plan.narrow_off;
+  const int total = off[a.hkv];
+  if (total == 0) return;
+  int32_t* queue = a.plan.counter + NARROW_QUEUE_SLOT;
+  for (;;) {
+    const int w = uniform(fetch_work(queue, &s_slot));
+    if (w >= total) break;
+    const int h = head_of(off, a.hkv, w);
+    const int2 tile = a.plan.by_width[(int64_t)h * a.nq + (a.nq - 1 - (w - off[h]))];
+    load_selection(a, h, tile.x, sel);
+    const int nkeys = uniform(sel.cum[sel.n]), rows = uniform(tile.y) * a.g;
+    const int* map = nullptr;
+    if (nkeys <= KMAP_KEYS) {
+      build_token_map(sel, s_tokmap, wv, lane);
+      map = s_tokmap;
+    }
+    narrow_fwd<DT, D>(a, h, tile.x, rows, sel, map, nkeys, s_lds, wv, lane);
+  }
+  leave_queue(queue, queue + NARROW_EXIT_SLOT - NARROW_QUEUE_SLOT);
+}
+
 // MODE 0 (FWD_RUN): the run tiles of the plan (every row of a tile shares
-// one key stream).  MODE 1 (FWD_UNION): the grouped tiles (see build_union),
+// one key stream; head dims up to 64: the wide ones).  MODE 1 (FWD_UNION): the grouped tiles (see build_union),
 // run with per-row key masks; a key-centric plan does not launch it (its
 // grouped tiles' rows run as gathered tiles).  MODE 2 (FWD_GATHER): gathered
 // tiles of a key-centric plan
@@ -99,9 +300,12 @@ sel_attn_fwd_kernel(AttnArgs a) {
 
   const int tid = threadIdx.x, lane = tid & 63, wv = uniform(tid >> 6);
   const int hb = lane >> 5, l32 = lane & 31;
+  // head dims with a narrow-tile kernel leave the narrow run tiles to it
+  constexpr bool WIDE = MODE == FWD_RUN && narrow_split(D);
   const int32_t* head_off =
-      GATHER ? a.kc.fitem_off : (UNION ? a.plan.ghead_off : a.plan.head_off);
-  const int2* tiles = UNION ? a.plan.gtiles : a.plan.tiles;
+      GATHER ? a.kc.fitem_off
+             : (UNION ? a.plan.ghead_off : (WIDE ? a.plan.wide_off : a.plan.head_off));
+  const int2* tiles = UNION ? a.plan.gtiles : (WIDE ? a.plan.by_width : a.plan.tiles);
   int32_t* queue = a.plan.counter + (GATHER ? KC_QUEUE_SLOT : (UNION ? 4 : 0));
   if constexpr (GATHER) {
     if (!kc_plan_ok(a)) return;  // no key-centric part for this run: read nothing
@@ -1147,6 +1351,13 @@ __global__ __launch_bounds__(256) void kc_merge_kernel(AttnArgs a) {
 
 template <int DT, int D>
 int launch_fwd_t(const AttnArgs& a, hipStream_t st) {
+  if constexpr (narrow_split(D)) {
+    const int grid =
+        persistent_grid(reinterpret_cast<const void*>(&narrow_fwd_kernel<DT, D>), 256, 0);
+    if (grid <= 0) return LSRM_ERR_LAUNCH;
+    hipLaunchKernelGGL((narrow_fwd_kernel<DT, D>), dim3(grid), dim3(256), 0, st, a);
+    LSRM_CHECK_LAUNCH();
+  }
   const void* fn = reinterpret_cast<const void*>(&sel_attn_fwd_kernel<DT, D, FWD_RUN>);
   const int grid = persistent_grid(fn, 256, 0);
   if (grid <= 0) return LSRM_ERR_LAUNCH;

@@ -106,8 +106,8 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
   const bool backward = (flags & LSRM_PLAN_BACKWARD) != 0;
   const int tq = ROWS / g;
   bool derive = false;  // the backward's query map comes from the key-centric one
-  int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, ws,
-                           w.plan, st, true);
+  int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, NARROW_ROWS / g, ws,
+                           w.plan, st);
   if (rc) return rc;
   if (backward) {
     // dK/dV rows: the run tiles that selected a block, then the queries of

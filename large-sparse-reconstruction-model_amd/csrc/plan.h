@@ -23,7 +23,19 @@ struct TilePlan {
   int2* gtiles;          // [hkv, n_q] grouped tiles (forward plans)
   int32_t* gtile_count;  // [hkv]
   int32_t* ghead_off;    // [hkv + 1]
+  // The run tiles again, by width: those of more than narrow_rows / g queries
+  // from the front of each head's part, the narrow ones from its end
+  // backwards.
+  int2* by_width;        // [hkv, n_q]
+  int32_t* wide_off;     // [hkv + 1]
+  int32_t* narrow_off;   // [hkv + 1]
 };
+
+// Rows (queries x query heads of the kv head) up to which a run tile counts
+// as narrow: it fills at most two of a workgroup's four 32-row waves.
+constexpr int NARROW_ROWS = 64;
+// Work and exit counters of the narrow-tile kernels inside TilePlan::counter.
+constexpr int NARROW_QUEUE_SLOT = 28, NARROW_EXIT_SLOT = 30;
 
 // Marks a plan whose backward part was built: the backward kernels exit
 // without touching memory when the slot does not hold the magic word (a
@@ -41,11 +53,12 @@ struct RevMap {
 };
 
 // Workspace carving: pass a Carver with base == nullptr to size.
-// group_short: move consecutive short run tiles into grouped tiles.
+// Consecutive short run tiles move into grouped tiles; the others are also
+// listed by width (narrow: at most narrow_q queries).
 int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
                     int64_t topk_n, const int32_t* cu_q, int64_t batch,
-                    const int32_t* cu_sb, int tq, Carver& ws, TilePlan& plan,
-                    hipStream_t st, bool group_short = false);
+                    const int32_t* cu_sb, int tq, int narrow_q, Carver& ws, TilePlan& plan,
+                    hipStream_t st);
 
 // rows_are_tiles: rows are the tiles of `plan` (row r of head h reads the
 // selection of query tiles[h*nq + r].x); otherwise rows are queries, and

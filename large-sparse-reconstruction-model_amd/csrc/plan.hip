@@ -26,18 +26,19 @@ __device__ inline int wave_sum(int v) {
 
 // Exclusive scan of one value per thread over a 256-thread block; returns the
 // exclusive prefix and writes the block total to *total.
-__device__ inline int block_excl_scan(int v, int* total) {
-  __shared__ int s_w[SCAN_T / 64];
+template <class T>
+__device__ inline T block_excl_scan(T v, T* total) {
+  __shared__ T s_w[SCAN_T / 64];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  int x = v;
+  T x = v;
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    int y = __shfl_up(x, o);
+    T y = __shfl_up(x, o);
     if (lane >= o) x += y;
   }
   if (lane == 63) s_w[w] = x;
   __syncthreads();
-  int off = 0, tot = 0;
+  T off = 0, tot = 0;
 #pragma unroll
   for (int i = 0; i < SCAN_T / 64; ++i) {
     if (i < w) off += s_w[i];
@@ -48,35 +49,47 @@ __device__ inline int block_excl_scan(int v, int* total) {
   return off + x - v;
 }
 
+// The type of a scan's values: int, or a pair of counts packed in 64 bits.
+struct SplitF;
+template <class F>
+struct ScanValue {
+  using type = int32_t;
+};
+template <>
+struct ScanValue<SplitF> {
+  using type = int64_t;
+};
+template <class F>
+using scan_t = typename ScanValue<F>::type;
+
 template <class F>
 __global__ __launch_bounds__(SCAN_T) void scan_reduce(F f, int64_t n,
-                                                      int32_t* sums,
+                                                      scan_t<F>* sums,
                                                       int nchunks) {
   const int seg = blockIdx.y;
   const int64_t base = (int64_t)blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_PER;
   const int64_t lim = f.limit(seg, n);
-  int s = 0;
+  scan_t<F> s = 0;
   for (int i = 0; i < SCAN_PER; ++i) {
     const int64_t idx = base + i;
     if (idx < lim) s += f(seg, idx);
   }
-  int tot;
+  scan_t<F> tot;
   block_excl_scan(s, &tot);
   if (threadIdx.x == 0) sums[(int64_t)seg * nchunks + blockIdx.x] = tot;
 }
 
 // In-place exclusive scan of each segment's chunk sums; totals[seg] = total.
-__global__ __launch_bounds__(SCAN_T) void scan_chunks(int32_t* sums,
-                                                      int nchunks,
-                                                      int32_t* totals) {
+template <class T>
+__global__ __launch_bounds__(SCAN_T) void scan_chunks(T* sums, int nchunks, T* totals) {
   const int seg = blockIdx.x;
-  int32_t* p = sums + (int64_t)seg * nchunks;
-  int carry = 0;
+  T* p = sums + (int64_t)seg * nchunks;
+  T carry = 0;
   for (int base = 0; base < nchunks; base += SCAN_T) {
     const int i = base + threadIdx.x;
-    const int v = i < nchunks ? p[i] : 0;
-    int tot;
-    const int ex = block_excl_scan(v, &tot);
+    const T v = i < nchunks ? p[i] : T(0);
+    T tot;
+    const T ex = block_excl_scan(v, &tot);
     if (i < nchunks) p[i] = carry + ex;
     carry += tot;
   }
@@ -85,21 +98,21 @@ __global__ __launch_bounds__(SCAN_T) void scan_chunks(int32_t* sums,
 
 template <class F, class W>
 __global__ __launch_bounds__(SCAN_T) void scan_apply(F f, W w, int64_t n,
-                                                     const int32_t* sums,
+                                                     const scan_t<F>* sums,
                                                      int nchunks) {
   const int seg = blockIdx.y;
   const int64_t base = (int64_t)blockIdx.x * SCAN_CHUNK + threadIdx.x * SCAN_PER;
   const int64_t lim = f.limit(seg, n);
-  int v[SCAN_PER];
-  int s = 0;
+  scan_t<F> v[SCAN_PER];
+  scan_t<F> s = 0;
 #pragma unroll
   for (int i = 0; i < SCAN_PER; ++i) {
     const int64_t idx = base + i;
-    v[i] = idx < lim ? f(seg, idx) : 0;
+    v[i] = idx < lim ? f(seg, idx) : scan_t<F>(0);
     s += v[i];
   }
-  int tot;
-  int ex = block_excl_scan(s, &tot) + sums[(int64_t)seg * nchunks + blockIdx.x];
+  scan_t<F> tot;
+  scan_t<F> ex = block_excl_scan(s, &tot) + sums[(int64_t)seg * nchunks + blockIdx.x];
 #pragma unroll
   for (int i = 0; i < SCAN_PER; ++i) {
     const int64_t idx = base + i;
@@ -111,14 +124,14 @@ __global__ __launch_bounds__(SCAN_T) void scan_apply(F f, W w, int64_t n,
 // Runs scan_reduce / scan_chunks / scan_apply over `nseg` segments of at
 // most n elements; totals[seg] receives each segment's sum.
 template <class F, class W>
-int run_scan(F f, W w, int64_t n, int nseg, int32_t* chunk_sums,
-             int32_t* totals, hipStream_t st) {
+int run_scan(F f, W w, int64_t n, int nseg, scan_t<F>* chunk_sums,
+             scan_t<F>* totals, hipStream_t st) {
   if (n <= 0 || nseg <= 0) return LSRM_OK;
   const int nchunks = ceil_div(n, SCAN_CHUNK);
   dim3 grid(nchunks, nseg);
   hipLaunchKernelGGL((scan_reduce<F>), grid, dim3(SCAN_T), 0, st, f, n,
                      chunk_sums, nchunks);
-  hipLaunchKernelGGL(scan_chunks, dim3(nseg), dim3(SCAN_T), 0, st, chunk_sums,
+  hipLaunchKernelGGL(scan_chunks<scan_t<F>>, dim3(nseg), dim3(SCAN_T), 0, st, chunk_sums,
                      nchunks, totals);
   hipLaunchKernelGGL((scan_apply<F, W>), grid, dim3(SCAN_T), 0, st, f, w, n,
                      chunk_sums, nchunks);
@@ -412,15 +425,19 @@ struct GroupW {
     if (t == lim - 1) gs[ex + v] = (int32_t)lim;
   }
 };
-// Second pass over the groups: grouped (>= 2 run tiles) or kept.
+// Second pass over the groups: grouped (>= 2 run tiles) or kept, and whether a
+// kept tile is narrow; the two counts are scanned together, packed in 64 bits.
 struct SplitF {
+  const int2* run_tiles;
   const int32_t* gstart;
   const int32_t* n_groups;
   int64_t nq;
+  int narrow_q;
   __device__ int64_t limit(int h, int64_t) const { return n_groups[h]; }
-  __device__ int operator()(int h, int64_t s) const {
+  __device__ int64_t operator()(int h, int64_t s) const {
     const int32_t* gs = gstart + (int64_t)h * (nq + 1);
-    return gs[s + 1] - gs[s] > 1 ? 1 : 0;
+    if (gs[s + 1] - gs[s] > 1) return 1;
+    return run_tiles[(int64_t)h * nq + gs[s]].y <= narrow_q ? int64_t{1} << 32 : 0;
   }
 };
 struct SplitW {
@@ -429,37 +446,49 @@ struct SplitW {
   int64_t nq;
   int2* tiles;
   int2* gtiles;
-  __device__ void operator()(int h, int64_t s, int ex, int v, int64_t) const {
+  int2* by_width;
+  __device__ void operator()(int h, int64_t s, int64_t ex, int64_t v, int64_t) const {
     const int32_t* gs = gstart + (int64_t)h * (nq + 1);
     const int t0 = gs[s], t1 = gs[s + 1];
-    const int2 first = run_tiles[(int64_t)h * nq + t0];
-    const int2 last = run_tiles[(int64_t)h * nq + t1 - 1];
-    const int2 out = make_int2(first.x, last.x + last.y - first.x);
-    if (v)
-      gtiles[(int64_t)h * nq + ex] = out;
-    else
-      tiles[(int64_t)h * nq + (s - ex)] = out;
+    const int64_t g = (int32_t)ex, nar = ex >> 32;  // grouped, narrow tiles before
+    const int64_t at = (int64_t)h * nq;
+    const int2 first = run_tiles[at + t0];
+    if (v == 1) {
+      const int2 last = run_tiles[at + t1 - 1];
+      gtiles[at + g] = make_int2(first.x, last.x + last.y - first.x);
+      return;
+    }
+    tiles[at + (s - g)] = first;
+    by_width[at + (v ? nq - 1 - nar : s - g - nar)] = first;
   }
 };
 
-// tile_count = groups - grouped tiles (grouping) or the run count.
-__global__ void plan_offsets_kernel(const int32_t* n_groups, int32_t* tile_count,
-                                    const int32_t* gtile_count, int hkv,
-                                    int32_t* head_off, int32_t* ghead_off,
-                                    int32_t* counter) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    int acc = 0, gacc = 0;
-    head_off[0] = 0;
-    ghead_off[0] = 0;
+// The lists' counts per head from the groups and the split's totals, and the
+// heads' offsets in every list (lane i takes list i: run tiles, grouped, wide,
+// narrow).
+__global__ void plan_offsets_kernel(const int32_t* n_groups, const int64_t* split,
+                                    TilePlan plan, int hkv) {
+  if (blockIdx.x != 0) return;
+  if (threadIdx.x < 4) {
+    const int i = threadIdx.x;
+    int32_t* off = i == 0 ? plan.head_off
+                          : (i == 1 ? plan.ghead_off : (i == 2 ? plan.wide_off : plan.narrow_off));
+    int acc = 0;
+    off[0] = 0;
     for (int h = 0; h < hkv; ++h) {
-      const int g = gtile_count[h];
-      const int c = n_groups ? n_groups[h] - g : tile_count[h];
-      tile_count[h] = c;
+      int c = 0;
+      if (n_groups) {
+        const int g = (int32_t)split[h], nar = (int)(split[h] >> 32), kept = n_groups[h] - g;
+        c = i == 0 ? kept : (i == 1 ? g : (i == 2 ? kept - nar : nar));
+      }
+      if (i == 0) plan.tile_count[h] = c;
+      if (i == 1) plan.gtile_count[h] = c;
       acc += c;
-      gacc += g;
-      head_off[h + 1] = acc;
-      ghead_off[h + 1] = gacc;
+      off[h + 1] = acc;
     }
+  }
+  int32_t* counter = plan.counter;
+  if (threadIdx.x == 0) {
     for (int i = 0; i < PLAN_BWD_SLOT; ++i) counter[i] = 0;
     counter[PLAN_BWD_SLOT] = 0;  // set again by mark_backward_plan
     counter[PLAN_KC_SLOT] = 0;   // set again by the key-centric part
@@ -478,34 +507,31 @@ int mark_backward_plan(int32_t* counter, hipStream_t st) {
 
 int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
                     int64_t topk_n, const int32_t* cu_q, int64_t batch,
-                    const int32_t* cu_sb, int tq, Carver& ws, TilePlan& plan,
-                    hipStream_t st, bool group_short) {
+                    const int32_t* cu_sb, int tq, int narrow_q, Carver& ws, TilePlan& plan,
+                    hipStream_t st) {
   uint8_t* brk = ws.take<uint8_t>((size_t)(hkv * nq));
   int32_t* run_start = ws.take<int32_t>((size_t)(hkv * (nq + 1)));
   int32_t* n_runs = ws.take<int32_t>((size_t)hkv);
-  int32_t* sums = ws.take<int32_t>((size_t)scan_sums_size(nq, hkv));
-  plan.tiles = ws.take<int2>((size_t)(hkv * (nq > 0 ? nq : 1)));
+  int64_t* split_sums = ws.take<int64_t>((size_t)scan_sums_size(nq, hkv));
+  int32_t* sums = reinterpret_cast<int32_t*>(split_sums);  // the 32-bit scans' before
+  const size_t n_tiles = (size_t)(hkv * (nq > 0 ? nq : 1));
+  plan.tiles = ws.take<int2>(n_tiles);
   plan.tile_count = ws.take<int32_t>((size_t)hkv);
   plan.head_off = ws.take<int32_t>((size_t)(hkv + 1));
   plan.counter = ws.take<int32_t>(64);
   plan.gtile_count = ws.take<int32_t>((size_t)hkv);
   plan.ghead_off = ws.take<int32_t>((size_t)(hkv + 1));
-  plan.gtiles = nullptr;
-  int2* run_tiles = plan.tiles;
-  int32_t* run_count = plan.tile_count;
-  int32_t* gstart = nullptr;
-  int32_t* n_groups = nullptr;
-  if (group_short) {
-    plan.gtiles = ws.take<int2>((size_t)(hkv * (nq > 0 ? nq : 1)));
-    run_tiles = ws.take<int2>((size_t)(hkv * (nq > 0 ? nq : 1)));
-    run_count = ws.take<int32_t>((size_t)hkv);
-    gstart = ws.take<int32_t>((size_t)(hkv * (nq + 1)));
-    n_groups = ws.take<int32_t>((size_t)hkv);
-  }
+  plan.wide_off = ws.take<int32_t>((size_t)(hkv + 1));
+  plan.narrow_off = ws.take<int32_t>((size_t)(hkv + 1));
+  plan.gtiles = ws.take<int2>(n_tiles);
+  plan.by_width = ws.take<int2>(n_tiles);
+  int2* run_tiles = ws.take<int2>(n_tiles);
+  int32_t* run_count = ws.take<int32_t>((size_t)hkv);
+  int32_t* gstart = ws.take<int32_t>((size_t)(hkv * (nq + 1)));
+  int32_t* n_groups = ws.take<int32_t>((size_t)hkv);
+  int64_t* split = ws.take<int64_t>((size_t)hkv);
   if (!ws.base || ws.dry) return LSRM_OK;
   if (!ws.ok()) return LSRM_ERR_WORKSPACE;
-  int rc0 = launch_zero_i32(plan.gtile_count, hkv, st);
-  if (rc0) return rc0;
 
   if (nq > 0) {
     dim3 grid(ceil_div(nq, 256), (unsigned)hkv);
@@ -542,29 +568,22 @@ int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
                   EmitTilesW{run_start, run_tiles, nq, tq}, nq, (int)hkv, sums,
                   run_count, st);
     if (rc) return rc;
-    if (group_short) {
-      const int short_q = tq / 4 > 1 ? tq / 4 : 1;
-      const int window_q = (3 * tq) / 4 > 1 ? (3 * tq) / 4 : 1;
-      // brk is free again: it takes the group starts
-      hipLaunchKernelGGL(group_breaks_kernel, grid, dim3(256), 0, st, run_tiles, run_count,
-                         cu_q, batch, topk, nq, (int)topk_n, short_q, window_q, brk);
-      LSRM_CHECK_LAUNCH();
-      rc = run_scan(GroupF{brk, run_count, nq},
-                    GroupW{gstart, nq}, nq, (int)hkv, sums, n_groups, st);
-      if (rc) return rc;
-      rc = run_scan(SplitF{gstart, n_groups, nq},
-                    SplitW{run_tiles, gstart, nq, plan.tiles, plan.gtiles}, nq, (int)hkv,
-                    sums, plan.gtile_count, st);
-      if (rc) return rc;
-    }
-  } else {
-    int rc = launch_zero_i32(plan.tile_count, hkv, st);
+    const int short_q = tq / 4 > 1 ? tq / 4 : 1;
+    const int window_q = (3 * tq) / 4 > 1 ? (3 * tq) / 4 : 1;
+    // brk is free again: it takes the group starts
+    hipLaunchKernelGGL(group_breaks_kernel, grid, dim3(256), 0, st, run_tiles, run_count,
+                       cu_q, batch, topk, nq, (int)topk_n, short_q, window_q, brk);
+    LSRM_CHECK_LAUNCH();
+    rc = run_scan(GroupF{brk, run_count, nq}, GroupW{gstart, nq}, nq, (int)hkv, sums, n_groups,
+                  st);
     if (rc) return rc;
-    n_groups = nullptr;
+    rc = run_scan(SplitF{run_tiles, gstart, n_groups, nq, narrow_q},
+                  SplitW{run_tiles, gstart, nq, plan.tiles, plan.gtiles, plan.by_width}, nq,
+                  (int)hkv, split_sums, split, st);
+    if (rc) return rc;
   }
-  hipLaunchKernelGGL(plan_offsets_kernel, dim3(1), dim3(64), 0, st,
-                     nq > 0 ? n_groups : nullptr, plan.tile_count, plan.gtile_count, (int)hkv,
-                     plan.head_off, plan.ghead_off, plan.counter);
+  hipLaunchKernelGGL(plan_offsets_kernel, dim3(1), dim3(64), 0, st, nq > 0 ? n_groups : nullptr,
+                     split, plan, (int)hkv);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }

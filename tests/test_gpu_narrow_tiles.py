@@ -1,0 +1,88 @@
+"""Run tiles of at most 64 rows at head dim 32, split over the keys between the
+waves (forward and dQ): tile widths around 32 and 64 rows, key streams around
+the 32-key blocks, one wave's turn and the token map's limit, empty streams,
+repeated blocks, and scores that keep raising the running maximum, against the
+fp32 oracle; run to run bitwise."""
+
+import numpy as np
+import pytest
+import torch
+
+import lsrm_hip as H
+from helpers import assert_attn_close
+from oracle.attention import sel_attn_ref
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _grad_close(a, b, dtype, what):
+    # A stream of a few keys gathers the gradients of all its rows, so sizes
+    # vary: the suite's tolerance for values of size 1, and beyond it two
+    # roundings (P or dS, then the result) of half a unit in the last place
+    # each, relative to the value.
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    a, b = a.float().cpu(), b.detach()
+    assert torch.isfinite(a).all(), what
+    assert ((a - b).abs() <= 2e-2 + ulp * b.abs()).all(), \
+        f"{what}: {float(((a - b).abs() - ulp * b.abs()).max()):.3e}"
+    assert float((a - b).abs().mean()) <= 2e-3 + ulp * float(b.abs().mean())
+
+
+@pytest.mark.parametrize("keys", [1, 31, 33, 128, 129, 257, 2047, 2100])
+@pytest.mark.parametrize("g,dtype", [(1, torch.bfloat16), (4, torch.float16),
+                                     (16, torch.bfloat16)])
+@pytest.mark.parametrize("scores", ["plain", "rising"])
+def test_narrow_tiles(keys, g, dtype, scores):
+    gen = torch.Generator().manual_seed(keys * 7 + g)
+    d, hkv, topk = 32, 2, 3
+    # widths in queries; neighbours of 8 or more queries share no block, so
+    # they are not grouped
+    lens = [w for w in (33, 64, 32, 9, 65, 31, 40, 8) if w * g <= 256] or [4, 2, 8, 3, 9, 1]
+    lens = lens * 2
+    # every third block holds the rest of the keys of a stream, the others few
+    sizes = [max(1, keys - 2), 1, 1] * len(lens)
+    n = sum(lens)
+    nk = sum(sizes)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(sizes)]), dtype=torch.int32)
+    nb = len(sizes)
+    rows = torch.stack([torch.arange(3) + 3 * i for i in range(len(lens))])
+    if keys < 3:
+        rows[:, 1:] = -1
+    rows[1, 1:] = -1
+    rows[1, 0] = -1                    # a tile that attends nothing
+    rows[2, 1] = rows[2, 0]            # a block listed twice
+    rows = rows.repeat_interleave(torch.tensor(lens), 0).expand(hkv, -1, -1).to(torch.int32)
+    cu_sb = torch.tensor([0, nb], dtype=torch.int32)
+    cu_q = torch.tensor([0, n], dtype=torch.int32)
+    q = (0.5 * torch.randn(n, hkv * g, d, generator=gen)).to(dtype)
+    do = (0.5 * torch.randn(n, hkv * g, d, generator=gen)).to(dtype)
+    k, v = ((0.5 * torch.randn(nk, hkv, d, generator=gen)).to(dtype) for _ in range(2))
+    if scores == "rising":  # the maximum moves by more than the rescaling step
+        q = (q.abs() + 0.5).to(dtype)
+        ramp = torch.linspace(-6, 6, nk)[:, None, None]
+        k = (ramp + 0.1 * k.float()).to(dtype)
+    scale = d ** -0.5
+    rows = rows.contiguous()
+    dev = [t.to(DEV) for t in (q, k, v, rows, cu_sb, cu, cu_q)]
+    plan = H.SelAttnPlan(q.shape, k.shape, *dev[3:], backward=True)
+    got = []
+    for _ in range(2):
+        o, lse = plan.fwd(*dev[:3], scale)
+        got.append((o, lse) + plan.bwd(do.to(DEV), *dev[:3], o, lse, scale))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+    o, lse, dq, dk, dv, delta = got[0]
+    qf, kf, vf = (t.float().requires_grad_() for t in (q, k, v))
+    ref, lse_ref = sel_attn_ref(qf, kf, vf, rows, cu_sb, cu, cu_q, scale)
+    ref.backward(do.float())
+    assert_attn_close(o, ref.detach(), "out")
+    fin = torch.isfinite(lse_ref)
+    assert torch.equal(torch.isfinite(lse.cpu()), fin)
+    # 16-bit inputs, fp32 products: a score of size s is off by under s * 2^-18
+    err = (lse.cpu()[fin] - lse_ref.detach()[fin]).abs()
+    assert float(err.max()) <= 2e-2
+    delta_ref = (o.float().cpu() * do.float()).sum(-1).transpose(0, 1)
+    torch.testing.assert_close(delta.cpu(), delta_ref, rtol=1e-4, atol=1e-4)
+    _grad_close(dq, qf.grad, dtype, "dq")
+    _grad_close(dk, kf.grad, dtype, "dk")
+    _grad_close(dv, vf.grad, dtype, "dv")
