@@ -1222,8 +1222,7 @@ sel_attn_dkdv_kernel(AttnArgs a) {
     __syncthreads();
   }
   };
-  // (a key-centric plan may list queries of run tiles too)
-  if (a.kc.fitems || uniform(a.plan.ghead_off[a.hkv]) > 0)
+  if (uniform(*a.qmap_n) > 0)
     items_loop(Phase<1>{});
   else
     items_loop(Phase<0>{});

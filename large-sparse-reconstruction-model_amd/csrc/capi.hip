@@ -313,6 +313,9 @@ int attn_setup(const void* q, const void* k, const void* v, int dtype,
   a.plan = w.plan;
   a.rev = w.rev;
   a.qrev = w.qrev;
+  a.qmap_n = dkdv_packed_q((flags & LSRM_PLAN_KEY_CENTRIC) != 0, ROWS / g) > 0
+                 ? cu_seqlens_q + batch
+                 : w.plan.ghead_off + hkv;
   a.items = w.items;
   a.kc = w.kc;
   a.kc_marker = kc_plan_marker(flags, (int)head_dim);
