@@ -9,6 +9,8 @@
 // so the sum is a fixed function of the pooled means), then take the forced
 // blocks followed by the best remaining blocks under (score descending,
 // block id ascending).  Selected ids are written ascending, -1 padded.
+#include <type_traits>
+
 #include "common.h"
 
 namespace lsrm {
@@ -34,11 +36,33 @@ constexpr int SEL_MAXK = 256;
 // multiply-adds (the kernel is bound by the fp64 FMA rate, not by LDS).
 // Converting each element once and the order of the fused multiply-adds
 // leave every score a fixed function of the pooled means.
+//
+// With `keys`, the kernel also writes for every row and class of eight columns
+// (those of one thread: a tile's columns tx + 16 j) the largest score, rounded
+// down to fp32, as an order-preserving key (NaN scores left out; 0 for a class
+// without a score): [hkv, nb, tiles, 16], read by topk_bound_kernel.
 constexpr int SCORE_TILE = 128;
 constexpr int SCORE_DC = 16;
+constexpr int SCORE_CLASSES = 16;  // per tile and row
+
+// Order-preserving key of an fp32 value, and the largest fp32 value <= x.
+__device__ inline uint32_t f32_key(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
+}
+__device__ inline float key_f32(uint32_t k) {
+  return __uint_as_float(k & 0x80000000u ? k ^ 0x80000000u : ~k);
+}
+__device__ inline float f32_below(double x) {
+  const float f = (float)x;
+  if (!((double)f > x)) return f;
+  const uint32_t u = __float_as_uint(f);
+  return __uint_as_float((u << 1) == 0 ? 0x80000001u : (u & 0x80000000u ? u + 1 : u - 1));
+}
+
 __global__ __launch_bounds__(256) void score_kernel(
     const float* __restrict__ pq, const float* __restrict__ pk, int64_t nb,
-    int hq, int hkv, int d, double* __restrict__ scores) {
+    int hq, int hkv, int d, double* __restrict__ scores, uint32_t* __restrict__ keys) {
   __shared__ double sq[SCORE_DC][SCORE_TILE + 1];
   __shared__ double sk[SCORE_DC][SCORE_TILE + 1];
   const int h = blockIdx.z;
@@ -112,6 +136,15 @@ __global__ __launch_bounds__(256) void score_kernel(
     for (int j = 0; j < 8; ++j) {
       const int64_t c = c0 + tx + 16 * j;
       if (c < nb) out[c] = acc[i][j];
+    }
+    if (keys) {
+      // (fmax leaves a NaN out; NaN only if every column is)
+      double best = __builtin_nan("");
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (c0 + tx + 16 * j < nb) best = __builtin_fmax(best, acc[i][j]);
+      keys[(((int64_t)h * nb + b) * gridDim.x + blockIdx.x) * SCORE_CLASSES + tx] =
+          best == best ? f32_key(f32_below(best)) : 0u;
     }
   }
 }
@@ -457,123 +490,172 @@ __global__ __launch_bounds__(256) void topk_wave_kernel(
   fill_token_rows(dst, total, ord, topk, lane, 64);
 }
 
-// One workgroup per (kv head, query block) row for rows of up to 4 * 64 * M
-// candidates: the forced blocks are taken first; each wave keeps a quarter
-// of the row in registers (M per lane) and lists its best R = k - forced
-// candidates (score descending, id ascending; wave_best_r); the four lists
-// are then merged by rank.  Every member of the row's best R is among its
-// quarter's best R, so the result equals a selection over the whole row.
-template <int M>
-__global__ __launch_bounds__(256) void topk_split_kernel(
-    const double* __restrict__ scores, int64_t nb,
-    const int32_t* __restrict__ cu_sb, int64_t batch,
-    const int32_t* __restrict__ cu_blk, int64_t n_tokens, int topk,
-    const int32_t* __restrict__ forced, int n_forced, int force_self,
-    int32_t* __restrict__ topk_idx, int32_t* __restrict__ compact) {
-  __shared__ int s_forced[SEL_MAXK];
-  __shared__ double s_ls[4][64];  // each wave's picks, best first: score, id
-  __shared__ int s_li[4][64];
-  __shared__ double s_cs[4][64];  // each wave's threshold survivors
-  __shared__ int s_ci[4][64];
-  __shared__ int s_nw[4];
-  __shared__ int s_sel[SEL_MAXK];
-  __shared__ int s_out[SEL_MAXK];
-  __shared__ int s_nf;
+// One wave per (query block, kv head) row of up to 64 * NM / 16 score tiles:
+// the row's classes (score_kernel's keys; those of tiles inside the row's batch
+// element) give a lower bound of its topk-th best score -- the largest value
+// that at least topk class maxima reach, and these are distinct columns -- and
+// only the columns that reach it are listed (about topk of them, at most eight
+// per class that reaches the bound) and ranked by wave_best_r.  The forced
+// blocks are taken first and count among the topk.  More than BOUND_CAP such
+// columns (ties in great number) take one scan of the row per pick.
+// Bound by reading the scores once (the row's arithmetic is a third of that):
+// 4 x 4881 rows of 4881 scores, top-32, 465 us with four waves per row that
+// each listed their quarter's best, 286 us here (763 MB of scores read and 268 MB of
+// token rows written: 3.8 TB/s).
+constexpr int BOUND_CAP = 1024;
+
+template <int NM>
+__global__ __launch_bounds__(64) void topk_bound_kernel(
+    const double* __restrict__ scores, const uint32_t* __restrict__ keys, int ntile, int64_t nb,
+    const int32_t* __restrict__ cu_sb, int64_t batch, const int32_t* __restrict__ cu_blk,
+    int64_t n_tokens, int topk, const int32_t* __restrict__ forced, int n_forced,
+    int force_self, int32_t* __restrict__ topk_idx, int32_t* __restrict__ compact) {
+  __shared__ int s_id[BOUND_CAP];
+  __shared__ double s_cs[64];
+  __shared__ int s_ci[64], s_at[64], s_sel[64], s_out[64];
   const int h = blockIdx.y;
   const int64_t b = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = threadIdx.x;
   const int64_t e = upper_index(cu_sb, 0, batch + 1, b);
   int32_t* crow = compact + ((int64_t)h * nb + b) * topk;
   if (e < 0 || e >= batch || b >= cu_sb[e + 1]) {
     clear_block_rows(cu_blk, b, n_tokens, topk, crow, topk_idx + (int64_t)h * n_tokens * topk,
-                     tid, 256);
+                     lane, 64);
     return;
   }
   const int64_t cs = cu_sb[e];
   const int nbb = (int)(cu_sb[e + 1] - cs);
   const double* row = scores + ((int64_t)h * nb + b) * nb + cs;
-  const int kmax = topk < nbb ? topk : nbb;
+  const uint32_t* krow = keys + ((int64_t)h * nb + b) * ntile * SCORE_CLASSES;
+  uint32_t key[NM];
+#pragma unroll
+  for (int m = 0; m < NM; ++m) {
+    const int ci = lane + 64 * m, tile = ci / SCORE_CLASSES;
+    const int64_t c0 = (int64_t)tile * SCORE_TILE;
+    const int64_t c1 = c0 + SCORE_TILE < nb ? c0 + SCORE_TILE : nb;
+    key[m] = tile < ntile && c0 >= cs && c1 <= cs + nbb ? krow[ci] : 0u;
+  }
   // Forced blocks in order, distinct, valid, at most kmax.
-  if (tid == 0) {
-    int n = 0;
-    auto add = [&](int id) {
-      if (n >= kmax || id < 0 || id >= nbb) return;
-      for (int t = 0; t < n; ++t)
-        if (s_forced[t] == id) return;
-      s_forced[n++] = id;
-    };
-    if (force_self) add((int)(b - cs));
-    for (int f = 0; f < n_forced; ++f) add(forced[f]);
-    s_nf = n;
+  const int kmax = topk < nbb ? topk : nbb;
+  int nf = 0;
+  auto add = [&](int id) {  // wave-uniform
+    if (nf >= kmax || id < 0 || id >= nbb) return;
+    if (__ballot(lane < nf && s_sel[lane] == id)) return;
+    if (lane == 0) s_sel[nf] = id;
+    ++nf;
+    __syncthreads();
+  };
+  if (force_self) add((int)(b - cs));
+  for (int f = 0; f < n_forced; ++f) add(forced[f]);
+  const int r_need = kmax - nf;
+  auto is_forced = [&](int id) {
+    for (int t = 0; t < nf; ++t)
+      if (s_sel[t] == id) return true;
+    return false;
+  };
+  // The bound, to 24 bits of the key.
+  uint32_t kb = 0u;
+  for (int bit = 31; bit >= 8; --bit) {
+    const uint32_t tryk = kb | (1u << bit);
+    int reach = 0;
+#pragma unroll
+    for (int m = 0; m < NM; ++m) reach += __popcll(__ballot(key[m] >= tryk));
+    if (reach >= topk) kb = tryk;
+  }
+  const double bound =
+      kb > f32_key(-__builtin_inff()) ? (double)key_f32(kb) : -__builtin_inf();
+  // The columns that reach it, in ascending order.
+  int n = 0;
+  constexpr int U = 8;
+  for (int base = 0; base < nbb; base += 64 * U) {
+    double x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = base + 64 * u + lane;
+      x[u] = i < nbb ? row[i] : __builtin_nan("");
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = base + 64 * u + lane;
+      if (x[u] != x[u]) x[u] = -__builtin_inf();  // NaN ranks lowest
+      const bool in = i < nbb && x[u] >= bound;
+      const unsigned long long m = __ballot(in);
+      if (m == 0ull) continue;
+      const int pos = n + __popcll(m & ((1ull << lane) - 1ull));
+      if (in && pos < BOUND_CAP) s_id[pos] = i;
+      n += __popcll(m);
+    }
   }
   __syncthreads();
-  const int nf = s_nf, r_need = kmax - nf;
-  // This wave's quarter [q0, q0 + 64 M) of the row.
-  const int q0 = wv * 64 * M;
-  double v[M];
-  uint32_t taken = 0u;  // bit m: candidate q0 + lane + 64 m is unavailable
+  // wave_best_r over the listed columns: their places ascend with their ids.
+  auto best = [&](auto per) {
+    constexpr int M = decltype(per)::value;
+    double v[M];
+    uint32_t taken = 0u;
 #pragma unroll
-  for (int m = 0; m < M; ++m) {
-    const int i = q0 + lane + 64 * m;
-    if (i < nbb) {
-      const double x = row[i];
-      v[m] = (x != x) ? -__builtin_inf() : x;
-    } else {
+    for (int m = 0; m < M; ++m) {
+      const int at = lane + 64 * m;
       v[m] = -__builtin_inf();
-      taken |= 1u << m;
-    }
-  }
-  for (int t = 0; t < nf; ++t) {
-    const int i = s_forced[t] - q0;
-    if (i >= 0 && i < 64 * M && (i & 63) == lane) taken |= 1u << (i >> 6);
-  }
-  const int nw = wave_best_r<M>(v, taken, q0, r_need, s_ls[wv], s_li[wv], s_cs[wv], s_ci[wv]);
-  if (lane == 0) s_nw[wv] = nw;
-  if (tid < nf) s_sel[tid] = s_forced[tid];
-  __syncthreads();
-  // Merge: the rank of each list entry in the union of the four lists
-  // (each sorted best first) is its index plus, for every other list, the
-  // number of that list's entries better than it (a binary search); the
-  // entries of rank < r_need are the row's best r_need, since each member
-  // of those is among its own quarter's best r_need.
-  if (lane < nw) {
-    const double es = s_ls[wv][lane];
-    const int ei = s_li[wv][lane];
-    int rank = lane;
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      if (t == wv) continue;
-      int lo = 0, hi = s_nw[t];
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (sel_better(s_ls[t][mid], s_li[t][mid], es, ei))
-          lo = mid + 1;
-        else
-          hi = mid;
+      if (at < n) {  // (read again: a few cached lines)
+        const double x = row[s_id[at]];
+        if (x == x) v[m] = x;
       }
-      rank += lo;
+      if (at >= n || is_forced(s_id[at])) taken |= 1u << m;
     }
-    if (rank < r_need) s_sel[nf + rank] = ei;
+    const int nw = wave_best_r<M>(v, taken, 0, r_need, nullptr, s_at, s_cs, s_ci);
+    __syncthreads();
+    if (lane < nw) s_sel[nf + lane] = s_id[s_at[lane]];
+  };
+  if (n <= 256) {
+    best(std::integral_constant<int, 4>{});
+  } else if (n <= BOUND_CAP) {
+    best(std::integral_constant<int, BOUND_CAP / 64>{});
+  } else {
+    double ps = 0.0;
+    int pi = -1;  // the pick before (none)
+    for (int r = 0; r < r_need; ++r) {
+      double bs = -__builtin_inf();
+      int bi = INT32_MAX;
+      for (int i = lane; i < nbb; i += 64) {
+        double x = row[i];
+        if (x != x) x = -__builtin_inf();
+        if ((pi < 0 || sel_better(ps, pi, x, i)) && sel_better(x, i, bs, bi) && !is_forced(i)) {
+          bs = x;
+          bi = i;
+        }
+      }
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const double os = __shfl_xor(bs, o);
+        const int oi = __shfl_xor(bi, o);
+        if (sel_better(os, oi, bs, bi)) {
+          bs = os;
+          bi = oi;
+        }
+      }
+      ps = bs;
+      pi = bi;
+      if (lane == 0) s_ci[r] = bi;
+    }
+    __syncthreads();
+    if (lane < r_need) s_sel[nf + lane] = s_ci[lane];
   }
-  __syncthreads();
   // Ascending order by rank (ids are distinct), -1 padding.
-  for (int j = tid; j < topk; j += 256) s_out[j] = -1;
+  if (lane < topk) s_out[lane] = -1;
   __syncthreads();
-  for (int j = tid; j < kmax; j += 256) {
-    const int id = s_sel[j];
+  if (lane < kmax) {
+    const int id = s_sel[lane];
     int r = 0;
     for (int m = 0; m < kmax; ++m) r += s_sel[m] < id;
     s_out[r] = id;
   }
   __syncthreads();
-  for (int j = tid; j < topk; j += 256) crow[j] = s_out[j];
+  if (lane < topk) crow[lane] = s_out[lane];
   int64_t t0 = cu_blk[b], t1 = cu_blk[b + 1];
   t0 = t0 < 0 ? 0 : (t0 > n_tokens ? n_tokens : t0);
   t1 = t1 < t0 ? t0 : (t1 > n_tokens ? n_tokens : t1);
-  int32_t* dst = topk_idx + ((int64_t)h * n_tokens + t0) * topk;
-  const int64_t total = (t1 - t0) * topk;
-  fill_token_rows(dst, total, s_out, topk, tid, 256);
+  fill_token_rows(topk_idx + ((int64_t)h * n_tokens + t0) * topk, (t1 - t0) * topk, s_out, topk,
+                  lane, 64);
 }
 
 // Rows of tokens outside every block ([0, cu_blk[0]) and [cu_blk[nb], n),
@@ -599,7 +681,13 @@ struct SelectWs {
   float* partial;
   int32_t* first;
   double* scores;
+  uint32_t* keys;  // class maxima of the scores (bounded_rows)
 };
+
+// Rows of this many blocks are selected behind a bound from class maxima (for
+// topk <= 64): below, one wave holds the row in registers; above, the classes
+// no longer fit a wave's registers.
+inline bool bounded_rows(int64_t nb) { return nb > 64 * 32 && nb <= 4 * 64 * 32; }
 
 void carve_select(Carver& ws, int64_t n, int64_t nb, int64_t hq, int64_t hkv,
                   int64_t d, SelectWs& s) {
@@ -610,6 +698,9 @@ void carve_select(Carver& ws, int64_t n, int64_t nb, int64_t hq, int64_t hkv,
                                       (hq > hkv ? hq : hkv) * d));
   s.first = ws.take<int32_t>((size_t)pool_first_count(n));
   s.scores = ws.take<double>((size_t)(hkv * nbc * nbc));
+  s.keys = bounded_rows(nb) ? ws.take<uint32_t>((size_t)(hkv * nbc * SCORE_CLASSES *
+                                                         ceil_div(nbc, SCORE_TILE)))
+                            : nullptr;
 }
 
 }  // namespace lsrm
@@ -680,7 +771,7 @@ static int select_blocks_impl(const void* q, const void* k, const float* pooled_
   const unsigned nt = (unsigned)ceil_div(n_blocks, SCORE_TILE);
   hipLaunchKernelGGL(score_kernel, dim3(nt, nt, (unsigned)hkv), dim3(256), 0,
                      st, s.pq, pk, n_blocks, (int)hq, (int)hkv,
-                     (int)head_dim, s.scores);
+                     (int)head_dim, s.scores, topk <= 64 ? s.keys : nullptr);
   LSRM_CHECK_LAUNCH();
   const unsigned rows4 = (unsigned)ceil_div(n_blocks * hkv, 4);
 #define LSRM_TOPK_WAVE(M)                                                     \
@@ -696,23 +787,19 @@ static int select_blocks_impl(const void* q, const void* k, const float* pooled_
     LSRM_TOPK_WAVE(16);
   else if (n_blocks <= 64 * 32)
     LSRM_TOPK_WAVE(32);
-  else if (n_blocks <= 4 * 64 * 32 && topk <= 64) {
-#define LSRM_TOPK_SPLIT(M)                                                                \
-  hipLaunchKernelGGL(topk_split_kernel<M>, dim3((unsigned)n_blocks, (unsigned)hkv),      \
-                     dim3(256), 0, st, s.scores, n_blocks, cu_seqblocks, batch,            \
-                     cu_block_tokens, n_tokens, (int)topk, forced_blocks, (int)n_forced,   \
-                     force_self, topk_idx, topk_compact)
-    if (n_blocks <= 4 * 64 * 12)
-      LSRM_TOPK_SPLIT(12);
-    else if (n_blocks <= 4 * 64 * 16)
-      LSRM_TOPK_SPLIT(16);
-    else if (n_blocks <= 4 * 64 * 20)
-      LSRM_TOPK_SPLIT(20);
-    else if (n_blocks <= 4 * 64 * 24)
-      LSRM_TOPK_SPLIT(24);
+  else if (bounded_rows(n_blocks) && topk <= 64) {
+#define LSRM_TOPK_BOUND(NM)                                                               \
+  hipLaunchKernelGGL(topk_bound_kernel<NM>, dim3((unsigned)n_blocks, (unsigned)hkv),     \
+                     dim3(64), 0, st, s.scores, s.keys, (int)nt, n_blocks, cu_seqblocks,   \
+                     batch, cu_block_tokens, n_tokens, (int)topk, forced_blocks,           \
+                     (int)n_forced, force_self, topk_idx, topk_compact)
+    if (nt * SCORE_CLASSES <= 64 * 8)
+      LSRM_TOPK_BOUND(8);
+    else if (nt * SCORE_CLASSES <= 64 * 12)
+      LSRM_TOPK_BOUND(12);
     else
-      LSRM_TOPK_SPLIT(32);
-#undef LSRM_TOPK_SPLIT
+      LSRM_TOPK_BOUND(16);
+#undef LSRM_TOPK_BOUND
   } else
     hipLaunchKernelGGL(topk_kernel, dim3((unsigned)n_blocks, (unsigned)hkv),
                        dim3(256), 0, st, s.scores, n_blocks, cu_seqblocks,
