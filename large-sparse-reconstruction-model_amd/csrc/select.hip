@@ -22,28 +22,33 @@ int launch_block_mean_pool(const void* x, int x_dtype, int64_t n, int64_t ch,
 int64_t pool_partial_rows(int64_t n, int64_t nb);
 int64_t pool_first_count(int64_t n);
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
 constexpr int SEL_MAXD = 128;
 constexpr int SEL_CAND_LDS = 8192;      // candidate scores cached in LDS
 constexpr int SEL_MAX_CAND = 65536;     // bitmap capacity (blocks per batch)
 constexpr int SEL_MAXK = 256;
 
-// scores[h, b, c] for b, c in [0, nb): 128x128 tile per workgroup, 8x8 per
-// thread (rows ty + 16 i, columns tx + 16 j), fp64 accumulation over (g, d)
-// in order.  The pooled rows are staged in LDS as doubles, SCORE_DC head-dim
-// columns at a time and transposed ([column][row]), so a thread's eight row
-// operands are wave-broadcast reads and its eight column operands are
-// conflict-free reads of consecutive doubles: 16 LDS reads per 64 fused
-// multiply-adds (the kernel is bound by the fp64 FMA rate, not by LDS).
-// Converting each element once and the order of the fused multiply-adds
-// leave every score a fixed function of the pooled means.
+// scores[h, b, c] for b, c in [0, nb): 128 rows x 64 columns per workgroup,
+// 32x64 per wave as 2x4 blocks of v_mfma_f64_16x16x4 (bound by that
+// instruction's rate, the fp64 rate of the chip; a wave's 64 accumulator
+// registers leave room for four waves per SIMD, which hide the short loop's
+// loads -- with 64x64 per wave and two waves it was busy 47% of the time; the vector form with 8x8 scores per thread needed
+// 16 LDS reads per 64 fused multiply-adds and reached a third of it: 423 ->
+// 337 us for 4 heads x 4881 x 4881 x 64).  The instruction adds its four
+// products one by one in ascending order, each a fused multiply-add (checked
+// bit for bit against that chain), so a score is the same fixed function of
+// the pooled means: fp64 accumulation over (g, d) in order.  The pooled rows
+// are staged in LDS as doubles, SCORE_DC head-dim columns at a time.
 //
-// With `keys`, the kernel also writes for every row and class of eight columns
-// (those of one thread: a tile's columns tx + 16 j) the largest score, rounded
+// With `keys`, the kernel also writes for every row and class of four columns
+// (16 apart in a tile) the largest score, rounded
 // down to fp32, as an order-preserving key (NaN scores left out; 0 for a class
-// without a score): [hkv, nb, tiles, 16], read by topk_bound_kernel.
-constexpr int SCORE_TILE = 128;
+// without a score): [hkv, nb, column tiles, 16],
+// read by topk_bound_kernel.
+constexpr int SCORE_ROWS = 128, SCORE_COLS = 64;
 constexpr int SCORE_DC = 16;
-constexpr int SCORE_CLASSES = 16;  // per tile and row
+constexpr int SCORE_CLASSES = 16;  // per column tile and row
 
 // Order-preserving key of an fp32 value, and the largest fp32 value <= x.
 __device__ inline uint32_t f32_key(float f) {
@@ -63,90 +68,129 @@ __device__ inline float f32_below(double x) {
 __global__ __launch_bounds__(256) void score_kernel(
     const float* __restrict__ pq, const float* __restrict__ pk, int64_t nb,
     int hq, int hkv, int d, double* __restrict__ scores, uint32_t* __restrict__ keys) {
-  __shared__ double sq[SCORE_DC][SCORE_TILE + 1];
-  __shared__ double sk[SCORE_DC][SCORE_TILE + 1];
+  // [column][row]: an operand is 16 rows of 4 columns.  Neighbouring columns lie
+  // half the banks apart, so a read's two runs of 16 doubles do not meet, and
+  // column pair p shifts its rows by XOR 4 p, so that the 16 columns x 4 rows
+  // of a staging write spread over the banks as well.
+  __shared__ double sq[SCORE_DC][SCORE_ROWS + 16];
+  __shared__ double sk[SCORE_DC][SCORE_COLS + 16];
   const int h = blockIdx.z;
-  const int64_t b0 = (int64_t)blockIdx.y * SCORE_TILE;
-  const int64_t c0 = (int64_t)blockIdx.x * SCORE_TILE;
+  const int64_t b0 = (int64_t)blockIdx.y * SCORE_ROWS;
+  const int64_t c0 = (int64_t)blockIdx.x * SCORE_COLS;
   const int g_n = hq / hkv;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  double acc[8][8];
+  const int lane = threadIdx.x & 63, r0 = (threadIdx.x >> 6) * 32;  // the wave's rows
+  const int l16 = lane & 15, l4 = lane >> 4;
+  f64x4 acc[2][4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.0;
+    for (int j = 0; j < 4; ++j) acc[i][j] = f64x4{0.0, 0.0, 0.0, 0.0};
 
-  // Chunks (g, dc) in order; each thread stages SCORE_PER elements of the Q
-  // rows and of the K rows per chunk.  The next chunk's global loads are
-  // issued into registers before the current chunk's multiply-adds, so
-  // their latency overlaps the arithmetic.
-  constexpr int SCORE_PER = SCORE_TILE * SCORE_DC / 256;
+  // Chunks (g, dc) in order; each thread stages column dd of PER_Q Q rows and
+  // PER_K K rows, 16 apart (rows past the last block repeat it: their scores
+  // are not stored).  The next chunk's global loads are issued into registers
+  // before the current chunk's products, so their latency overlaps the
+  // arithmetic.  A last, partial chunk is filled with zeros: fma(0, 0, s)
+  // leaves s as it is, up to the sign of a zero sum.  Vector instructions do
+  // not overlap the fp64 matrix ones, so the loop keeps its addresses as row
+  // pointers and immediate LDS offsets.
+  constexpr int PER_Q = SCORE_ROWS / 16, PER_K = SCORE_COLS / 16;
   const int n_dc = (d + SCORE_DC - 1) / SCORE_DC;
   const int n_chunk = g_n * n_dc;
-  float pq_r[SCORE_PER], pk_r[SCORE_PER];
-  auto fetch = [&](int ci) __attribute__((always_inline)) {
-    const int g = ci / n_dc, dc = (ci - g * n_dc) * SCORE_DC;
-    const int hh = h * g_n + g;
-    const int dn = d - dc < SCORE_DC ? d - dc : SCORE_DC;
+  const int dd = threadIdx.x % SCORE_DC, rt = threadIdx.x / SCORE_DC;
+  const float *qp[PER_Q], *kp[PER_K];
 #pragma unroll
-    for (int u = 0; u < SCORE_PER; ++u) {
-      const int i = (int)threadIdx.x + 256 * u;
-      const int r = i / SCORE_DC, dd = i % SCORE_DC;
-      const bool in_d = dd < dn;
-      pq_r[u] = (in_d && b0 + r < nb)
-                    ? pq[(b0 + r) * (int64_t)hq * d + (int64_t)hh * d + dc + dd]
-                    : 0.0f;
-      pk_r[u] = (in_d && c0 + r < nb)
-                    ? pk[(c0 + r) * (int64_t)hkv * d + (int64_t)h * d + dc + dd]
-                    : 0.0f;
+  for (int u = 0; u < PER_Q; ++u) {
+    const int64_t b = b0 + rt + 16 * u < nb ? b0 + rt + 16 * u : nb - 1;
+    qp[u] = pq + (b * hq + (int64_t)h * g_n) * d + dd;
+  }
+#pragma unroll
+  for (int u = 0; u < PER_K; ++u) {
+    const int64_t c = c0 + rt + 16 * u < nb ? c0 + rt + 16 * u : nb - 1;
+    kp[u] = pk + (c * hkv + h) * (int64_t)d + dd;
+  }
+  float pq_r[PER_Q], pk_r[PER_K];
+  auto fetch = [&](int g, int dc) __attribute__((always_inline)) {
+    if (dc + SCORE_DC <= d) {  // workgroup-uniform: a whole chunk
+#pragma unroll
+      for (int u = 0; u < PER_Q; ++u) pq_r[u] = qp[u][g * d + dc];
+#pragma unroll
+      for (int u = 0; u < PER_K; ++u) pk_r[u] = kp[u][dc];
+    } else {
+      const bool in_d = dc + dd < d;
+#pragma unroll
+      for (int u = 0; u < PER_Q; ++u) pq_r[u] = in_d ? qp[u][g * d + dc] : 0.0f;
+#pragma unroll
+      for (int u = 0; u < PER_K; ++u) pk_r[u] = in_d ? kp[u][dc] : 0.0f;
     }
   };
-  fetch(0);
+  double* wq = &sq[dd][rt ^ (((dd >> 1) & 3) << 2)];
+  double* wk = &sk[dd][rt ^ (((dd >> 1) & 3) << 2)];
+  // columns s * 4 + l4 of step s: the shift of steps 0, 2 and of steps 1, 3
+  const double *aq[2], *ak[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int row = l16 ^ (((2 * x + (l4 >> 1)) & 3) << 2);
+    aq[x] = &sq[l4][r0 + row];
+    ak[x] = &sk[l4][row];
+  }
+  int g = 0, dc = 0;
+  fetch(0, 0);
   for (int ci = 0; ci < n_chunk; ++ci) {
-    const int dc = (ci % n_dc) * SCORE_DC;
-    const int dn = d - dc < SCORE_DC ? d - dc : SCORE_DC;
 #pragma unroll
-    for (int u = 0; u < SCORE_PER; ++u) {
-      const int i = (int)threadIdx.x + 256 * u;
-      const int r = i / SCORE_DC, dd = i % SCORE_DC;
-      sq[dd][r] = (double)pq_r[u];
-      sk[dd][r] = (double)pk_r[u];
-    }
+    for (int u = 0; u < PER_Q; ++u) wq[16 * u] = (double)pq_r[u];
+#pragma unroll
+    for (int u = 0; u < PER_K; ++u) wk[16 * u] = (double)pk_r[u];
     __syncthreads();
-    if (ci + 1 < n_chunk) fetch(ci + 1);
-    for (int dd = 0; dd < dn; ++dd) {
-      double a[8], bv[8];
+    dc += SCORE_DC;
+    if (dc >= d) {
+      dc = 0;
+      ++g;
+    }
+    if (ci + 1 < n_chunk) fetch(g, dc);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) a[i] = sq[dd][ty + 16 * i];
+    for (int s = 0; s < SCORE_DC / 4; ++s) {
+      double a[2], bv[4];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) bv[j] = sk[dd][tx + 16 * j];
+      for (int i = 0; i < 2; ++i) a[i] = aq[s & 1][s * 4 * (SCORE_ROWS + 16) + 16 * i];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int j = 0; j < 4; ++j) bv[j] = ak[s & 1][s * 4 * (SCORE_COLS + 16) + 16 * j];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = __builtin_fma(a[i], bv[j], acc[i][j]);
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], bv[j], acc[i][j], 0, 0, 0);
     }
     __syncthreads();
   }
+  // acc[i][j][v]: row r0 + 16 i + 4 v + l4, column 16 j + l16
+  const int64_t bl = b0 + r0 + l4;
+  double* orow = scores + ((int64_t)h * nb + bl) * nb + c0 + l16;
+  uint32_t* krow =
+      keys ? keys + (((int64_t)h * nb + bl) * gridDim.x + blockIdx.x) * SCORE_CLASSES + l16
+           : nullptr;
+  bool in_c[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int64_t b = b0 + ty + 16 * i;
-    if (b >= nb) continue;
-    double* out = scores + ((int64_t)h * nb + b) * nb;
+  for (int j = 0; j < 4; ++j) in_c[j] = c0 + 16 * j + l16 < nb;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int64_t c = c0 + tx + 16 * j;
-      if (c < nb) out[c] = acc[i][j];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = 16 * i + 4 * v;
+      if (bl + row < nb) {
+        // (fmax leaves a NaN out; NaN only if every column is)
+        double best = __builtin_nan("");
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (in_c[j]) {
+            orow[16 * j] = acc[i][j][v];
+            best = __builtin_fmax(best, acc[i][j][v]);
+          }
+        if (krow) *krow = best == best ? f32_key(f32_below(best)) : 0u;
+      }
+      orow += 4 * nb;
+      if (krow) krow += (int64_t)4 * gridDim.x * SCORE_CLASSES;
     }
-    if (keys) {
-      // (fmax leaves a NaN out; NaN only if every column is)
-      double best = __builtin_nan("");
-#pragma unroll
-      for (int j = 0; j < 8; ++j)
-        if (c0 + tx + 16 * j < nb) best = __builtin_fmax(best, acc[i][j]);
-      keys[(((int64_t)h * nb + b) * gridDim.x + blockIdx.x) * SCORE_CLASSES + tx] =
-          best == best ? f32_key(f32_below(best)) : 0u;
-    }
-  }
 }
 
 // dst[t * topk + j] = ord[j] for the `total` / topk token rows at dst, the
@@ -490,11 +534,11 @@ __global__ __launch_bounds__(256) void topk_wave_kernel(
   fill_token_rows(dst, total, ord, topk, lane, 64);
 }
 
-// One wave per (query block, kv head) row of up to 64 * NM / 16 score tiles:
+// One wave per (query block, kv head) row of up to 64 * NM / 16 column tiles:
 // the row's classes (score_kernel's keys; those of tiles inside the row's batch
 // element) give a lower bound of its topk-th best score -- the largest value
 // that at least topk class maxima reach, and these are distinct columns -- and
-// only the columns that reach it are listed (about topk of them, at most eight
+// only the columns that reach it are listed (about topk of them, at most four
 // per class that reaches the bound) and ranked by wave_best_r.  The forced
 // blocks are taken first and count among the topk.  More than BOUND_CAP such
 // columns (ties in great number) take one scan of the row per pick.
@@ -531,8 +575,8 @@ __global__ __launch_bounds__(64) void topk_bound_kernel(
 #pragma unroll
   for (int m = 0; m < NM; ++m) {
     const int ci = lane + 64 * m, tile = ci / SCORE_CLASSES;
-    const int64_t c0 = (int64_t)tile * SCORE_TILE;
-    const int64_t c1 = c0 + SCORE_TILE < nb ? c0 + SCORE_TILE : nb;
+    const int64_t c0 = (int64_t)tile * SCORE_COLS;
+    const int64_t c1 = c0 + SCORE_COLS < nb ? c0 + SCORE_COLS : nb;
     key[m] = tile < ntile && c0 >= cs && c1 <= cs + nbb ? krow[ci] : 0u;
   }
   // Forced blocks in order, distinct, valid, at most kmax.
@@ -699,7 +743,7 @@ void carve_select(Carver& ws, int64_t n, int64_t nb, int64_t hq, int64_t hkv,
   s.first = ws.take<int32_t>((size_t)pool_first_count(n));
   s.scores = ws.take<double>((size_t)(hkv * nbc * nbc));
   s.keys = bounded_rows(nb) ? ws.take<uint32_t>((size_t)(hkv * nbc * SCORE_CLASSES *
-                                                         ceil_div(nbc, SCORE_TILE)))
+                                                         ceil_div(nbc, SCORE_COLS)))
                             : nullptr;
 }
 
@@ -768,9 +812,10 @@ static int select_blocks_impl(const void* q, const void* k, const float* pooled_
     if (rc) return rc;
     pk = s.pk;
   }
-  const unsigned nt = (unsigned)ceil_div(n_blocks, SCORE_TILE);
-  hipLaunchKernelGGL(score_kernel, dim3(nt, nt, (unsigned)hkv), dim3(256), 0,
-                     st, s.pq, pk, n_blocks, (int)hq, (int)hkv,
+  const unsigned nt = (unsigned)ceil_div(n_blocks, SCORE_COLS);
+  hipLaunchKernelGGL(score_kernel,
+                     dim3(nt, (unsigned)ceil_div(n_blocks, SCORE_ROWS), (unsigned)hkv),
+                     dim3(256), 0, st, s.pq, pk, n_blocks, (int)hq, (int)hkv,
                      (int)head_dim, s.scores, topk <= 64 ? s.keys : nullptr);
   LSRM_CHECK_LAUNCH();
   const unsigned rows4 = (unsigned)ceil_div(n_blocks * hkv, 4);
@@ -793,12 +838,12 @@ static int select_blocks_impl(const void* q, const void* k, const float* pooled_
                      dim3(64), 0, st, s.scores, s.keys, (int)nt, n_blocks, cu_seqblocks,   \
                      batch, cu_block_tokens, n_tokens, (int)topk, forced_blocks,           \
                      (int)n_forced, force_self, topk_idx, topk_compact)
-    if (nt * SCORE_CLASSES <= 64 * 8)
-      LSRM_TOPK_BOUND(8);
-    else if (nt * SCORE_CLASSES <= 64 * 12)
+    if (nt * SCORE_CLASSES <= 64 * 12)
       LSRM_TOPK_BOUND(12);
+    else if (nt * SCORE_CLASSES <= 64 * 20)
+      LSRM_TOPK_BOUND(20);
     else
-      LSRM_TOPK_BOUND(16);
+      LSRM_TOPK_BOUND(32);
 #undef LSRM_TOPK_BOUND
   } else
     hipLaunchKernelGGL(topk_kernel, dim3((unsigned)n_blocks, (unsigned)hkv),
