@@ -670,6 +670,129 @@ bool launch_half_chunks(const void* x, int64_t n, int64_t ch, const int32_t* cu,
   }
 }
 
+// Launches of few waves: their time is the chain of row loads of one wave, not
+// the bytes.  A wave takes 256 bytes of a chunk's rows -- one 4-byte word (E
+// channels) per lane and row -- so that all 64 rows of the chunk and the block
+// lookup are in flight at once, and the ends of the next 64 blocks with it.
+// Same pieces and sequential fp32 sums as the other kernels (bit-identical
+// partials).  4099 x 256 bf16 rows: 16.1 -> 9.6 us (two chunks per wave, 16
+// rounds of four rows, in the 256-channel kernel).  NT = 2 takes a second
+// tensor's waves after the first's.
+constexpr int64_t POOL_SMALL_WAVES = 2048;  // two per SIMD: one round of waves
+
+template <int DT, int NT>
+__global__ __launch_bounds__(256) void pool_pieces_small(
+    const void* __restrict__ xa, int64_t n, int64_t ch, const int32_t* __restrict__ cu,
+    int64_t nb, float* __restrict__ partial_a, const void* __restrict__ xb,
+    float* __restrict__ partial_b) {
+  constexpr int E = DT == LSRM_F32 ? 1 : 2;  // channels per word
+  const int lane = threadIdx.x & 63;
+  const uint32_t wpc = (uint32_t)(ch / (64 * E));  // waves per chunk
+  const uint32_t n_waves = (uint32_t)((n + POOL_CHUNK - 1) / POOL_CHUNK) * wpc;
+  uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (wave >= NT * n_waves) return;
+  const bool second = NT == 2 && wave >= n_waves;
+  if (second) wave -= n_waves;
+  const int64_t j = wave / wpc;
+  const int64_t c0 = (int64_t)((wave - (uint32_t)j * wpc) * 64 + lane) * E;
+  const int64_t r0 = j * POOL_CHUNK;
+  const int64_t r1 = r0 + POOL_CHUNK < n ? r0 + POOL_CHUNK : n;
+  const uint32_t* xp = reinterpret_cast<const uint32_t*>(second ? xb : xa) + (r0 * ch + c0) / E;
+  float* partial = second ? partial_b : partial_a;
+  uint32_t w[POOL_CHUNK];
+#pragma unroll
+  for (int u = 0; u < POOL_CHUNK; ++u)
+    w[u] = __builtin_nontemporal_load(xp + (r0 + u < r1 ? u : r1 - 1 - r0) * (ch / E));
+  // b = last block whose start is <= r0 (-1: before the first block, nb: past
+  // the last): a two-level count of the nondecreasing offsets.
+  const int64_t S = (nb + 64) / 64;
+  const int64_t i1 = lane * S;
+  const int c1 = __popcll(__ballot(i1 <= nb && (int64_t)cu[i1 <= nb ? i1 : nb] <= r0));
+  int64_t b = -1;
+  if (c1 > 0) {
+    const int64_t base = (int64_t)(c1 - 1) * S;
+    int cnt = 0;
+    for (int64_t m = 0; m < S; m += 64) {
+      const int64_t i2 = base + m + lane;
+      const bool in = m + lane < S && i2 <= nb;
+      cnt += __popcll(__ballot(in && (int64_t)cu[in ? i2 : 0] <= r0));
+    }
+    b = base + cnt - 1;
+  }
+  // Lane l holds the end of block wb + l (the start of the next one).
+  int64_t wb = b;
+  int32_t ends = cu[b + 1 + lane < nb ? b + 1 + lane : nb];
+  auto end_of = [&](int64_t blk) __attribute__((always_inline)) -> int64_t {
+    if (blk >= nb) return INT64_MAX;
+    if (blk - wb >= 64) {
+      wb = blk;
+      ends = cu[blk + 1 + lane < nb ? blk + 1 + lane : nb];
+    }
+    return __builtin_amdgcn_readlane(ends, (int)(blk - wb));
+  };
+  // Block by block: the rows [lo, hi) of the chunk that block b owns, added in
+  // order (the row tests are scalar; one copy of the adds keeps the kernel
+  // small, since its instructions are fetched anew by every launch).
+  int64_t lo = 0;
+  for (;; ++b) {
+    const int64_t be = end_of(b);
+    const int64_t hi = (be < r1 ? be : r1) - r0;
+    if (b >= nb) break;
+    if (hi > lo) {
+      if (b >= 0) {
+        const int l = (int)lo, e = (int)hi;
+        float acc[E];
+#pragma unroll
+        for (int i = 0; i < E; ++i) acc[i] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < POOL_CHUNK; ++u) {
+          if (u < l || u >= e) continue;
+          if constexpr (E == 1) {
+            acc[0] = acc[0] + __uint_as_float(w[u]);
+          } else {
+            acc[0] = acc[0] + to_f32<DT>((uint16_t)(w[u] & 0xffffu));
+            acc[E - 1] = acc[E - 1] + to_f32<DT>((uint16_t)(w[u] >> 16));
+          }
+        }
+        float* dst = partial + (b + j) * ch + c0;
+#pragma unroll
+        for (int i = 0; i < E; ++i) dst[i] = acc[i];
+      }
+      lo = hi;
+    }
+    if (be >= r1) break;
+  }
+}
+
+// Whether pool_pieces_small takes NT tensors of these rows: whole 256-byte
+// pieces and at most POOL_SMALL_WAVES waves.  Beyond that the byte rate decides
+// and the wider kernels are faster (8 bytes in flight per lane and byte read).
+bool small_pool(const void* x, int x_dtype, int64_t n, int64_t ch, int nt) {
+  const int64_t row_bytes = ch * (x_dtype == LSRM_F32 ? 4 : 2);
+  return n > 0 && row_bytes % 256 == 0 && ((uintptr_t)x % 4) == 0 &&
+         nt * ((n + POOL_CHUNK - 1) / POOL_CHUNK) * (row_bytes / 256) <= POOL_SMALL_WAVES;
+}
+
+template <int NT>
+int launch_pieces_small(const void* xa, const void* xb, int x_dtype, int64_t n, int64_t ch,
+                        const int32_t* cu, int64_t nb, float* pa, float* pb, hipStream_t st) {
+  const int64_t waves = NT * ((n + POOL_CHUNK - 1) / POOL_CHUNK) *
+                        (ch * (x_dtype == LSRM_F32 ? 4 : 2) / 256);
+  const dim3 grid((unsigned)((waves + 3) / 4));
+#define LSRM_POOL_S(DT)                                                                        \
+  hipLaunchKernelGGL((pool_pieces_small<DT, NT>), grid, dim3(256), 0, st, xa, n, ch, cu, nb, pa, \
+                     xb, pb)
+  switch (x_dtype) {
+    case LSRM_F32: LSRM_POOL_S(LSRM_F32); break;
+    case LSRM_F16: LSRM_POOL_S(LSRM_F16); break;
+    case LSRM_BF16: LSRM_POOL_S(LSRM_BF16); break;
+    default: return LSRM_ERR_UNSUPPORTED;
+  }
+#undef LSRM_POOL_S
+  LSRM_CHECK_LAUNCH();
+  return LSRM_OK;
+}
+
 int64_t pool_partial_rows(int64_t n, int64_t nb) {
   return nb + (n + POOL_CHUNK - 1) / POOL_CHUNK;
 }
@@ -691,7 +814,11 @@ int launch_block_mean_pool(const void* x, int x_dtype, int64_t n, int64_t ch,
   const bool slab = vec && x_dtype != LSRM_F32 && n_vec % 64 == 0 &&
                    n_chunks * n_vec < (int64_t{1} << 31);
   const bool inline_first = slab && nb + 1 <= 512;
-  if (n > 0 && slab) {
+  if (small_pool(x, x_dtype, n, ch, 1)) {
+    const int rc = launch_pieces_small<1>(x, nullptr, x_dtype, n, ch, cu, nb, partial, nullptr,
+                                          st);
+    if (rc) return rc;
+  } else if (n > 0 && slab) {
     if (!inline_first)
       hipLaunchKernelGGL(pool_chunk_first, dim3((unsigned)((n_chunks + 255) / 256)),
                          dim3(256), 0, st, cu, nb, n_chunks, first);
@@ -763,7 +890,7 @@ int launch_block_mean_pool(const void* x, int x_dtype, int64_t n, int64_t ch,
 }
 
 // Two tensors of one shape and block partition: one piece launch and one
-// combine launch for both when the slab path applies, otherwise the
+// combine launch for both when the slab path or the one for few waves applies, otherwise the
 // single-tensor launches one after the other (identical results).
 int launch_block_mean_pool2(const void* xa, const void* xb, int x_dtype, int64_t n, int64_t ch,
                             const int32_t* cu, int64_t nb, void* out_a, int out_a_dtype,
@@ -774,7 +901,9 @@ int launch_block_mean_pool2(const void* xa, const void* xb, int x_dtype, int64_t
                     ((uintptr_t)xa % 16) == 0 && ((uintptr_t)xb % 16) == 0 &&
                     ((uintptr_t)partial_a % 16) == 0 && ((uintptr_t)partial_b % 16) == 0 &&
                     2 * ((n + POOL_CHUNK - 1) / POOL_CHUNK) * (ch / POOL_VEC) < (int64_t{1} << 31);
-  if (!slab || n == 0) {
+  const bool small = small_pool(xa, x_dtype, n, ch, 2) && ((uintptr_t)xb % 4) == 0 &&
+                     ((uintptr_t)partial_a % 16) == 0 && ((uintptr_t)partial_b % 16) == 0;
+  if (!small && (!slab || n == 0)) {
     int rc = launch_block_mean_pool(xa, x_dtype, n, ch, cu, nb, out_a, out_a_dtype, partial_a,
                                     first, st);
     if (rc) return rc;
@@ -784,10 +913,13 @@ int launch_block_mean_pool2(const void* xa, const void* xb, int x_dtype, int64_t
   const int64_t n_vec = ch / POOL_VEC;
   const int64_t n_chunks = (n + POOL_CHUNK - 1) / POOL_CHUNK;
   const bool inline_first = nb + 1 <= 512;
-  if (!inline_first)
-    hipLaunchKernelGGL(pool_chunk_first, dim3((unsigned)((n_chunks + 255) / 256)), dim3(256), 0,
-                       st, cu, nb, n_chunks, first);
-  {
+  if (small) {
+    const int rc = launch_pieces_small<2>(xa, xb, x_dtype, n, ch, cu, nb, partial_a, partial_b, st);
+    if (rc) return rc;
+  } else {
+    if (!inline_first)
+      hipLaunchKernelGGL(pool_chunk_first, dim3((unsigned)((n_chunks + 255) / 256)), dim3(256), 0,
+                         st, cu, nb, n_chunks, first);
     const uint16_t* a = reinterpret_cast<const uint16_t*>(xa);
     const uint16_t* b = reinterpret_cast<const uint16_t*>(xb);
     if (x_dtype == LSRM_F16)
