@@ -146,7 +146,7 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
     rc = build_key_items(cu_blk, nb, nk, ws, w.items, st);
     if (rc) return rc;
     if (ws.base && !ws.dry) {
-      rc = mark_backward_plan(w.plan.counter, st);
+      rc = mark_backward_plan(w.plan, hkv, packed_q > 0, st);
       if (rc) return rc;
     }
   }
@@ -313,9 +313,7 @@ int attn_setup(const void* q, const void* k, const void* v, int dtype,
   a.plan = w.plan;
   a.rev = w.rev;
   a.qrev = w.qrev;
-  a.qmap_n = dkdv_packed_q((flags & LSRM_PLAN_KEY_CENTRIC) != 0, ROWS / g) > 0
-                 ? cu_seqlens_q + batch
-                 : w.plan.ghead_off + hkv;
+  a.qmap_n = w.plan.counter + PLAN_QMAP_SLOT;
   a.items = w.items;
   a.kc = w.kc;
   a.kc_marker = kc_plan_marker(flags, (int)head_dim);

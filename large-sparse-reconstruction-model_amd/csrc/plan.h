@@ -42,7 +42,11 @@ constexpr int NARROW_QUEUE_SLOT = 28, NARROW_EXIT_SLOT = 30;
 // forward-only plan in a workspace large enough for the backward).
 constexpr int PLAN_BWD_SLOT = 32;
 constexpr int32_t PLAN_BWD_MAGIC = 0x4c42574b;
-int mark_backward_plan(int32_t* counter, hipStream_t st);
+// [PLAN_QMAP_SLOT] > 0: the plan's query map may list queries (it has grouped
+// tiles, or `packed`: queries of run tiles are listed too), whatever flags a
+// later run is given.
+constexpr int PLAN_QMAP_SLOT = 34;
+int mark_backward_plan(const TilePlan& plan, int64_t hkv, bool packed, hipStream_t st);
 
 // CSR map block -> rows (tiles or queries) that selected it, per kv head.
 struct RevMap {

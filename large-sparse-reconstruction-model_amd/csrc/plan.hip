@@ -495,12 +495,16 @@ __global__ void plan_offsets_kernel(const int32_t* n_groups, const int64_t* spli
   }
 }
 
-__global__ void mark_backward_plan_kernel(int32_t* counter) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) counter[PLAN_BWD_SLOT] = PLAN_BWD_MAGIC;
+__global__ void mark_backward_plan_kernel(TilePlan plan, int hkv, int packed) {
+  if (threadIdx.x == 0 && blockIdx.x == 0) {
+    plan.counter[PLAN_QMAP_SLOT] = packed ? 1 : plan.ghead_off[hkv];
+    plan.counter[PLAN_BWD_SLOT] = PLAN_BWD_MAGIC;
+  }
 }
 
-int mark_backward_plan(int32_t* counter, hipStream_t st) {
-  hipLaunchKernelGGL(mark_backward_plan_kernel, dim3(1), dim3(64), 0, st, counter);
+int mark_backward_plan(const TilePlan& plan, int64_t hkv, bool packed, hipStream_t st) {
+  hipLaunchKernelGGL(mark_backward_plan_kernel, dim3(1), dim3(64), 0, st, plan, (int)hkv,
+                     packed ? 1 : 0);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }

@@ -52,3 +52,32 @@ def test_backward_mixed_runs(g, d, batch):
     for name, a, b in (("out", o, ref), ("dq", dq, qf.grad), ("dk", dk, kf.grad),
                        ("dv", dv, vf.grad)):
         assert_attn_close(a, b.detach(), name)
+
+
+def test_packed_plan_run_without_flags():
+    # A key-centric backward plan also serves the entry point without plan
+    # flags: with runs of three equal rows only (no grouped tile), every query
+    # is in the packed map and must still be found there.
+    gen = torch.Generator().manual_seed(3)
+    n, hkv, g, d, nb, topk = 384, 2, 16, 32, 8, 3
+    rows = torch.stack([torch.randperm(nb, generator=gen)[:topk] for _ in range(hkv * n // 3)])
+    rows = rows.view(hkv, n // 3, topk).repeat_interleave(3, dim=1).to(torch.int32).contiguous()
+    cu = torch.arange(nb + 1, dtype=torch.int32) * (n // nb)
+    cu_sb, cu_q = (torch.tensor([0, x], dtype=torch.int32) for x in (nb, n))
+    q, do = (torch.randn(n, hkv * g, d, generator=gen).to(torch.bfloat16) * 0.5
+             for _ in range(2))
+    k, v = (torch.randn(n, hkv, d, generator=gen).to(torch.bfloat16) * 0.5 for _ in range(2))
+    q, k, v, do, rows, cu_sb, cu, cu_q = (t.to(DEV) for t in (q, k, v, do, rows, cu_sb, cu, cu_q))
+    plan = H.SelAttnPlan(q.shape, k.shape, rows, cu_sb, cu, cu_q, backward=True, key_centric=True)
+    o, lse = plan.fwd(q, k, v, d ** -0.5)
+    want = plan.bwd(do, q, k, v, o, lse, d ** -0.5)
+    dq, dk, dv = torch.empty_like(q), torch.zeros_like(k), torch.zeros_like(v)
+    delta = torch.empty(hkv * g, n, dtype=torch.float32, device=DEV)
+    p = H._ptr
+    assert H.lib().lsrm_sel_attn_bwd_run(
+        p(do), p(q), p(k), p(v), p(o), p(lse), H.BF16, n, n, hkv * g, hkv, d, p(rows), topk,
+        p(cu_sb), p(cu), nb, p(cu_q), 1, d ** -0.5, p(dq), p(dk), p(dv), p(delta), p(plan.ws),
+        plan.ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+    assert float(dk.float().abs().max()) > 0
+    for a, b in zip((dq, dk, dv, delta), want):
+        assert torch.equal(a, b)
