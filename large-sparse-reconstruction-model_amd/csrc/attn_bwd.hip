@@ -212,17 +212,16 @@ narrow_dq_kernel(AttnArgs a) {
   leave_queue(queue, queue + NARROW_EXIT_SLOT - NARROW_QUEUE_SLOT);
 }
 
-// MODE 0 (DQ_RUN): the run tiles of the plan (head dims up to 64: the wide ones).  MODE 1 (DQ_UNION): the
-// grouped tiles, run once over the union of their rows' blocks with per-row
-// key masks, or once per run of identical rows with the other rows' P forced
-// to zero (the passes of the forward's grouped tiles; no softmax state is
-// carried, so either way each row's dQ is a plain sum over the keys it
-// attends); a key-centric plan does not launch it (its grouped tiles' rows
-// run as gathered tiles).
-// MODE 2 (DQ_GATHER): the gathered tiles of a key-centric plan over blocks
-// the resident kernels do not take (no keys, or more than kc_res_max), each
-// row writing the block's share of its dQ (one slot of its row, in the
-// input type) for kc_dq_merge_kernel.
+// MODE 0 (DQ_RUN): the run tiles of the plan (head dim 32: the wide ones).
+// MODE 1 (DQ_UNION): the grouped tiles, run once over the union of their rows'
+// blocks with per-row key masks, or once per run of identical rows with the
+// other rows' P forced to zero (the passes of the forward's grouped tiles; no
+// softmax state is carried, so either way each row's dQ is a plain sum over
+// the keys it attends); a key-centric plan does not launch it (its grouped
+// tiles' rows run as gathered tiles). MODE 2 (DQ_GATHER): the gathered tiles
+// of a key-centric plan over blocks the resident kernels do not take (no keys,
+// or more than kc_res_max), each row writing the block's share of its dQ (one
+// slot of its row, in the input type) for kc_dq_merge_kernel.
 constexpr int DQ_RUN = 0, DQ_UNION = 1, DQ_GATHER = 2;
 
 template <int DT, int D, int MODE>

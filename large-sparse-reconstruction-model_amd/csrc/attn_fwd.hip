@@ -268,16 +268,15 @@ narrow_fwd_kernel(AttnArgs a) {
   leave_queue(queue, queue + NARROW_EXIT_SLOT - NARROW_QUEUE_SLOT);
 }
 
-// MODE 0 (FWD_RUN): the run tiles of the plan (every row of a tile shares
-// one key stream; head dims up to 64: the wide ones).  MODE 1 (FWD_UNION): the grouped tiles (see build_union),
-// run with per-row key masks; a key-centric plan does not launch it (its
-// grouped tiles' rows run as gathered tiles).  MODE 2 (FWD_GATHER): gathered
-// tiles of a key-centric plan
-// -- the queries that listed one block, attending that block alone, each row
-// written as a partial result (O over the block normalised by its own sum,
-// in the input type, and its log2 LSE) for kc_merge_kernel.  Separate
-// instantiations, so the run-tile kernel carries none of the other modes'
-// code or state.
+// MODE 0 (FWD_RUN): the run tiles of the plan (every row of a tile shares one
+// key stream; head dim 32: the wide ones).  MODE 1 (FWD_UNION): the grouped
+// tiles (see build_union), run with per-row key masks; a key-centric plan does
+// not launch it (its grouped tiles' rows run as gathered tiles). MODE 2
+// (FWD_GATHER): gathered tiles of a key-centric plan -- the queries that
+// listed one block, attending that block alone, each row written as a partial
+// result (O over the block normalised by its own sum, in the input type, and
+// its log2 LSE) for kc_merge_kernel.  Separate instantiations, so the run-tile
+// kernel carries none of the other modes' code or state.
 constexpr int FWD_RUN = 0, FWD_UNION = 1, FWD_GATHER = 2;
 
 template <int DT, int D, int MODE>

@@ -33,19 +33,19 @@ constexpr int SEL_MAXK = 256;
 // 32x64 per wave as 2x4 blocks of v_mfma_f64_16x16x4 (bound by that
 // instruction's rate, the fp64 rate of the chip; a wave's 64 accumulator
 // registers leave room for four waves per SIMD, which hide the short loop's
-// loads -- with 64x64 per wave and two waves it was busy 47% of the time; the vector form with 8x8 scores per thread needed
-// 16 LDS reads per 64 fused multiply-adds and reached a third of it: 423 ->
-// 337 us for 4 heads x 4881 x 4881 x 64).  The instruction adds its four
+// loads -- with 64x64 per wave and two waves it was busy 47% of the time).
+// The vector form with 8x8 scores per thread needed 16 LDS reads per 64 fused
+// multiply-adds and reached less: 423 -> 337 us for 4 heads x 4881 x 4881
+// x 64, of which 175 us at the fp64 rate.  The instruction adds its four
 // products one by one in ascending order, each a fused multiply-add (checked
 // bit for bit against that chain), so a score is the same fixed function of
 // the pooled means: fp64 accumulation over (g, d) in order.  The pooled rows
 // are staged in LDS as doubles, SCORE_DC head-dim columns at a time.
 //
 // With `keys`, the kernel also writes for every row and class of four columns
-// (16 apart in a tile) the largest score, rounded
-// down to fp32, as an order-preserving key (NaN scores left out; 0 for a class
-// without a score): [hkv, nb, column tiles, 16],
-// read by topk_bound_kernel.
+// (16 apart in a tile) the largest score, rounded down to fp32, as an
+// order-preserving key (NaN scores left out; 0 for a class without a score):
+// [hkv, nb, column tiles, 16], read by topk_bound_kernel.
 constexpr int SCORE_ROWS = 128, SCORE_COLS = 64;
 constexpr int SCORE_DC = 16;
 constexpr int SCORE_CLASSES = 16;  // per column tile and row
