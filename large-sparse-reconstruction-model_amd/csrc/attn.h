@@ -680,23 +680,26 @@ __device__ inline uint32_t group_offset(const SelLds& s, GroupCursor& c, int P,
 
 // ------------------------------------------------------- narrow run tiles --
 // Run tiles of at most NARROW_ROWS rows (short runs of per-token rows at many
-// query heads per kv head) would leave two or three of a workgroup's four
-// waves idle for the tile's whole key stream.  They are split over the keys
-// instead: the waves of one 32-row block (four for up to 32 rows, two for up
-// to 64) take the stream's 32-key blocks in turn, each at its own pace.  A
+// query heads per kv head) would leave three of a workgroup's four waves idle
+// for the tile's whole key stream.  They are split over the keys instead: the
+// waves take the stream's 32-key blocks in turn, each at its own pace.  A
 // block's K and V rows belong to one wave, so they go straight into its
 // registers (two blocks ahead, no barrier); only the operand that is needed
 // transposed passes through a wave's own piece of LDS.  The waves' fp32 sums
 // are added in LDS in a fixed order at the end.
 //
 // Bound by L2 requests for the gathered rows (3D-aware rows of 122880 tokens
-// at 32 / 2 heads of 32: 26600 tiles per kv head, 480 M requests of 64 bytes,
-// 8.7 of 16 per clock and XCD): forward 3.69 -> 3.28 ms, dQ 5.11 -> 3.34 ms;
-// with the stream staged in LDS for all four waves, one barrier per 128 keys
-// and three steps in flight, 3.62 and 3.50 ms.  At head dim 64 a run tile's K
-// and V traffic sets its time whatever its rows, and the run-tile kernels move
-// it with wider requests: 454 blocks of 32..512 queries at 24 heads took 9.1 ms
-// as run tiles, 10.3 ms split by width (9.2 with the stream in LDS).
+// at 32 / 2 heads of 32, 26600 run tiles per kv head).  Whole forward passes
+// over 98304 queries at 32 / 2 heads, runs of equal top-16 rows, as run tiles
+// and with their narrow tiles split: tiles of 32 rows 1.71 -> 1.46 ms over
+// blocks of 24 keys and 10.4 -> 10.7 over blocks of 246 (equal within the
+// runs' spread); tiles of 48 rows, two waves per row block, 1.20 -> 1.06 and
+// 7.0 -> 9.1; of 64 rows 0.92 -> 0.83 and 5.3 -> 6.9.  So the line lies at one
+// row block (NARROW_ROWS); wider tiles run as run tiles.  At head dim 64 a run
+// tile's K and V traffic sets its time whatever its rows, and the run-tile
+// kernels move it with wider requests: 454 blocks of 32..512 queries at 24
+// heads took 9.1 ms as run tiles, 10.3 ms split by width (9.2 with the stream
+// in LDS).
 constexpr bool narrow_split(int d) { return d <= 32; }
 
 // One wave's walk over its 32-key blocks of a narrow tile's stream.

@@ -34,7 +34,7 @@ namespace lsrm {
 // ------------------------------------------------------------------- dQ --
 
 // dQ of a narrow run tile (see attn.h): every wave sums dS K over its own keys,
-// and the waves of one row block are added in LDS.
+// and the waves' sums are added in LDS.
 template <int DT, int D>
 __device__ inline __attribute__((always_inline)) void narrow_dq(
     const AttnArgs& a, int h, int q0, int rows, const SelLds& sel, const int* map, int nkeys,
@@ -42,19 +42,16 @@ __device__ inline __attribute__((always_inline)) void narrow_dq(
   using G = KvTile<D>;
   constexpr int NS = D / 16, ND = D / 32;
   const int hb = lane >> 5, l32 = lane & 31;
-  // waves over the keys of one row block, this wave's row block and turn
-  const int nkw = rows <= 32 ? 4 : 2;
-  const int rb = rows <= 32 ? 0 : (wv & 1), kq = rows <= 32 ? wv : (wv >> 1);
-  const int r = rb * 32 + l32;
-  const bool row_ok = r < rows;
-  const int64_t qi = q0 + (row_ok ? r / a.g : 0);
-  const int hh = h * a.g + (row_ok ? r % a.g : 0);
+  constexpr int NKW = 4;  // waves over the keys; wave wv takes blocks wv, wv + 4, ..
+  const bool row_ok = l32 < rows;
+  const int64_t qi = q0 + (row_ok ? l32 / a.g : 0);
+  const int hh = h * a.g + (row_ok ? l32 % a.g : 0);
   NarrowBlocks<D> blocks;
   blocks.init(a, h, sel, map, nkeys, lane);
   const int nblk = (nkeys + 31) / 32;
   u32x4 kb[2][NS], vb[2][NS];
-  if (kq < nblk) blocks.load(kq, kb[0], vb[0]);
-  if (kq + nkw < nblk) blocks.load(kq + nkw, kb[1], vb[1]);
+  if (wv < nblk) blocks.load(wv, kb[0], vb[0]);
+  if (wv + NKW < nblk) blocks.load(wv + NKW, kb[1], vb[1]);
   u32x4 qb[NS], dob[NS];
   float dpart = 0.0f;
 #pragma unroll
@@ -81,7 +78,7 @@ __device__ inline __attribute__((always_inline)) void narrow_dq(
   if (row_ok) {
     const float l = a.lse_in[(int64_t)hh * a.nq + qi];
     if (l > -__builtin_inf()) bias = -l;
-    if (hb == 0 && kq == 0) a.lse[(int64_t)hh * a.nq + qi] = delta;
+    if (hb == 0 && wv == 0) a.lse[(int64_t)hh * a.nq + qi] = delta;
   }
   char* sk = lds + wv * (32 * D * 2);
   uint32_t vl_off[ND][2];
@@ -115,7 +112,7 @@ __device__ inline __attribute__((always_inline)) void narrow_dq(
     for (int s = 0; s < NS; ++s)
       *reinterpret_cast<u32x4*>(sk + G::off(l32, 2 * s + hb)) = kr[s];
     wave_lds_order();
-    if (b + 2 * nkw < nblk) blocks.load(b + 2 * nkw, kr, vr);
+    if (b + 2 * NKW < nblk) blocks.load(b + 2 * NKW, kr, vr);
     if (b * 32 + 32 > nkeys) {
 #pragma unroll
       for (int v = 0; v < 16; ++v)
@@ -143,30 +140,27 @@ __device__ inline __attribute__((always_inline)) void narrow_dq(
         dqacc[db] = mfma32<DT>(u32x4{lo[0], lo[1], hi[0], hi[1]}, ds[c], dqacc[db]);
       }
   };
-  if (rb * 32 < rows) {  // wave-uniform
-    for (int b = kq; b < nblk; b += 2 * nkw) {
-      block(b, kb[0], vb[0]);
-      if (b + nkw < nblk) block(b + nkw, kb[1], vb[1]);
-    }
+  for (int b = wv; b < nblk; b += 2 * NKW) {
+    block(b, kb[0], vb[0]);
+    if (b + NKW < nblk) block(b + NKW, kb[1], vb[1]);
   }
   __syncthreads();  // every wave has left its blocks
   constexpr int RED = ND * 16;  // words per lane
   float* red = reinterpret_cast<float*>(lds) + lane;
-  if (kq > 0) {
-    float* mine = red + (rb * (nkw - 1) + kq - 1) * RED * 64;
+  if (wv > 0) {
+    float* mine = red + (wv - 1) * RED * 64;
 #pragma unroll
     for (int db = 0; db < ND; ++db)
 #pragma unroll
       for (int v = 0; v < 16; ++v) mine[(db * 16 + v) * 64] = dqacc[db][v];
   }
   __syncthreads();
-  if (kq > 0 || !row_ok) return;
-  const float* others = red + rb * (nkw - 1) * RED * 64;
-  for (int w = 0; w < nkw - 1; ++w)
+  if (wv > 0 || !row_ok) return;
+  for (int w = 0; w < NKW - 1; ++w)
 #pragma unroll
     for (int db = 0; db < ND; ++db)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) dqacc[db][v] += others[(w * RED + db * 16 + v) * 64];
+      for (int v = 0; v < 16; ++v) dqacc[db][v] += red[(w * RED + db * 16 + v) * 64];
   uint16_t* drow = a.out + (qi * a.hq + hh) * D;
 #pragma unroll
   for (int db = 0; db < ND; ++db)

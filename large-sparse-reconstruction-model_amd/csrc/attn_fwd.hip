@@ -69,9 +69,9 @@ __device__ inline float row_max(const f32x16* sc) {
 
 // A narrow run tile (see attn.h): rows of queries q0 .. of kv head h over the
 // stream in `sel`.  The softmax runs online with lazy rescaling (p <= 2^8),
-// each wave over its own keys; at the end the waves of one row block are
-// merged in fp32: M = max m_w, O = sum 2^(m_w - M) O_w, l likewise.
-// `red` (LDS): a wave's V blocks while it runs, then the waves' sums.
+// each wave over its own keys; at the end the waves are merged in fp32:
+// M = max m_w, O = sum 2^(m_w - M) O_w, l likewise.
+// `lds`: the waves' V blocks while they run, then the waves' sums.
 template <int DT, int D>
 __device__ inline __attribute__((always_inline)) void narrow_fwd(
     const AttnArgs& a, int h, int q0, int rows, const SelLds& sel, const int* map, int nkeys,
@@ -79,19 +79,16 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
   using G = KvTile<D>;
   constexpr int NS = D / 16, ND = D / 32;
   const int hb = lane >> 5, l32 = lane & 31;
-  // waves over the keys of one row block, this wave's row block and turn
-  const int nkw = rows <= 32 ? 4 : 2;
-  const int rb = rows <= 32 ? 0 : (wv & 1), kq = rows <= 32 ? wv : (wv >> 1);
-  const int r = rb * 32 + l32;
-  const bool row_ok = r < rows;
-  const int64_t qi = q0 + (row_ok ? r / a.g : 0);
-  const int hh = h * a.g + (row_ok ? r % a.g : 0);
+  constexpr int NKW = 4;  // waves over the keys; wave wv takes blocks wv, wv + 4, ..
+  const bool row_ok = l32 < rows;
+  const int64_t qi = q0 + (row_ok ? l32 / a.g : 0);
+  const int hh = h * a.g + (row_ok ? l32 % a.g : 0);
   NarrowBlocks<D> blocks;
   blocks.init(a, h, sel, map, nkeys, lane);
   const int nblk = (nkeys + 31) / 32;
   u32x4 kb[2][NS], vb[2][NS];
-  if (kq < nblk) blocks.load(kq, kb[0], vb[0]);
-  if (kq + nkw < nblk) blocks.load(kq + nkw, kb[1], vb[1]);
+  if (wv < nblk) blocks.load(wv, kb[0], vb[0]);
+  if (wv + NKW < nblk) blocks.load(wv + NKW, kb[1], vb[1]);
   u32x4 qb[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s)
@@ -127,7 +124,7 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
     for (int s = 0; s < NS; ++s)
       *reinterpret_cast<u32x4*>(sv + G::off(l32, 2 * s + hb)) = vr[s];
     wave_lds_order();
-    if (b + 2 * nkw < nblk) blocks.load(b + 2 * nkw, kr, vr);
+    if (b + 2 * NKW < nblk) blocks.load(b + 2 * NKW, kr, vr);
     if (b * 32 + 32 > nkeys) {
 #pragma unroll
       for (int v = 0; v < 16; ++v)
@@ -178,17 +175,15 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
         oacc[db] = mfma32<DT>(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb[c], oacc[db]);
       }
   };
-  if (rb * 32 < rows) {  // wave-uniform
-    for (int b = kq; b < nblk; b += 2 * nkw) {
-      block(b, kb[0], vb[0]);
-      if (b + nkw < nblk) block(b + nkw, kb[1], vb[1]);
-    }
+  for (int b = wv; b < nblk; b += 2 * NKW) {
+    block(b, kb[0], vb[0]);
+    if (b + NKW < nblk) block(b + NKW, kb[1], vb[1]);
   }
   __syncthreads();  // every wave has left its blocks
   constexpr int RED = ND * 16 + 2;  // words per lane
   float* red = reinterpret_cast<float*>(lds) + lane;
-  if (kq > 0) {
-    float* mine = red + (rb * (nkw - 1) + kq - 1) * RED * 64;
+  if (wv > 0) {
+    float* mine = red + (wv - 1) * RED * 64;
 #pragma unroll
     for (int db = 0; db < ND; ++db)
 #pragma unroll
@@ -197,11 +192,10 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
     mine[(ND * 16 + 1) * 64] = l_run;
   }
   __syncthreads();
-  if (kq > 0 || rb * 32 >= rows) return;
-  const float* others = red + rb * (nkw - 1) * RED * 64;
+  if (wv > 0) return;
   float m = m_run;
-  for (int w = 0; w < nkw - 1; ++w)
-    m = __builtin_elementwise_maximum(m, others[(w * RED + ND * 16) * 64]);
+  for (int w = 0; w < NKW - 1; ++w)
+    m = __builtin_elementwise_maximum(m, red[(w * RED + ND * 16) * 64]);
   auto weight = [&](float mw) {
     return mw == -__builtin_inf() ? 0.0f : __builtin_amdgcn_exp2f(mw - m);
   };
@@ -211,8 +205,8 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
   for (int db = 0; db < ND; ++db)
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[db][v] *= f0;
-  for (int w = 0; w < nkw - 1; ++w) {
-    const float* o = others + w * RED * 64;
+  for (int w = 0; w < NKW - 1; ++w) {
+    const float* o = red + w * RED * 64;
     const float f = weight(o[ND * 16 * 64]);
     l_run = __builtin_fmaf(f, o[(ND * 16 + 1) * 64], l_run);
 #pragma unroll

@@ -32,8 +32,9 @@ struct TilePlan {
 };
 
 // Rows (queries x query heads of the kv head) up to which a run tile counts
-// as narrow: it fills at most two of a workgroup's four 32-row waves.
-constexpr int NARROW_ROWS = 64;
+// as narrow: it fills one of a workgroup's four 32-row waves (attn.h has the
+// measurements behind the line).
+constexpr int NARROW_ROWS = 32;
 // Work and exit counters of the narrow-tile kernels inside TilePlan::counter.
 constexpr int NARROW_QUEUE_SLOT = 28, NARROW_EXIT_SLOT = 30;
 

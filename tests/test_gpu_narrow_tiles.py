@@ -1,8 +1,9 @@
-"""Run tiles of at most 64 rows at head dim 32, split over the keys between the
+"""Run tiles of at most 32 rows at head dim 32, split over the keys between the
 waves (forward and dQ): tile widths around 32 and 64 rows, key streams around
 the 32-key blocks, one wave's turn and the token map's limit, empty streams,
 repeated blocks, and scores that keep raising the running maximum, against the
-fp32 oracle; run to run bitwise."""
+fp32 oracle; run to run bitwise.  Results do not depend on a tile's width
+beyond the order of the fp32 sums."""
 
 import numpy as np
 import pytest
@@ -86,3 +87,34 @@ def test_narrow_tiles(keys, g, dtype, scores):
     _grad_close(dq, qf.grad, dtype, "dq")
     _grad_close(dk, kf.grad, dtype, "dk")
     _grad_close(dv, vf.grad, dtype, "dv")
+
+
+def _passes(nq, g, dtype, sizes, listed, gen):
+    """Forward and dQ of nq queries that all list the same blocks, and of
+    those queries among as many as fill a 128-row tile -> the two results for
+    the nq queries."""
+    d, hkv, full = 32, 2, 128 // g
+    nk = sum(sizes)
+    q, do = (torch.randn(full, hkv * g, d, generator=gen).to(dtype) for _ in range(2))
+    k, v = (torch.randn(nk, hkv, d, generator=gen).to(dtype).to(DEV) for _ in range(2))
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(sizes)]), dtype=torch.int32, device=DEV)
+    cu_sb = torch.tensor([0, len(sizes)], dtype=torch.int32, device=DEV)
+    res = []
+    for n in (nq, full):
+        rows = torch.tensor(listed, dtype=torch.int32).expand(hkv, n, -1).contiguous().to(DEV)
+        cu_q = torch.tensor([0, n], dtype=torch.int32, device=DEV)
+        x = [t[:n].contiguous().to(DEV) for t in (q, do)]
+        plan = H.SelAttnPlan(x[0].shape, k.shape, rows, cu_sb, cu, cu_q, backward=True)
+        o, lse = plan.fwd(x[0], k, v, d ** -0.5)
+        dq = plan.bwd(x[1], x[0], k, v, o, lse, d ** -0.5)[0]
+        res.append([o[:nq].cpu(), lse[:, :nq].cpu(), dq[:nq].cpu()])
+    return res
+
+
+@pytest.mark.parametrize("nq,g", [(3, 16), (4, 16), (33, 1), (64, 1), (10, 4)])
+@pytest.mark.parametrize("blocks", [3, 40])
+def test_wider_tiles_are_run_tiles(nq, g, blocks):
+    # 33 to 64 rows: the kernel of a full tile, so the same bits
+    gen = torch.Generator().manual_seed(nq)
+    a, b = _passes(nq, g, torch.bfloat16, [61] * blocks, list(range(blocks)), gen)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
