@@ -68,15 +68,19 @@ __device__ inline float row_max(const f32x16* sc) {
 }
 
 // A narrow run tile (see attn.h): rows of queries q0 .. of kv head h over the
-// stream in `sel`.  The softmax runs online with lazy rescaling (p <= 2^8),
-// each wave over its own keys; at the end the waves are merged in fp32:
-// M = max m_w, O = sum 2^(m_w - M) O_w, l likewise.
-// `lds`: the waves' V blocks while they run, then the waves' sums.
+// stream in `sel`.  Every wave starts from one reference, the row maximum of
+// the stream's first KT keys (the reference of the run-tile kernel, so that P
+// rounds as it does there whichever kernel takes the row), and follows its own
+// maximum from there with lazy rescaling (p <= 2^8); at the end the waves are
+// merged in fp32: M = max m_w, O = sum 2^(m_w - M) O_w, l likewise.
+// `lds`: the waves' V blocks while they run, then the waves' sums; `ref`: the
+// row maxima of the first two 32-key blocks.
 template <int DT, int D>
 __device__ inline __attribute__((always_inline)) void narrow_fwd(
     const AttnArgs& a, int h, int q0, int rows, const SelLds& sel, const int* map, int nkeys,
-    char* lds, int wv, int lane) {
+    char* lds, float (*ref)[32], int wv, int lane) {
   using G = KvTile<D>;
+  static_assert(KT == 64, "the first two 32-key blocks are the reference's keys");
   constexpr int NS = D / 16, ND = D / 32;
   const int hb = lane >> 5, l32 = lane & 31;
   constexpr int NKW = 4;  // waves over the keys; wave wv takes blocks wv, wv + 4, ..
@@ -112,34 +116,48 @@ __device__ inline __attribute__((always_inline)) void narrow_fwd(
   for (int i = 0; i < ND; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) oacc[i][v] = 0.0f;
-  float m_run = -__builtin_inf(), l_run = 0.0f;
-  auto block = [&](int b, u32x4* kr, u32x4* vr) __attribute__((always_inline)) {
+  // S^T = K Q^T of block b (keys past the stream score -inf), and its row
+  // maximum in log2 units.
+  auto scores = [&](int b, const u32x4* kr) __attribute__((always_inline)) {
     f32x16 sc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
 #pragma unroll
     for (int s = 0; s < NS; ++s) sc = mfma32<DT>(kr[s], qb[s], sc);
-    wave_lds_order();  // the block before this one has been read
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      *reinterpret_cast<u32x4*>(sv + G::off(l32, 2 * s + hb)) = vr[s];
-    wave_lds_order();
-    if (b + 2 * NKW < nblk) blocks.load(b + 2 * NKW, kr, vr);
     if (b * 32 + 32 > nkeys) {
 #pragma unroll
       for (int v = 0; v < 16; ++v)
         if (b * 32 + acc_row(v, hb) >= nkeys) sc[v] = -__builtin_inf();
     }
+    return sc;
+  };
+  auto block_max = [&](const f32x16& sc) __attribute__((always_inline)) {
     const float m3 = max3f(max3f(sc[0], sc[1], sc[2]), max3f(sc[3], sc[4], sc[5]),
                            max3f(sc[6], sc[7], sc[8]));
     const float mx = max3f(m3, max3f(sc[9], sc[10], sc[11]),
                            max3f(sc[12], sc[13], max3f(sc[14], sc[15], sc[15])));
     const auto sw = __builtin_amdgcn_permlane32_swap(
         __builtin_bit_cast(unsigned, mx), __builtin_bit_cast(unsigned, mx), false, false);
-    const float m_tile =
-        __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)sw[0]),
-                                      __builtin_bit_cast(float, (unsigned)sw[1])) *
-        a.scale_log2;
+    return __builtin_elementwise_maximum(__builtin_bit_cast(float, (unsigned)sw[0]),
+                                         __builtin_bit_cast(float, (unsigned)sw[1])) *
+           a.scale_log2;
+  };
+  if (wv < 2) {
+    float m = -__builtin_inf();
+    if (wv < nblk) m = block_max(scores(wv, kb[0]));
+    if (hb == 0) ref[wv][l32] = m;
+  }
+  __syncthreads();
+  float m_run = __builtin_elementwise_maximum(ref[0][l32], ref[1][l32]), l_run = 0.0f;
+  auto block = [&](int b, u32x4* kr, u32x4* vr) __attribute__((always_inline)) {
+    const f32x16 sc = scores(b, kr);
+    wave_lds_order();  // the block before this one has been read
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      *reinterpret_cast<u32x4*>(sv + G::off(l32, 2 * s + hb)) = vr[s];
+    wave_lds_order();
+    if (b + 2 * NKW < nblk) blocks.load(b + 2 * NKW, kr, vr);
+    const float m_tile = block_max(sc);
     if (__builtin_amdgcn_ballot_w64(m_tile > m_run + RESCALE_LOG2) != 0) {
       const float m_new = __builtin_elementwise_maximum(m_run, m_tile);
       const float alpha =
@@ -239,6 +257,7 @@ narrow_fwd_kernel(AttnArgs a) {
   __shared__ __align__(1024) char s_lds[RED_BYTES > V_BYTES ? RED_BYTES : V_BYTES];
   __shared__ SelLds sel;
   __shared__ int s_tokmap[KMAP_KEYS];
+  __shared__ float s_ref[2][32];
   __shared__ int s_slot;
   const int lane = threadIdx.x & 63, wv = uniform(threadIdx.x >> 6);
   const int32_t* off = a.plan.narrow_off;
@@ -257,7 +276,7 @@ narrow_fwd_kernel(AttnArgs a) {
       build_token_map(sel, s_tokmap, wv, lane);
       map = s_tokmap;
     }
-    narrow_fwd<DT, D>(a, h, tile.x, rows, sel, map, nkeys, s_lds, wv, lane);
+    narrow_fwd<DT, D>(a, h, tile.x, rows, sel, map, nkeys, s_lds, s_ref, wv, lane);
   }
   leave_queue(queue, queue + NARROW_EXIT_SLOT - NARROW_QUEUE_SLOT);
 }

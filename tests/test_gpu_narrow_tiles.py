@@ -118,3 +118,19 @@ def test_wider_tiles_are_run_tiles(nq, g, blocks):
     gen = torch.Generator().manual_seed(nq)
     a, b = _passes(nq, g, torch.bfloat16, [61] * blocks, list(range(blocks)), gen)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("nq,g", [(2, 16), (1, 16), (32, 1), (19, 1), (8, 4)])
+@pytest.mark.parametrize("blocks,size", [(1, 3), (1, 50), (3, 61), (40, 61)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_narrow_tiles_round_as_run_tiles(nq, g, blocks, size, dtype):
+    # One reference for P whatever the tile's width: the same 16-bit P, so the
+    # results differ by the order of the fp32 sums alone.  That is less than
+    # 2440 * 2^-24 < 2^-12 of the sums' terms at most and near 50 * 2^-24 as a
+    # random walk, against a rounding step of 2^-8 (bf16) or 2^-11 (fp16) of
+    # the result: far fewer than one result in fifty rounds the other way.
+    gen = torch.Generator().manual_seed(nq + blocks)
+    a, b = _passes(nq, g, dtype, [size] * blocks, list(range(blocks)), gen)
+    torch.testing.assert_close(a[1], b[1], rtol=0, atol=1e-5)
+    for x, y in ((a[0], b[0]), (a[2], b[2])):
+        assert float((x != y).float().mean()) <= 0.02
