@@ -237,7 +237,7 @@ __device__ inline double readlane_f64(double x, int j) {
 }
 
 // The best R candidates (score descending, id ascending) of those a wave
-// holds -- M per lane: candidate (lane, m) has id q0 + lane + 64 m and score
+// holds -- M per lane: candidate (lane, m) has id lane + 64 m and score
 // v[m], and bit m of `taken` marks it unavailable -- written to ls / li in
 // that order (ls may be null: ids only); returns how many there are
 // (min(R, available)).
@@ -250,7 +250,7 @@ __device__ inline double readlane_f64(double x, int j) {
 // wave butterfly.  Both give the same list, since the best R under a strict
 // total order are unique.
 template <int M>
-__device__ int wave_best_r(const double (&v)[M], uint32_t taken, int q0, int R,
+__device__ int wave_best_r(const double (&v)[M], uint32_t taken, int R,
                            double* __restrict__ ls, int* __restrict__ li,
                            double* __restrict__ cs, int* __restrict__ ci) {
   const int lane = threadIdx.x & 63;
@@ -259,9 +259,9 @@ __device__ int wave_best_r(const double (&v)[M], uint32_t taken, int q0, int R,
   int bi = INT32_MAX;
 #pragma unroll
   for (int m = 0; m < M; ++m)
-    if (!((taken >> m) & 1u) && sel_better(v[m], q0 + lane + 64 * m, bs, bi)) {
+    if (!((taken >> m) & 1u) && sel_better(v[m], lane + 64 * m, bs, bi)) {
       bs = v[m];
-      bi = q0 + lane + 64 * m;
+      bi = lane + 64 * m;
     }
   const int nv = __popcll(__ballot(bi != INT32_MAX));
   int S = 65;
@@ -277,7 +277,7 @@ __device__ int wave_best_r(const double (&v)[M], uint32_t taken, int q0, int R,
     S = 0;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      const int id = q0 + lane + 64 * m;
+      const int id = lane + 64 * m;
       const bool p = !((taken >> m) & 1u) && !sel_better(ts, ti, v[m], id);
       const unsigned long long bm = __ballot(p);
       const int pos = S + (int)__builtin_amdgcn_mbcnt_hi(
@@ -312,9 +312,9 @@ __device__ int wave_best_r(const double (&v)[M], uint32_t taken, int q0, int R,
     int ri = INT32_MAX;
 #pragma unroll
     for (int m = 0; m < M; ++m)
-      if (!((tk >> m) & 1u) && sel_better(v[m], q0 + lane + 64 * m, rs, ri)) {
+      if (!((tk >> m) & 1u) && sel_better(v[m], lane + 64 * m, rs, ri)) {
         rs = v[m];
-        ri = q0 + lane + 64 * m;
+        ri = lane + 64 * m;
       }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -327,8 +327,7 @@ __device__ int wave_best_r(const double (&v)[M], uint32_t taken, int q0, int R,
     }
     ri = __builtin_amdgcn_readfirstlane(ri);
     if (ri == INT32_MAX) break;  // no candidate left
-    const int lc = ri - q0;
-    if ((lc & 63) == lane) tk |= 1u << (lc >> 6);
+    if ((ri & 63) == lane) tk |= 1u << (ri >> 6);
     if (lane == 0) {
       if (ls) ls[nw] = rs;
       li[nw] = ri;
@@ -513,7 +512,7 @@ __global__ __launch_bounds__(256) void topk_wave_kernel(
   for (int f = 0; f < n_forced; ++f) take(forced[f]);
   __shared__ double s_cs[4][64];
   __shared__ int s_ci[4][64];
-  n += wave_best_r<M>(v, taken, 0, kmax - n, nullptr, sel + n, s_cs[wv], s_ci[wv]);
+  n += wave_best_r<M>(v, taken, kmax - n, nullptr, sel + n, s_cs[wv], s_ci[wv]);
   asm volatile("" ::: "memory");
   // Ascending ids (distinct), -1 padding: id -> its rank among the chosen.
   __shared__ int s_out[4][SEL_MAXK];
@@ -541,11 +540,14 @@ __global__ __launch_bounds__(256) void topk_wave_kernel(
 // only the columns that reach it are listed (about topk of them, at most four
 // per class that reaches the bound) and ranked by wave_best_r.  The forced
 // blocks are taken first and count among the topk.  More than BOUND_CAP such
-// columns (ties in great number) take one scan of the row per pick.
+// columns (ties in great number) are taken in pieces, each ranked beside the
+// best so far: whole selections of 4 x 4881 rows, top-32, take 0.65 ms, 0.70
+// with all scores equal or NaN (0.92 with four waves per row, 4.56 with one
+// scan of the row per pick); 4 x 8192 rows, top-64, 1.38 and 1.57 (2.45, 34.8).
 // Bound by reading the scores once (the row's arithmetic is a third of that):
 // 4 x 4881 rows of 4881 scores, top-32, 465 us with four waves per row that
 // each listed their quarter's best, 286 us here (763 MB of scores read and 268 MB of
-// token rows written: 3.8 TB/s).
+// token rows written: 3.6 TB/s).
 constexpr int BOUND_CAP = 1024;
 
 template <int NM>
@@ -555,7 +557,7 @@ __global__ __launch_bounds__(64) void topk_bound_kernel(
     int64_t n_tokens, int topk, const int32_t* __restrict__ forced, int n_forced,
     int force_self, int32_t* __restrict__ topk_idx, int32_t* __restrict__ compact) {
   __shared__ int s_id[BOUND_CAP];
-  __shared__ double s_cs[64];
+  __shared__ double s_cs[64], s_ls[64];
   __shared__ int s_ci[64], s_at[64], s_sel[64], s_out[64];
   const int h = blockIdx.y;
   const int64_t b = blockIdx.x;
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(64) void topk_bound_kernel(
       }
       if (at >= n || is_forced(s_id[at])) taken |= 1u << m;
     }
-    const int nw = wave_best_r<M>(v, taken, 0, r_need, nullptr, s_at, s_cs, s_ci);
+    const int nw = wave_best_r<M>(v, taken, r_need, nullptr, s_at, s_cs, s_ci);
     __syncthreads();
     if (lane < nw) s_sel[nf + lane] = s_id[s_at[lane]];
   };
@@ -654,36 +656,41 @@ __global__ __launch_bounds__(64) void topk_bound_kernel(
     best(std::integral_constant<int, 4>{});
   } else if (n <= BOUND_CAP) {
     best(std::integral_constant<int, BOUND_CAP / 64>{});
-  } else {
-    double ps = 0.0;
-    int pi = -1;  // the pick before (none)
-    for (int r = 0; r < r_need; ++r) {
-      double bs = -__builtin_inf();
-      int bi = INT32_MAX;
-      for (int i = lane; i < nbb; i += 64) {
-        double x = row[i];
-        if (x != x) x = -__builtin_inf();
-        if ((pi < 0 || sel_better(ps, pi, x, i)) && sel_better(x, i, bs, bi) && !is_forced(i)) {
-          bs = x;
-          bi = i;
-        }
-      }
+  } else if (r_need > 0) {
+    // 960 columns at a time beside the best so far (places 0 .. 63, best
+    // first).  Those have smaller ids than the columns, so places rank ties
+    // as ids do, and only a column above the last of them can enter.
+    constexpr int M = BOUND_CAP / 64;
+    int nc = 0;
+    double cv = 0.0, last = 0.0;  // this lane's score of the best so far, the last one
+    for (int base = 0; base < nbb; base += 64 * (M - 1)) {
+      double v[M];
+      v[0] = cv;
+      uint32_t taken = lane < nc ? 0u : 1u;
+      bool enters = false;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        const double os = __shfl_xor(bs, o);
-        const int oi = __shfl_xor(bi, o);
-        if (sel_better(os, oi, bs, bi)) {
-          bs = os;
-          bi = oi;
-        }
+      for (int m = 1; m < M; ++m) {
+        const int i = base + 64 * (m - 1) + lane;
+        const double x = i < nbb ? row[i] : -__builtin_inf();
+        v[m] = x == x ? x : -__builtin_inf();
+        if (i >= nbb || is_forced(i)) taken |= 1u << m;
+        enters |= v[m] > last;
       }
-      ps = bs;
-      pi = bi;
-      if (lane == 0) s_ci[r] = bi;
+      if (nc == r_need && !__ballot(enters)) continue;
+      const int nw = wave_best_r<M>(v, taken, r_need, s_ls, s_at, s_cs, s_ci);
+      __syncthreads();
+      const int at = lane < nw ? s_at[lane] : 0;
+      const int id = at < 64 ? s_id[at] : base + at - 64;
+      if (lane < nw) cv = s_ls[lane];
+      __syncthreads();
+      if (lane < nw) s_id[lane] = id;
+      nc = nw;
+      last = readlane_f64(cv, nw > 0 ? nw - 1 : 0);
+      __syncthreads();
     }
-    __syncthreads();
-    if (lane < r_need) s_sel[nf + lane] = s_ci[lane];
+    if (lane < nc) s_sel[nf + lane] = s_id[lane];
   }
+  __syncthreads();
   // Ascending order by rank (ids are distinct), -1 padding.
   if (lane < topk) s_out[lane] = -1;
   __syncthreads();

@@ -68,3 +68,45 @@ def test_scores(kind):
     else:                       # the best scores are neighbours
         pk[:, 0] = -(torch.arange(nb) - 1200).abs() / 64.0
     _check(pq, pk, [0, nb], topk, [1])
+
+
+@pytest.mark.parametrize("nb,topk", [(2880, 64), (2881, 33), (4881, 32), (8192, 64)])
+@pytest.mark.parametrize("kind", ["equal", "nan", "late", "steps"])
+def test_ties_in_pieces(nb, topk, kind):
+    # more columns at the bound than are listed: pieces of 960 columns
+    pq, pk = torch.zeros(nb, 32), torch.zeros(nb, 32)
+    pq[:, 0] = 1.0
+    i = torch.arange(nb)
+    if kind == "equal":
+        pk[:, 0] = 0.25
+    elif kind == "nan":
+        pk[:, 0] = float("nan")
+    elif kind == "late":    # a few columns above the ties in every piece
+        pk[(i % 960 == 959) | (i == nb - 1), 0] = 1.0 + nb
+    else:                   # the better columns come later, piece by piece
+        pk[:, 0] = (i // 700).float()
+    _check(pq, pk, [0, nb], topk, [1, 960, nb - 2, 961])
+
+
+def test_ties_cost_no_scan_per_pick():
+    # one layer's scores all equal (zero projections) or NaN (a diverged step)
+    # against ordinary ones: the same pass over the scores, some more ranking
+    nb, topk = 4881, 32
+    cu = torch.arange(nb + 1, dtype=torch.int32, device=DEV)
+    sb = torch.tensor([0, nb], dtype=torch.int32, device=DEV)
+    q, k = torch.randn(2, nb, 4, 64, device=DEV)
+
+    def best(keys):
+        times = []
+        for _ in range(6):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            H.select_blocks(q, keys, sb, cu, topk)
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    usual = best(k)
+    for value in (0.25, float("nan")):
+        assert best(torch.full_like(k, value)) <= 2 * usual
