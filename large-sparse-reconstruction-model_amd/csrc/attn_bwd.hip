@@ -242,7 +242,8 @@ sel_attn_dq_kernel(AttnArgs a) {
   const int32_t* head_off =
       GATHER ? a.kc.fitem_off
              : (UNION ? a.plan.ghead_off : (WIDE ? a.plan.wide_off : a.plan.head_off));
-  const int2* tiles = UNION ? a.plan.gtiles : (WIDE ? a.plan.by_width : a.plan.tiles);
+  const bool by_width = WIDE && a.plan.counter[BY_WIDTH_SLOT] != 0;  // else wide_off is head_off
+  const int2* tiles = UNION ? a.plan.gtiles : (by_width ? a.plan.by_width : a.plan.tiles);
   int32_t* queue = a.plan.counter + (GATHER ? KC_QUEUE_SLOT : (UNION ? 4 : 0));
   // A plan built without its backward part: nothing here is valid to read.
   if (a.plan.counter[PLAN_BWD_SLOT] != PLAN_BWD_MAGIC) return;

@@ -106,8 +106,12 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
   const bool backward = (flags & LSRM_PLAN_BACKWARD) != 0;
   const int tq = ROWS / g;
   bool derive = false;  // the backward's query map comes from the key-centric one
-  int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, NARROW_ROWS / g, ws,
-                           w.plan, st);
+  // Run tiles are listed by width for the head dims whose kernels read that
+  // list (0: not known yet).  The list is carved for all of them, since plans
+  // without the key-centric part serve every head dim.
+  const int narrow_q = narrow_split((int)head_dim) ? NARROW_ROWS / g : 0;
+  int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, narrow_q, ws, w.plan,
+                           st);
   if (rc) return rc;
   if (backward) {
     // dK/dV rows: the run tiles that selected a block, then the queries of

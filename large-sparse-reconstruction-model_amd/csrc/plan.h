@@ -23,9 +23,9 @@ struct TilePlan {
   int2* gtiles;          // [hkv, n_q] grouped tiles (forward plans)
   int32_t* gtile_count;  // [hkv]
   int32_t* ghead_off;    // [hkv + 1]
-  // The run tiles again, by width: those of more than narrow_rows / g queries
-  // from the front of each head's part, the narrow ones from its end
-  // backwards.
+  // The run tiles again, by width: those of more than narrow_q queries from
+  // the front of each head's part, the narrow ones from its end backwards.
+  // Filled where counter[BY_WIDTH_SLOT] is set (with narrow_q > 0).
   int2* by_width;        // [hkv, n_q]
   int32_t* wide_off;     // [hkv + 1]
   int32_t* narrow_off;   // [hkv + 1]
@@ -37,6 +37,8 @@ struct TilePlan {
 constexpr int NARROW_ROWS = 32;
 // Work and exit counters of the narrow-tile kernels inside TilePlan::counter.
 constexpr int NARROW_QUEUE_SLOT = 28, NARROW_EXIT_SLOT = 30;
+// [BY_WIDTH_SLOT]: 1 when the plan lists the run tiles by width.
+constexpr int BY_WIDTH_SLOT = 36;
 
 // Marks a plan whose backward part was built: the backward kernels exit
 // without touching memory when the slot does not hold the magic word (a
@@ -58,8 +60,8 @@ struct RevMap {
 };
 
 // Workspace carving: pass a Carver with base == nullptr to size.
-// Consecutive short run tiles move into grouped tiles; the others are also
-// listed by width (narrow: at most narrow_q queries).
+// Consecutive short run tiles move into grouped tiles; with narrow_q > 0 the
+// others are also listed by width (narrow: at most narrow_q queries).
 int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
                     int64_t topk_n, const int32_t* cu_q, int64_t batch,
                     const int32_t* cu_sb, int tq, int narrow_q, Carver& ws, TilePlan& plan,

@@ -50,13 +50,14 @@ __device__ inline T block_excl_scan(T v, T* total) {
 }
 
 // The type of a scan's values: int, or a pair of counts packed in 64 bits.
+template <bool BY_WIDTH>
 struct SplitF;
 template <class F>
 struct ScanValue {
   using type = int32_t;
 };
 template <>
-struct ScanValue<SplitF> {
+struct ScanValue<SplitF<true>> {
   using type = int64_t;
 };
 template <class F>
@@ -425,8 +426,10 @@ struct GroupW {
     if (t == lim - 1) gs[ex + v] = (int32_t)lim;
   }
 };
-// Second pass over the groups: grouped (>= 2 run tiles) or kept, and whether a
-// kept tile is narrow; the two counts are scanned together, packed in 64 bits.
+// Second pass over the groups: grouped (>= 2 run tiles) or kept, and for a list
+// by width whether a kept tile is narrow; the two counts are scanned together,
+// packed in 64 bits.
+template <bool BY_WIDTH>
 struct SplitF {
   const int2* run_tiles;
   const int32_t* gstart;
@@ -434,23 +437,28 @@ struct SplitF {
   int64_t nq;
   int narrow_q;
   __device__ int64_t limit(int h, int64_t) const { return n_groups[h]; }
-  __device__ int64_t operator()(int h, int64_t s) const {
+  __device__ scan_t<SplitF> operator()(int h, int64_t s) const {
     const int32_t* gs = gstart + (int64_t)h * (nq + 1);
     if (gs[s + 1] - gs[s] > 1) return 1;
-    return run_tiles[(int64_t)h * nq + gs[s]].y <= narrow_q ? int64_t{1} << 32 : 0;
+    if constexpr (BY_WIDTH)
+      return run_tiles[(int64_t)h * nq + gs[s]].y <= narrow_q ? int64_t{1} << 32 : 0;
+    else
+      return 0;
   }
 };
+template <bool BY_WIDTH>
 struct SplitW {
+  using T = scan_t<SplitF<BY_WIDTH>>;
   const int2* run_tiles;
   const int32_t* gstart;
   int64_t nq;
   int2* tiles;
   int2* gtiles;
   int2* by_width;
-  __device__ void operator()(int h, int64_t s, int64_t ex, int64_t v, int64_t) const {
+  __device__ void operator()(int h, int64_t s, T ex, T v, int64_t) const {
     const int32_t* gs = gstart + (int64_t)h * (nq + 1);
     const int t0 = gs[s], t1 = gs[s + 1];
-    const int64_t g = (int32_t)ex, nar = ex >> 32;  // grouped, narrow tiles before
+    const int64_t g = (int32_t)ex;  // grouped tiles before
     const int64_t at = (int64_t)h * nq;
     const int2 first = run_tiles[at + t0];
     if (v == 1) {
@@ -459,15 +467,19 @@ struct SplitW {
       return;
     }
     tiles[at + (s - g)] = first;
-    by_width[at + (v ? nq - 1 - nar : s - g - nar)] = first;
+    if constexpr (BY_WIDTH) {
+      const int64_t nar = ex >> 32;  // narrow tiles before
+      by_width[at + (v ? nq - 1 - nar : s - g - nar)] = first;
+    }
   }
 };
 
 // The lists' counts per head from the groups and the split's totals, and the
 // heads' offsets in every list (lane i takes list i: run tiles, grouped, wide,
-// narrow).
-__global__ void plan_offsets_kernel(const int32_t* n_groups, const int64_t* split,
-                                    TilePlan plan, int hkv) {
+// narrow).  T: the split's scan type (64 bits: with narrow tiles counted).
+template <class T>
+__global__ void plan_offsets_kernel(const int32_t* n_groups, const T* split, TilePlan plan,
+                                    int hkv) {
   if (blockIdx.x != 0) return;
   if (threadIdx.x < 4) {
     const int i = threadIdx.x;
@@ -478,7 +490,8 @@ __global__ void plan_offsets_kernel(const int32_t* n_groups, const int64_t* spli
     for (int h = 0; h < hkv; ++h) {
       int c = 0;
       if (n_groups) {
-        const int g = (int32_t)split[h], nar = (int)(split[h] >> 32), kept = n_groups[h] - g;
+        const int g = (int32_t)split[h], kept = n_groups[h] - g;
+        const int nar = sizeof(T) == 8 ? (int)((int64_t)split[h] >> 32) : 0;
         c = i == 0 ? kept : (i == 1 ? g : (i == 2 ? kept - nar : nar));
       }
       if (i == 0) plan.tile_count[h] = c;
@@ -492,6 +505,7 @@ __global__ void plan_offsets_kernel(const int32_t* n_groups, const int64_t* spli
     for (int i = 0; i < PLAN_BWD_SLOT; ++i) counter[i] = 0;
     counter[PLAN_BWD_SLOT] = 0;  // set again by mark_backward_plan
     counter[PLAN_KC_SLOT] = 0;   // set again by the key-centric part
+    counter[BY_WIDTH_SLOT] = sizeof(T) == 8 ? 1 : 0;
   }
 }
 
@@ -505,6 +519,27 @@ __global__ void mark_backward_plan_kernel(TilePlan plan, int hkv, int packed) {
 int mark_backward_plan(const TilePlan& plan, int64_t hkv, bool packed, hipStream_t st) {
   hipLaunchKernelGGL(mark_backward_plan_kernel, dim3(1), dim3(64), 0, st, plan, (int)hkv,
                      packed ? 1 : 0);
+  LSRM_CHECK_LAUNCH();
+  return LSRM_OK;
+}
+
+// The last scan and the lists' offsets: the grouped tiles go to their list, and
+// with BY_WIDTH the others also to the one by width.
+template <bool BY_WIDTH>
+int split_tiles(const int2* run_tiles, const int32_t* gstart, const int32_t* n_groups, int64_t hkv,
+                int64_t nq, int narrow_q, int64_t* sums, int64_t* split, const TilePlan& plan,
+                hipStream_t st) {
+  using T = scan_t<SplitF<BY_WIDTH>>;
+  T* totals = reinterpret_cast<T*>(split);
+  if (nq > 0) {
+    const int rc =
+        run_scan(SplitF<BY_WIDTH>{run_tiles, gstart, n_groups, nq, narrow_q},
+                 SplitW<BY_WIDTH>{run_tiles, gstart, nq, plan.tiles, plan.gtiles, plan.by_width},
+                 nq, (int)hkv, reinterpret_cast<T*>(sums), totals, st);
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(plan_offsets_kernel<T>, dim3(1), dim3(64), 0, st,
+                     nq > 0 ? n_groups : nullptr, totals, plan, (int)hkv);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }
@@ -581,15 +616,9 @@ int build_tile_plan(const int32_t* topk, int64_t hkv, int64_t nq,
     rc = run_scan(GroupF{brk, run_count, nq}, GroupW{gstart, nq}, nq, (int)hkv, sums, n_groups,
                   st);
     if (rc) return rc;
-    rc = run_scan(SplitF{run_tiles, gstart, n_groups, nq, narrow_q},
-                  SplitW{run_tiles, gstart, nq, plan.tiles, plan.gtiles, plan.by_width}, nq,
-                  (int)hkv, split_sums, split, st);
-    if (rc) return rc;
   }
-  hipLaunchKernelGGL(plan_offsets_kernel, dim3(1), dim3(64), 0, st, nq > 0 ? n_groups : nullptr,
-                     split, plan, (int)hkv);
-  LSRM_CHECK_LAUNCH();
-  return LSRM_OK;
+  const auto split_lists = narrow_q > 0 ? split_tiles<true> : split_tiles<false>;
+  return split_lists(run_tiles, gstart, n_groups, hkv, nq, narrow_q, split_sums, split, plan, st);
 }
 
 // --------------------------------------------------------- reverse map --

@@ -134,3 +134,33 @@ def test_narrow_tiles_round_as_run_tiles(nq, g, blocks, size, dtype):
     torch.testing.assert_close(a[1], b[1], rtol=0, atol=1e-5)
     for x, y in ((a[0], b[0]), (a[2], b[2])):
         assert float((x != y).float().mean()) <= 0.02
+
+
+def test_list_by_width_only_where_it_is_read():
+    # One run tile per query: a plan for head dim 64 leaves the list by width
+    # unwritten, one for head dim 32 writes it; run at head dim 32, both give
+    # the same rows up to the order of the fp32 sums.
+    gen = torch.Generator().manual_seed(5)
+    n, hkv, g, d, nb, topk, flags = 2048, 2, 32, 32, 40, 3, H.PLAN_BACKWARD
+    rows = (torch.arange(n)[:, None] + torch.tensor([0, 7, 19])) % nb
+    rows = rows.expand(hkv, -1, -1).to(torch.int32).contiguous().to(DEV)
+    cu = (torch.arange(nb + 1, dtype=torch.int32) * 33).to(DEV)
+    cu_sb, cu_q = (torch.tensor([0, x], dtype=torch.int32, device=DEV) for x in (nb, n))
+    q, do = (torch.randn(n, hkv * g, d, generator=gen).to(torch.bfloat16).to(DEV)
+             for _ in range(2))
+    k, v = (torch.randn(nb * 33, hkv, d, generator=gen).to(torch.bfloat16).to(DEV)
+            for _ in range(2))
+    untouched, results = {}, {}
+    for plan_d in (32, 64):
+        plan = H.SelAttnPlan(q.shape, k.shape, rows, cu_sb, cu, cu_q, backward=True)
+        plan.ws.fill_(0x5a)
+        p = H._ptr
+        assert H.lib().lsrm_sel_attn_plan2(
+            p(rows), n, k.shape[0], hkv * g, hkv, plan_d, topk, p(cu_sb), p(cu), nb, p(cu_q), 1,
+            flags, p(plan.ws), plan.ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+        untouched[plan_d] = int((plan.ws == 0x5a).sum())
+        o, lse = plan.fwd(q, k, v, d ** -0.5)
+        results[plan_d] = (o, lse) + plan.bwd(do, q, k, v, o, lse, d ** -0.5)
+    assert untouched[64] - untouched[32] >= 7 * hkv * n  # (some bytes are the filler)
+    for a, b in zip(*results.values()):  # 16-bit rounding steps of the few that round otherwise
+        torch.testing.assert_close(a, b, rtol=2.0 ** -7, atol=2e-3)
