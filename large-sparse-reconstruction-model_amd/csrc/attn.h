@@ -43,7 +43,7 @@ struct AttnArgs {
   RevMap rev;        // backward: block -> run tiles that selected it
   RevMap qrev;       // backward: block -> queries of grouped tiles that
                      // selected it (one entry per listing, ascending)
-  const int32_t* qmap_n; // backward: > 0 when qrev may list queries
+  const int32_t* qmap_n; // backward: > 0 when qrev lists queries
                          // (the plan's PLAN_QMAP_SLOT)
   KeyItems items;    // backward: key chunks of every block
   KcPlan kc;         // key-centric plans only (kc.fitems null otherwise)

@@ -150,7 +150,7 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
     rc = build_key_items(cu_blk, nb, nk, ws, w.items, st);
     if (rc) return rc;
     if (ws.base && !ws.dry) {
-      rc = mark_backward_plan(w.plan, hkv, packed_q > 0, st);
+      rc = mark_backward_plan(w.plan, hkv, packed_q > 0 ? w.qrev.totals : nullptr, st);
       if (rc) return rc;
     }
   }

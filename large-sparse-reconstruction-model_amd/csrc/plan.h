@@ -45,11 +45,12 @@ constexpr int BY_WIDTH_SLOT = 36;
 // forward-only plan in a workspace large enough for the backward).
 constexpr int PLAN_BWD_SLOT = 32;
 constexpr int32_t PLAN_BWD_MAGIC = 0x4c42574b;
-// [PLAN_QMAP_SLOT] > 0: the plan's query map may list queries (it has grouped
-// tiles, or `packed`: queries of run tiles are listed too), whatever flags a
-// later run is given.
+// [PLAN_QMAP_SLOT] > 0: the plan's query map lists queries (of grouped tiles
+// or, where the plan packs short run tiles, of those too), whatever flags a
+// later run is given.  totals: the map's listings per kv head; null for a map
+// that holds the grouped tiles' queries alone.
 constexpr int PLAN_QMAP_SLOT = 34;
-int mark_backward_plan(const TilePlan& plan, int64_t hkv, bool packed, hipStream_t st);
+int mark_backward_plan(const TilePlan& plan, int64_t hkv, const int32_t* totals, hipStream_t st);
 
 // CSR map block -> rows (tiles or queries) that selected it, per kv head.
 struct RevMap {

@@ -509,16 +509,17 @@ __global__ void plan_offsets_kernel(const int32_t* n_groups, const T* split, Til
   }
 }
 
-__global__ void mark_backward_plan_kernel(TilePlan plan, int hkv, int packed) {
+__global__ void mark_backward_plan_kernel(TilePlan plan, int hkv, const int32_t* totals) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
-    plan.counter[PLAN_QMAP_SLOT] = packed ? 1 : plan.ghead_off[hkv];
+    int listed = totals ? 0 : plan.ghead_off[hkv];
+    for (int h = 0; totals && h < hkv; ++h) listed |= totals[h] > 0 ? 1 : 0;
+    plan.counter[PLAN_QMAP_SLOT] = listed;
     plan.counter[PLAN_BWD_SLOT] = PLAN_BWD_MAGIC;
   }
 }
 
-int mark_backward_plan(const TilePlan& plan, int64_t hkv, bool packed, hipStream_t st) {
-  hipLaunchKernelGGL(mark_backward_plan_kernel, dim3(1), dim3(64), 0, st, plan, (int)hkv,
-                     packed ? 1 : 0);
+int mark_backward_plan(const TilePlan& plan, int64_t hkv, const int32_t* totals, hipStream_t st) {
+  hipLaunchKernelGGL(mark_backward_plan_kernel, dim3(1), dim3(64), 0, st, plan, (int)hkv, totals);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }

@@ -81,3 +81,30 @@ def test_packed_plan_run_without_flags():
     assert float(dk.float().abs().max()) > 0
     for a, b in zip((dq, dk, dv, delta), want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("run,listed", [(5, False), (4, True), (1, True)])
+@pytest.mark.parametrize("key_centric", [True, False])
+def test_query_map_counts_as_used_only_if_it_lists(run, listed, key_centric):
+    # Runs longer than half a tile are neither packed nor grouped: dK/dV runs
+    # without the map's steps (they cost 3 to 10% of its time), whether or not
+    # the plan is key-centric.  The word lies two behind the backward marker.
+    gen = torch.Generator().manual_seed(run)
+    n, hkv, g, d, nb, topk = 640, 2, 16, 32, 40, 3
+    rows = torch.stack([torch.randperm(nb, generator=gen)[:topk] for _ in range(hkv * n // run)])
+    rows = rows.view(hkv, n // run, topk).repeat_interleave(run, dim=1).to(torch.int32)
+    cu = torch.arange(nb + 1, dtype=torch.int32) * (n // nb)
+    cu_sb, cu_q = (torch.tensor([0, x], dtype=torch.int32) for x in (nb, n))
+    rows, cu_sb, cu, cu_q = (t.contiguous().to(DEV) for t in (rows, cu_sb, cu, cu_q))
+    plan = H.SelAttnPlan((n, hkv * g, d), (n, hkv, d), rows, cu_sb, cu, cu_q, backward=True,
+                         key_centric=key_centric)
+    plan.ws.zero_()  # and built again: the memory may hold an older plan's words
+    p = H._ptr
+    assert H.lib().lsrm_sel_attn_plan2(
+        p(rows), n, n, hkv * g, hkv, d, topk, p(cu_sb), p(cu), nb, p(cu_q), 1, plan.flags,
+        p(plan.ws), plan.ws.numel(), torch.cuda.current_stream().cuda_stream) == 0
+    words = plan.ws[:plan.ws.numel() // 4 * 4].view(torch.int32).cpu()
+    at = (words == 0x4c42574b).nonzero().flatten().tolist()
+    assert len(at) == 1
+    grouped = run == 1  # without the key-centric part only grouped tiles are listed
+    assert (int(words[at[0] + 2]) > 0) == (listed if key_centric else grouped)
