@@ -740,12 +740,4 @@ struct NarrowBlocks {
   }
 };
 
-// Orders a wave's own LDS writes before its later reads of other lanes' data
-// (one wave's LDS operations execute in order; this holds the compiler to it).
-__device__ inline void wave_lds_order() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 }  // namespace lsrm

@@ -139,6 +139,14 @@ __device__ inline int64_t upper_index(const int32_t* a, int64_t lo,
   return l - 1;
 }
 
+// Orders a wave's own LDS writes before its later reads of other lanes' data
+// (one wave's LDS operations execute in order; this holds the compiler to it).
+__device__ inline void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }

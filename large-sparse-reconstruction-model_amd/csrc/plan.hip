@@ -6,7 +6,7 @@
 // _scatter_queries_kernel / host-looped segmented sort
 // (sparse/ops/triton_native_sparse_attention_impl_kvcentric.py:494-684),
 // all on the device and without host synchronisation: for rows that are
-// queries, a stable counting sort over chunks of queries; for rows that are
+// queries, stable counting passes over chunks of them; for rows that are
 // run tiles, count -> scan -> atomic scatter -> per-segment sort.
 #include <algorithm>
 
@@ -869,31 +869,53 @@ __global__ __launch_bounds__(256) void rev_sort_kernel(
   for (int64_t i = threadIdx.x; i < len; i += blockDim.x) seg[i] = out[i];
 }
 
-// --------------------------------- query rows: one stable counting sort --
+// --------------------------------- query rows: stable counting passes --
 // Rows that are queries (all of them, or those marked in `only`): a head's
-// queries are cut into chunks, each chunk's listings counted per block in
-// LDS, the counts scanned in (block, chunk) order, and each chunk's listings
-// placed in (query, slot) order behind the chunk's offset in every block.
-// Two reads of the marked rows and one write of each listing: bound by LDS
-// atomics and the scattered 4-byte writes.  A chunk without marked queries
-// costs its mask bytes, so a plan over block rows (nothing marked) does no
-// sort at all.  A radix sort of (block, listing) pairs took, pairs and
-// placement included, 1240 us at 24 heads x 131072 per-token top-16 rows and
-// 1450 us at 4 x 524288 top-32 block rows with nothing marked.
-constexpr int REV_WIN = 4096;          // blocks per workgroup (48 KB of LDS)
-constexpr int64_t REV_WAVES = 4096;    // chunks over all heads: 16 waves per CU
-constexpr int64_t REV_COUNTS = 8 << 20;  // chunk counts over all heads, at most (32 MB)
+// queries are cut into chunks, each chunk's listings counted per block in LDS,
+// the counts scanned in (block, chunk) order, and each chunk's listings placed
+// in (query, slot) order behind the chunk's offset in every block.  Where the
+// counts would outgrow the listings (rev_one_pass) two such passes sort by the
+// low and then by the high half of the block number, the first from the rows,
+// the second from the first's (block, listing) pairs.  A chunk without marked
+// queries costs its mask bytes and its zero counts, which are written and
+// scanned like others.
+//
+// Bound by the vector instructions of the ranks and by the scattered writes.
+// Whole maps (us), against a radix sort of (block, listing) pairs and against
+// chunks placed through one 64-query mask per block:
+//   2 heads x 131072 top-16 rows over 462 / 4881 / 30000 blocks:
+//     136 / 137 / 138, 115 / 322 / 710, here 66 / 115 / 140
+//   24 x 131072 top-16 over 462 / 4881 / 30000:
+//     1246 / 1611 / 1668, 905 / 2570 / 6700, here 566 / 961 / 1417
+//   rows that list a block twice: as others with the sort and here, 3 to 6
+//   times as long with masks.
+// Backward plan of 4 x 524288 top-32 block rows over 4881 blocks (no listing):
+// 1795 with the sort, 400 here.
+constexpr int REV_WIN = 8192;            // buckets per workgroup (32 KB of LDS)
+// Whether one pass takes the whole block number: a second pass costs its six
+// launches and another trip of every listing, one pass counts and writes that
+// spread over more blocks.  One / two passes (us): 2 heads x 131072 top-16
+// rows, 2048 blocks 95 / 111, 4881 blocks 147 / 115; 8 x 65536 top-32, 4881
+// blocks 331 / 297; 24 x 131072 top-16, 4881 blocks 961 / 1007, 8192 blocks 848
+// / 1116, 16384 blocks 1514 / 1323.
+inline bool rev_one_pass(int64_t listings, int64_t nb) {
+  return nb <= 2048 || (nb <= 8192 && listings >= (int64_t{1} << 25));
+}
+// Chunks over all heads (one wave per SIMD; of two passes, with less work in
+// each, four) and chunk counts over all heads, at most (16 and 8 MB).
+constexpr int64_t REV_WAVES = 1024, REV_COUNTS = 4 << 20;
+constexpr int64_t REV_WAVES_2 = 4096, REV_COUNTS_2 = 2 << 20;
 
 struct RevChunks {
-  int64_t len, n;  // queries per chunk (a multiple of 64), chunks per head
+  int64_t len, n;  // items per chunk (a multiple of `unit`), chunks per head
 };
-inline RevChunks rev_chunks(int64_t hkv, int64_t nq, int64_t nb) {
-  int64_t n = std::min<int64_t>(ceil_div(REV_WAVES, hkv), REV_COUNTS / (hkv * (nb > 0 ? nb : 1)));
-  n = std::max<int64_t>(1, std::min<int64_t>(n, (nq + 63) / 64));
+inline RevChunks rev_chunks(bool one, int64_t hkv, int64_t items, int64_t unit, int64_t buckets) {
+  int64_t n = std::min<int64_t>(ceil_div(one ? REV_WAVES : REV_WAVES_2, hkv),
+                                (one ? REV_COUNTS : REV_COUNTS_2) / (hkv * buckets));
+  n = std::max<int64_t>(1, std::min<int64_t>(n, (items + unit - 1) / unit));
   RevChunks c;
-  c.len = (((nq + n - 1) / n) + 63) / 64 * 64;
-  if (c.len < 64) c.len = 64;
-  c.n = std::max<int64_t>(1, (nq + c.len - 1) / c.len);
+  c.len = std::max<int64_t>(unit, ((items + n - 1) / n + unit - 1) / unit * unit);
+  c.n = std::max<int64_t>(1, (items + c.len - 1) / c.len);
   return c;
 }
 
@@ -906,9 +928,32 @@ struct RevQueries {
   const int32_t* cu_sb;
   int64_t nb;
   const uint8_t* only;  // [hkv, nq], or null: every query
-  int64_t chunk_len;
-  int n_chunks;
+  bool encode;          // a listing stores q * k + slot, else q
 };
+
+// One pass: what it reads, and its buckets.
+struct RevPass {
+  RevQueries rows;      // read when pairs is null
+  const int2* pairs;    // [hkv, in_cap]: the listings' blocks and what they store
+  const int32_t* n_in;  // [hkv]: their number
+  int64_t in_cap;
+  int shift, mask;      // block c lies in bucket (c >> shift) & mask
+  int64_t buckets;
+  int64_t chunk_len;    // queries, or pairs, per chunk
+  int n_chunks, hkv;
+};
+
+// Workgroup -> (head, chunk): each XCD takes consecutive chunks, so that the
+// neighbouring counts and listings that they write meet in one L2.
+struct RevItem {
+  int h, chunk;
+};
+__device__ inline bool rev_item(const RevPass& a, RevItem* it) {
+  const int item = (int)(blockIdx.x % 8) * (int)(gridDim.x / 8) + (int)(blockIdx.x / 8);
+  it->h = item / a.n_chunks;
+  it->chunk = item - it->h * a.n_chunks;
+  return it->h < a.hkv;
+}
 
 // The queries q0 .. q0 + 63 of head h that are listed (bit i: q0 + i).
 __device__ inline uint64_t rev_marked(const RevQueries& a, int h, int64_t q0, int lane) {
@@ -916,13 +961,12 @@ __device__ inline uint64_t rev_marked(const RevQueries& a, int h, int64_t q0, in
   return __ballot(q < a.nq && (!a.only || a.only[(int64_t)h * a.nq + q]));
 }
 
-// Calls f(r, j, c) for every listed id of queries q0 .. q0 + 63 whose global
-// block lies in [w0, w1): r the query's index in the group, j the slot, c the
-// block.  U ids per load (4: rows of whole, aligned 16-byte pieces).  One
-// wave; consecutive lanes hold consecutive ids.
+// Calls f(c) for the block c of every listing of the marked queries among
+// q0 .. q0 + 63.  U ids per load (4: rows of whole, aligned 16-byte pieces).
+// One wave; consecutive lanes hold consecutive ids.
 template <int U, class F>
 __device__ inline void rev_listings(const RevQueries& a, int h, int64_t q0, uint64_t marked,
-                                    int lane, int64_t w0, int64_t w1, F f) {
+                                    int lane, F f) {
   int b, bs0, nbb0;
   bool st;
   query_batch(a.cu_q, a.batch, a.cu_sb, q0, &b, &bs0, &nbb0, &st);
@@ -945,39 +989,57 @@ __device__ inline void rev_listings(const RevQueries& a, int h, int64_t q0, uint
 #pragma unroll
     for (int e = 0; e < U; ++e) {
       const int64_t c = (int64_t)bs + v[e];
-      if (v[e] >= 0 && v[e] < nbb && c >= w0 && c < w1) f(r, (i - r * units) * U + e, c);
+      if (v[e] >= 0 && v[e] < nbb && c >= 0 && c < a.nb) f((int)c);
     }
   }
 }
 
+// U: ids per load of the rows; 0: from the pairs.
 template <int U>
-__global__ __launch_bounds__(256) void rev_chunk_count_kernel(RevQueries a,
+__global__ __launch_bounds__(256) void rev_chunk_count_kernel(RevPass a,
                                                               int32_t* __restrict__ counts) {
   extern __shared__ int hist[];
-  const int h = blockIdx.y, chunk = blockIdx.x;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int64_t w0 = (int64_t)blockIdx.z * REV_WIN;
-  const int64_t w1 = w0 + REV_WIN < a.nb ? w0 + REV_WIN : a.nb;
-  for (int i = threadIdx.x; i < w1 - w0; i += blockDim.x) hist[i] = 0;
+  RevItem it;
+  if (!rev_item(a, &it)) return;
+  const int h = it.h, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int w0 = (int)blockIdx.z * REV_WIN;
+  const int nw = (int)(a.buckets - w0 < REV_WIN ? a.buckets - w0 : REV_WIN);
+  for (int i = threadIdx.x; i < nw; i += blockDim.x) hist[i] = 0;
   __syncthreads();
-  const int64_t c0 = chunk * a.chunk_len;
-  const int64_t c1 = c0 + a.chunk_len < a.nq ? c0 + a.chunk_len : a.nq;
-  for (int64_t q0 = c0 + wv * 64; q0 < c1; q0 += 256) {
-    const uint64_t m = rev_marked(a, h, q0, lane);
-    if (m)
-      rev_listings<U>(a, h, q0, m, lane, w0, w1,
-                      [&](int, int, int64_t c) { atomicAdd(&hist[c - w0], 1); });
+  auto add = [&](int c) {
+    const int x = ((c >> a.shift) & a.mask) - w0;
+    if (x >= 0 && x < nw) atomicAdd(&hist[x], 1);
+  };
+  const int64_t c0 = it.chunk * a.chunk_len;
+  if constexpr (U > 0) {
+    const int64_t c1 = c0 + a.chunk_len < a.rows.nq ? c0 + a.chunk_len : a.rows.nq;
+    for (int64_t q0 = c0 + wv * 64; q0 < c1; q0 += 256) {
+      const uint64_t m = rev_marked(a.rows, h, q0, lane);
+      if (m) rev_listings<U>(a.rows, h, q0, m, lane, add);
+    }
+  } else {
+    const int64_t n = a.n_in[h], c1 = c0 + a.chunk_len < n ? c0 + a.chunk_len : n;
+    const int2* pairs = a.pairs + (int64_t)h * a.in_cap;
+    constexpr int G = 8;  // loads in flight
+    for (int64_t i0 = c0 + threadIdx.x; i0 < c1; i0 += 256 * G) {
+      int x[G];
+#pragma unroll
+      for (int u = 0; u < G; ++u) x[u] = i0 + 256 * u < c1 ? pairs[i0 + 256 * u].x : -1;
+#pragma unroll
+      for (int u = 0; u < G; ++u)
+        if (x[u] >= 0) add(x[u]);
+    }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < w1 - w0; i += blockDim.x)
-    counts[((int64_t)h * a.nb + w0 + i) * a.n_chunks + chunk] = hist[i];
+  for (int i = threadIdx.x; i < nw; i += blockDim.x)
+    counts[((int64_t)h * a.buckets + w0 + i) * a.n_chunks + it.chunk] = hist[i];
 }
 
-// Chunk counts in (block, chunk) order -> offsets in place, and the CSR
-// offsets of the blocks.
+// Chunk counts in (bucket, chunk) order -> offsets in place, and the CSR
+// offsets of the buckets.
 struct ChunkCountF {
   const int32_t* counts;
-  int64_t per_head;  // nb * n_chunks
+  int64_t per_head;  // buckets * n_chunks
   __device__ int64_t limit(int, int64_t n) const { return n; }
   __device__ int operator()(int h, int64_t i) const { return counts[(int64_t)h * per_head + i]; }
 };
@@ -989,107 +1051,262 @@ struct ChunkOffW {
   int64_t nb;
   __device__ void operator()(int h, int64_t i, int ex, int v, int64_t lim) const {
     counts[(int64_t)h * per_head + i] = ex;
-    const int32_t c = (int32_t)i / n_chunks;  // i < REV_COUNTS + nb
+    const int32_t c = (int32_t)i / n_chunks;  // i < REV_COUNTS + buckets
     int32_t* p = cu_rev + (int64_t)h * (nb + 1);
     if (c * n_chunks == (int32_t)i) p[c] = ex;
     if (i == lim - 1) p[nb] = ex + v;
   }
 };
 
-// One wave per chunk, 64 queries at a time: every listed block collects the
-// group's queries in a 64-bit mask, so that a listing's place is the block's
-// offset plus the queries below its own in the mask.  A group in which a row
-// lists a block twice takes its listings 64 at a time in order instead.
-template <int U>
-__global__ __launch_bounds__(64) void rev_chunk_place_kernel(RevQueries a,
+// One wave per chunk.  Its listings are taken REV_STEPS x 64 at a time in
+// order; a listing's place is the bucket's offset plus the number of lower
+// lanes that hold the same bucket, found from one ballot per bit of the bucket
+// number, and the lowest lane of each bucket moves the offset past all of them
+// (rows that list a block twice cost nothing extra).  The next listings are
+// loaded before and taken in before the places of these are written, so that no
+// load waits for the scattered writes.  FIRST of two passes: pairs for the
+// second; the last (or only) pass: out [hkv, cap], what the listings store, and
+// after a first pass their blocks in `sorted` [hkv, in_cap].
+constexpr int REV_STEPS = 16;
+enum RevKind { REV_ONLY, REV_FIRST, REV_SECOND };
+template <RevKind KIND, int BITS>
+__global__ __launch_bounds__(64) void rev_chunk_place_kernel(RevPass a,
                                                              const int32_t* __restrict__ offs,
-                                                             int32_t* __restrict__ rev,
-                                                             int64_t cap, bool encode) {
-  extern __shared__ unsigned long long masks[];  // [blocks], then the offsets
-  const int h = blockIdx.y, chunk = blockIdx.x, lane = threadIdx.x;
-  const int64_t w0 = (int64_t)blockIdx.z * REV_WIN;
-  const int64_t w1 = w0 + REV_WIN < a.nb ? w0 + REV_WIN : a.nb;
-  const int nw = (int)(w1 - w0);
-  int* next = reinterpret_cast<int*>(masks + nw);
-  const int64_t c0 = chunk * a.chunk_len;
-  const int64_t c1 = c0 + a.chunk_len < a.nq ? c0 + a.chunk_len : a.nq;
-  int32_t* out = rev + (int64_t)h * cap;
-  bool ready = false;
-  for (int64_t q0 = c0; q0 < c1; q0 += 64) {
-    const uint64_t m = rev_marked(a, h, q0, lane);
-    if (!m) continue;
-    if (!ready) {  // the first marked group of the chunk
-      for (int i = lane; i < nw; i += 64) {
-        masks[i] = 0ull;
-        next[i] = offs[((int64_t)h * a.nb + w0 + i) * a.n_chunks + chunk];
-      }
-      ready = true;
-    }
-    __syncthreads();
-    bool twice = false;
-    rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int, int64_t c) {
-      twice |= (atomicOr(&masks[c - w0], 1ull << r) >> r) & 1ull;
-    });
-    __syncthreads();
-    if (!__ballot(twice)) {
-      rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int j, int64_t c) {
-        const int64_t pos =
-            next[c - w0] + __popcll(masks[c - w0] & ((1ull << r) - 1ull));
-        if (pos < cap) out[pos] = (int32_t)(encode ? (q0 + r) * a.k + j : q0 + r);
-      });
-      __syncthreads();
-      // the block's first listing moves its offset past the group
-      rev_listings<U>(a, h, q0, m, lane, w0, w1, [&](int r, int, int64_t c) {
-        const unsigned long long mm = masks[c - w0];
-        if (mm && __ffsll(mm) - 1 == r) {
-          next[c - w0] += __popcll(mm);
-          masks[c - w0] = 0ull;
-        }
-      });
-    } else {
-      rev_listings<1>(a, h, q0, m, lane, w0, w1,
-                      [&](int, int, int64_t c) { masks[c - w0] = 0ull; });
-      const int32_t* rows = a.topk + ((int64_t)h * a.nq + q0) * a.k;
-      for (int i0 = 0; i0 < 64 * a.k; i0 += 64) {  // 64 listings in order
-        const int r = (i0 + lane) / a.k;
-        int c = -1;  // this lane's block within the window
-        if ((m >> r) & 1ull) {
-          int b, bs, nbb;
-          bool st;
-          query_batch(a.cu_q, a.batch, a.cu_sb, q0 + r, &b, &bs, &nbb, &st);
-          const int v = rows[i0 + lane];
-          const int64_t cg = (int64_t)bs + v;
-          if (v >= 0 && v < nbb && cg >= w0 && cg < w1) c = (int)(cg - w0);
-        }
-        uint64_t pend = __ballot(c >= 0);
-        while (pend) {  // one block's listings at a time (wave-uniform)
-          const int l = __builtin_ctzll(pend);
-          const int cl = __builtin_amdgcn_readlane(c, l);
-          const uint64_t same = __ballot(c == cl);
-          int base = 0;
-          if (lane == l) base = atomicAdd(&next[cl], __popcll(same));
-          base = __builtin_amdgcn_readlane(base, l);
-          const int64_t pos = base + __popcll(same & ((1ull << lane) - 1ull));
-          if (c == cl && pos < cap) {
-            const int64_t q = q0 + r;
-            out[pos] = (int32_t)(encode ? q * a.k + (i0 + lane - r * a.k) : q);
-          }
-          pend &= ~same;
-        }
-      }
-    }
-    __syncthreads();
+                                                             int32_t* __restrict__ out,
+                                                             int64_t cap,
+                                                             int2* __restrict__ out_pairs,
+                                                             int32_t* __restrict__ sorted) {
+  constexpr int S = REV_STEPS;
+  constexpr bool ROWS = KIND != REV_SECOND;
+  extern __shared__ int next[];  // [buckets of the window]
+  RevItem it;
+  if (!rev_item(a, &it)) return;
+  const int h = it.h, lane = threadIdx.x;
+  const int w0 = (int)blockIdx.z * REV_WIN;
+  const int nw = (int)(a.buckets - w0 < REV_WIN ? a.buckets - w0 : REV_WIN);
+  const int64_t c0 = it.chunk * a.chunk_len;
+  const RevQueries& q = a.rows;
+  const int k = ROWS ? q.k : 1;
+  const int64_t n_in = ROWS ? q.nq : (int64_t)a.n_in[h];
+  const int64_t c1 = c0 + a.chunk_len < n_in ? c0 + a.chunk_len : n_in;
+  if (c0 >= c1) return;
+  if (ROWS && q.only) {
+    uint64_t m = 0;
+    for (int64_t q0 = c0; q0 < c1 && !m; q0 += 64) m = rev_marked(q, h, q0, lane);
+    if (!m) return;
   }
+  for (int i = lane; i < nw; i += 64)
+    next[i] = offs[((int64_t)h * a.buckets + w0 + i) * a.n_chunks + it.chunk];
+  wave_lds_order();
+  const uint32_t total = (uint32_t)((c1 - c0) * k);  // listings (n_q * topk < 2^31)
+  const int32_t* src = ROWS ? q.topk + ((int64_t)h * q.nq + c0) * k : nullptr;
+  const int2* pairs = ROWS ? nullptr : a.pairs + (int64_t)h * a.in_cap + c0;
+  const uint8_t* only = ROWS && q.only ? q.only + (int64_t)h * q.nq + c0 : nullptr;
+  out += (int64_t)h * cap;
+  out_pairs += (int64_t)h * a.in_cap;
+  sorted += (int64_t)h * a.in_cap;
+  // row and slot of a lane's listing, 64 listings further
+  const int dr = 64 / k, dj = 64 - dr * k;
+  auto advance = [&](int& r, int& j) __attribute__((always_inline)) {
+    j += dj;
+    const int over = j >= k ? 1 : 0;
+    j -= over ? k : 0;
+    r += dr + over;
+  };
+  int r_load = lane / k, j_load = lane - r_load * k, r_put = r_load, j_put = j_load;
+  const int r_last = (int)(c1 - c0) - 1;
+  int32_t v[S], w[S];  // ids (or blocks), and what the listings store
+  uint8_t mk[S];
+  auto load = [&](uint32_t base) __attribute__((always_inline)) {  // (past the end: the last one)
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const uint32_t i = base + s * 64 + lane;
+      if constexpr (ROWS) {
+        v[s] = src[i < total ? i : total - 1];
+      } else {
+        const int2 p = pairs[i < total ? i : total - 1];
+        v[s] = p.x;
+        w[s] = p.y;
+      }
+      mk[s] = 1;
+    }
+    if (only) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        mk[s] = only[r_load < r_last ? r_load : r_last];
+        advance(r_load, j_load);
+      }
+    }
+  };
+  // The batch element at hand: its listings [i_lo, i_hi) of the chunk, its blocks.
+  int b = 0, bs = 0, nbb = 0;
+  int64_t i_lo = 0, i_hi = 0;
+  auto element = [&]() {
+    i_lo = ((int64_t)q.cu_q[b] - c0) * k;
+    i_hi = ((int64_t)q.cu_q[b + 1] - c0) * k;
+    bs = q.cu_sb[b];
+    nbb = q.cu_sb[b + 1] - bs;
+  };
+  if constexpr (ROWS) {
+    b = batch_of(q.cu_q, q.batch, c0);
+    element();
+  }
+  int blk[S], val[S];  // the listings' blocks (-1: none), and what they store
+  auto take = [&](uint32_t base) __attribute__((always_inline)) {
+    const uint32_t end = base + S * 64 < total ? base + S * 64 : total;
+    if constexpr (!ROWS) {
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        blk[s] = base + s * 64 + lane < end ? v[s] : -1;
+        val[s] = w[s];
+      }
+      return;
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) blk[s] = -1;
+    for (;;) {
+      const uint32_t lo = i_lo > 0 ? (uint32_t)(i_lo < end ? i_lo : end) : 0u;
+      const uint32_t hi = i_hi > 0 ? (uint32_t)(i_hi < end ? i_hi : end) : 0u;
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        const uint32_t i = base + s * 64 + lane;
+        const int64_t c = (int64_t)bs + v[s];
+        if (i >= lo && i < hi && mk[s] && v[s] >= 0 && v[s] < nbb && c >= 0 && c < q.nb)
+          blk[s] = (int)c;
+      }
+      if (i_hi >= end || b + 1 >= q.batch) break;  // the last element of these listings
+      ++b;
+      element();
+    }
+  };
+  load(0);
+  take(0);
+  for (uint32_t base = 0; base < total; base += S * 64) {
+    load(base + S * 64);
+    int pos[S], key[S], put[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      const int x = ((blk[s] >> a.shift) & a.mask) - w0;
+      const bool in = blk[s] >= 0 && x >= 0 && x < nw;
+      const uint64_t same = __ballot(in);
+      uint32_t lo = (uint32_t)same, hi = (uint32_t)(same >> 32);
+#pragma unroll
+      for (int i = 0; i < BITS; ++i) {
+        const int on = (x << (31 - i)) >> 31;  // all ones where bit i is set
+        const uint64_t m = __ballot(on != 0);
+        lo &= ~((uint32_t)m ^ (uint32_t)on);
+        hi &= ~((uint32_t)(m >> 32) ^ (uint32_t)on);
+      }
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, 0u));
+      int at = 0;
+      if (in) at = next[x];
+      wave_lds_order();
+      if (in && rank == 0) next[x] = at + __popc(lo) + __popc(hi);
+      wave_lds_order();
+      pos[s] = in ? at + rank : -1;
+      key[s] = blk[s];
+      if constexpr (ROWS) {
+        put[s] = q.encode ? (int)(c0 * k + base + s * 64 + lane) : (int)(c0 + r_put);
+        advance(r_put, j_put);
+      } else {
+        put[s] = val[s];
+      }
+    }
+    take(base + S * 64);
+    // the loads end here, ahead of the writes
+#pragma unroll
+    for (int s = 0; s < S; ++s) asm volatile("" : "+v"(blk[s]));
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+      if constexpr (KIND == REV_FIRST) {
+        if (pos[s] >= 0) out_pairs[pos[s]] = make_int2(key[s], put[s]);
+      } else {
+        if (pos[s] >= 0 && pos[s] < cap) out[pos[s]] = put[s];
+        if (KIND == REV_SECOND && pos[s] >= 0) sorted[pos[s]] = key[s];
+      }
+    }
+  }
+}
+
+// Offsets of the blocks in each head's sorted listings: one thread per block, a
+// binary search.
+__global__ __launch_bounds__(256) void rev_offsets_kernel(const int32_t* __restrict__ sorted,
+                                                          int64_t in_cap,
+                                                          const int32_t* __restrict__ n_in,
+                                                          int64_t nb, int32_t* __restrict__ cu_rev) {
+  const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int h = blockIdx.y;
+  if (c > nb) return;
+  const int32_t* p = sorted + (int64_t)h * in_cap;
+  int64_t lo = 0, hi = n_in[h];  // answer in [lo, hi]
+  while (lo < hi) {
+    const int64_t mid = (lo + hi) >> 1;
+    if (p[mid] < c)
+      lo = mid + 1;
+    else
+      hi = mid;
+  }
+  cu_rev[(int64_t)h * (nb + 1) + c] = (int32_t)lo;
+}
+
+// Counts, scans and places one pass (chunks as rev_chunks gives them).
+template <RevKind KIND>
+int run_rev_pass(RevPass a, const RevChunks& ch, int32_t* counts, int32_t* sums, int32_t* cu,
+                 int32_t* totals, int32_t* out, int64_t cap, int2* out_pairs, int32_t* sorted,
+                 hipStream_t st) {
+  a.chunk_len = ch.len;
+  a.n_chunks = (int)ch.n;
+  const int64_t win = std::min<int64_t>(a.buckets, REV_WIN), per_head = a.buckets * ch.n;
+  const dim3 grid((unsigned)((ch.n * a.hkv + 7) / 8 * 8), 1, (unsigned)ceil_div(a.buckets, REV_WIN));
+  const size_t lds = (size_t)win * sizeof(int);
+  const bool vec = a.rows.k % 4 == 0 && ((uintptr_t)a.rows.topk % 16) == 0;
+  const auto count = KIND == REV_SECOND
+                         ? rev_chunk_count_kernel<0>
+                         : (vec ? rev_chunk_count_kernel<4> : rev_chunk_count_kernel<1>);
+  hipLaunchKernelGGL(count, grid, dim3(256), lds, st, a, counts);
+  LSRM_CHECK_LAUNCH();
+  const int rc = run_scan(ChunkCountF{counts, per_head},
+                          ChunkOffW{counts, per_head, a.n_chunks, cu, a.buckets}, per_head, a.hkv,
+                          sums, totals, st);
+  if (rc) return rc;
+  // the instantiation for the next larger number of bits of a bucket in a window
+  const auto place = win <= 16     ? rev_chunk_place_kernel<KIND, 4>
+                     : win <= 64   ? rev_chunk_place_kernel<KIND, 6>
+                     : win <= 128  ? rev_chunk_place_kernel<KIND, 7>
+                     : win <= 256  ? rev_chunk_place_kernel<KIND, 8>
+                     : win <= 512  ? rev_chunk_place_kernel<KIND, 9>
+                     : win <= 1024 ? rev_chunk_place_kernel<KIND, 10>
+                     : win <= 4096 ? rev_chunk_place_kernel<KIND, 12>
+                                   : rev_chunk_place_kernel<KIND, 13>;
+  static_assert(REV_WIN <= 1 << 13, "a bucket's number in a window has 13 bits");
+  hipLaunchKernelGGL(place, grid, dim3(64), lds, st, a, counts, out, cap, out_pairs, sorted);
+  LSRM_CHECK_LAUNCH();
+  return LSRM_OK;
 }
 
 int build_query_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq, int64_t topk_n,
                             const int32_t* cu_q, int64_t batch, const int32_t* cu_sb,
                             int64_t nb, Carver& ws, RevMap& map, hipStream_t st,
                             const uint8_t* only, bool encode_slot) {
-  const RevChunks ch = rev_chunks(hkv, nq, nb);
-  const int64_t per_head = (nb > 0 ? nb : 1) * ch.n;
+  const bool two = !rev_one_pass(hkv * nq * topk_n, nb);
+  int shift = 0;  // bits of the first of two passes: half of the block number's
+  while (two && ((int64_t)1 << (2 * shift)) < nb) ++shift;
+  const int64_t n = nq * topk_n > 0 ? nq * topk_n : 1;  // listings per head, at most
+  const int64_t buckets[2] = {two ? int64_t{1} << shift : (nb > 0 ? nb : 1),
+                              two ? (nb + (int64_t{1} << shift) - 1) >> shift : 1};
+  const RevChunks ch[2] = {rev_chunks(!two, hkv, nq, 64, buckets[0]),
+                           rev_chunks(!two, hkv, two ? n : 1, REV_STEPS * 64, buckets[1])};
+  const int64_t per_head = std::max(buckets[0] * ch[0].n, buckets[1] * ch[1].n);
   int32_t* counts = ws.take<int32_t>((size_t)(hkv * per_head));
   int32_t* sums = ws.take<int32_t>((size_t)scan_sums_size(per_head, hkv));
+  int32_t *cu = nullptr, *n_in = nullptr, *sorted = nullptr;
+  int2* pairs = nullptr;
+  if (two) {
+    cu = ws.take<int32_t>((size_t)(hkv * (std::max(buckets[0], buckets[1]) + 1)));
+    n_in = ws.take<int32_t>((size_t)hkv);
+    pairs = ws.take<int2>((size_t)(hkv * n));
+    sorted = ws.take<int32_t>((size_t)(hkv * n));
+  }
   if (!map.cu_rev) map.cu_rev = ws.take<int32_t>((size_t)(hkv * (nb + 1)));
   if (!map.rev) map.rev = ws.take<int32_t>((size_t)(hkv * (map.cap > 0 ? map.cap : 1)));
   if (!map.totals) map.totals = ws.take<int32_t>((size_t)hkv);
@@ -1100,26 +1317,29 @@ int build_query_reverse_map(const int32_t* topk, int64_t hkv, int64_t nq, int64_
     if (rc) return rc;
     return launch_zero_i32(map.totals, hkv, st);
   }
-  const RevQueries a{topk, nq,   (int)topk_n, cu_q, batch,
-                     cu_sb, nb, only,        ch.len, (int)ch.n};
-  const dim3 grid((unsigned)ch.n, (unsigned)hkv, (unsigned)ceil_div(nb, REV_WIN));
-  const size_t win = (size_t)std::min<int64_t>(nb, REV_WIN);
-  const bool vec = topk_n % 4 == 0 && ((uintptr_t)topk % 16) == 0;
-  if (vec)
-    hipLaunchKernelGGL(rev_chunk_count_kernel<4>, grid, dim3(256), win * 4, st, a, counts);
-  else
-    hipLaunchKernelGGL(rev_chunk_count_kernel<1>, grid, dim3(256), win * 4, st, a, counts);
-  LSRM_CHECK_LAUNCH();
-  const int rc = run_scan(ChunkCountF{counts, per_head},
-                          ChunkOffW{counts, per_head, (int)ch.n, map.cu_rev, nb}, per_head,
-                          (int)hkv, sums, map.totals, st);
+  RevPass a{};
+  a.rows = RevQueries{topk, nq, (int)topk_n, cu_q, batch, cu_sb, nb, only, encode_slot};
+  a.in_cap = n;
+  a.hkv = (int)hkv;
+  a.buckets = buckets[0];
+  if (!two) {
+    a.mask = INT32_MAX;
+    return run_rev_pass<REV_ONLY>(a, ch[0], counts, sums, map.cu_rev, map.totals, map.rev, map.cap,
+                                  nullptr, nullptr, st);
+  }
+  a.mask = (int)buckets[0] - 1;
+  int rc = run_rev_pass<REV_FIRST>(a, ch[0], counts, sums, cu, n_in, nullptr, 0, pairs, nullptr, st);
   if (rc) return rc;
-  if (vec)
-    hipLaunchKernelGGL(rev_chunk_place_kernel<4>, grid, dim3(64), win * 12, st, a, counts,
-                       map.rev, map.cap, encode_slot);
-  else
-    hipLaunchKernelGGL(rev_chunk_place_kernel<1>, grid, dim3(64), win * 12, st, a, counts,
-                       map.rev, map.cap, encode_slot);
+  a.pairs = pairs;
+  a.n_in = n_in;
+  a.shift = shift;
+  a.mask = INT32_MAX;
+  a.buckets = buckets[1];
+  rc = run_rev_pass<REV_SECOND>(a, ch[1], counts, sums, cu, map.totals, map.rev, map.cap, nullptr,
+                                sorted, st);
+  if (rc) return rc;
+  hipLaunchKernelGGL(rev_offsets_kernel, dim3(ceil_div(nb + 1, 256), (unsigned)hkv), dim3(256), 0,
+                     st, sorted, n, map.totals, nb, map.cu_rev);
   LSRM_CHECK_LAUNCH();
   return LSRM_OK;
 }
