@@ -293,10 +293,9 @@ int lsrm_sel_attn_fwd_run(const void* q, const void* k, const void* v,
  * plan's flags runs the key-centric pass.  head_dim sizes the partials and
  * sets which blocks the forward keeps whole in LDS (up to 512 keys at
  * head_dim <= 64, 256 above), so the runs pass the plan's head_dim like its
- * other inputs.  Without LSRM_PLAN_KEY_CENTRIC a plan serves every head_dim;
- * one given a head_dim above 32 does not list its short tiles apart for the
- * kernels at 32, which then run them as other tiles (results agree to the
- * order of fp32 sums).
+ * other inputs.  Without LSRM_PLAN_KEY_CENTRIC a plan serves every head_dim:
+ * short tiles that it does not list apart for the kernels at head_dim 32 run
+ * as other tiles there (results agree to the order of fp32 sums).
  * Replaces: ..._impl_kvcentric.py:931-1010 for per-token rows (the
  * reference has no key-centric forward; the queries of a block are the
  * reverse map of 575-684, which its backward builds).

@@ -48,6 +48,7 @@ struct AttnArgs {
   KeyItems items;    // backward: key chunks of every block
   KcPlan kc;         // key-centric plans only (kc.fitems null otherwise)
   int32_t kc_marker; // kc_plan_marker of the flags and head dim of this run
+  bool narrow;       // narrow run tiles run apart (narrow_tiles)
 };
 
 // A key-centric kernel runs only on a plan whose key-centric part was built
@@ -692,15 +693,37 @@ __device__ inline uint32_t group_offset(const SelLds& s, GroupCursor& c, int P,
 // at 32 / 2 heads of 32, 26600 run tiles per kv head).  Whole forward passes
 // over 98304 queries at 32 / 2 heads, runs of equal top-16 rows, as run tiles
 // and with their narrow tiles split: tiles of 32 rows 1.71 -> 1.46 ms over
-// blocks of 24 keys and 10.4 -> 10.7 over blocks of 246 (equal within the
-// runs' spread); tiles of 48 rows, two waves per row block, 1.20 -> 1.06 and
-// 7.0 -> 9.1; of 64 rows 0.92 -> 0.83 and 5.3 -> 6.9.  So the line lies at one
-// row block (NARROW_ROWS); wider tiles run as run tiles.  At head dim 64 a run
+// blocks of 24 keys and 10.4 -> 10.7 over blocks of 246; tiles of 48 rows, two
+// waves per row block, 1.20 -> 1.06 and 7.0 -> 9.1; of 64 rows 0.92 -> 0.83 and
+// 5.3 -> 6.9.  So the line lies at one row block (NARROW_ROWS); wider tiles run
+// as run tiles, and narrow_tiles has the other lines.  At head dim 64 a run
 // tile's K and V traffic sets its time whatever its rows, and the run-tile
 // kernels move it with wider requests: 454 blocks of 32..512 queries at 24
 // heads took 9.1 ms as run tiles, 10.3 ms split by width (9.2 with the stream
 // in LDS).
 constexpr bool narrow_split(int d) { return d <= 32; }
+
+// Whether the narrow run tiles are listed and run apart (at a head dim with
+// kernels for them; otherwise they run as the other run tiles do).
+//   - Key-centric plans: rows of neighbouring queries list mostly the same
+//     blocks, whose keys the L2 holds (3D-aware rows of 122880 tokens, streams
+//     of 3900 keys: forward 3.69 -> 3.28 ms, dQ 5.11 -> 3.34).
+//   - Other plans: for mean streams of 256 keys up to what the token map holds.
+//     Runs of equal top-16 rows as run tiles and split, forward / whole backward
+//     in us: 131072 queries at 2 / 2 heads in runs of 16, blocks of 8 keys 211 /
+//     913 -> 219 / 917, of 24 keys 271 / 1003 -> 227 / 934, of 96 keys 560 / 1636
+//     -> 520 / 1418, of 128 keys 732 / 1834 -> 748 / 1661, of 246 keys 1669 / 3182
+//     -> 1678 / 3218; 98304 queries at 32 / 2 heads in runs of 2 over blocks of
+//     900 keys 42.8 / 75.1 -> 43.8 / 76.0 ms.
+//   - And where short tiles are likely or the launch is little: an empty one
+//     costs 2 us (1024 / 4096 queries at 2 heads in blocks of 64: forward 23.0 /
+//     28.4 -> 25.0 / 30.0 us), so with blocks of more than 48 rows on average
+//     only from 2^18 rows on (forward passes of 75 us and more).
+inline bool narrow_tiles(bool key_centric, int64_t hkv, int64_t g, int64_t nq, int64_t nk,
+                         int64_t nb, int64_t topk_n) {
+  return key_centric || (nk * topk_n >= 256 * nb && nk * topk_n <= KMAP_KEYS * nb &&
+                         (nq * g <= 48 * nb || hkv * nq * g >= (int64_t{1} << 18)));
+}
 
 // One wave's walk over its 32-key blocks of a narrow tile's stream.
 template <int D>

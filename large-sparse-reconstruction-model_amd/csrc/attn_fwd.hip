@@ -314,10 +314,11 @@ sel_attn_fwd_kernel(AttnArgs a) {
   const int hb = lane >> 5, l32 = lane & 31;
   // head dims with a narrow-tile kernel leave the narrow run tiles to it
   constexpr bool WIDE = MODE == FWD_RUN && narrow_split(D);
+  // (all tiles where the plan does not list them apart, or this run does not)
+  const bool by_width = WIDE && a.narrow && a.plan.counter[BY_WIDTH_SLOT] != 0;
   const int32_t* head_off =
       GATHER ? a.kc.fitem_off
-             : (UNION ? a.plan.ghead_off : (WIDE ? a.plan.wide_off : a.plan.head_off));
-  const bool by_width = WIDE && a.plan.counter[BY_WIDTH_SLOT] != 0;  // else wide_off is head_off
+             : (UNION ? a.plan.ghead_off : (by_width ? a.plan.wide_off : a.plan.head_off));
   const int2* tiles = UNION ? a.plan.gtiles : (by_width ? a.plan.by_width : a.plan.tiles);
   int32_t* queue = a.plan.counter + (GATHER ? KC_QUEUE_SLOT : (UNION ? 4 : 0));
   if constexpr (GATHER) {
@@ -1365,11 +1366,13 @@ __global__ __launch_bounds__(256) void kc_merge_kernel(AttnArgs a) {
 template <int DT, int D>
 int launch_fwd_t(const AttnArgs& a, hipStream_t st) {
   if constexpr (narrow_split(D)) {
-    const int grid =
-        persistent_grid(reinterpret_cast<const void*>(&narrow_fwd_kernel<DT, D>), 256, 0);
-    if (grid <= 0) return LSRM_ERR_LAUNCH;
-    hipLaunchKernelGGL((narrow_fwd_kernel<DT, D>), dim3(grid), dim3(256), 0, st, a);
-    LSRM_CHECK_LAUNCH();
+    if (a.narrow) {
+      const int grid =
+          persistent_grid(reinterpret_cast<const void*>(&narrow_fwd_kernel<DT, D>), 256, 0);
+      if (grid <= 0) return LSRM_ERR_LAUNCH;
+      hipLaunchKernelGGL((narrow_fwd_kernel<DT, D>), dim3(grid), dim3(256), 0, st, a);
+      LSRM_CHECK_LAUNCH();
+    }
   }
   const void* fn = reinterpret_cast<const void*>(&sel_attn_fwd_kernel<DT, D, FWD_RUN>);
   const int grid = persistent_grid(fn, 256, 0);

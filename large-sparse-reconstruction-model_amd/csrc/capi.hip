@@ -109,7 +109,11 @@ int attn_plan(Carver& ws, const int32_t* topk, int64_t nq, int64_t nk,
   // Run tiles are listed by width for the head dims whose kernels read that
   // list (0: not known yet).  The list is carved for all of them, since plans
   // without the key-centric part serve every head dim.
-  const int narrow_q = narrow_split((int)head_dim) ? NARROW_ROWS / g : 0;
+  const int narrow_q = narrow_split((int)head_dim) &&
+                               narrow_tiles((flags & LSRM_PLAN_KEY_CENTRIC) != 0, hkv, g, nq, nk,
+                                            nb, topk_n)
+                           ? NARROW_ROWS / g
+                           : 0;
   int rc = build_tile_plan(topk, hkv, nq, topk_n, cu_q, batch, cu_sb, tq, narrow_q, ws, w.plan,
                            st);
   if (rc) return rc;
@@ -321,6 +325,7 @@ int attn_setup(const void* q, const void* k, const void* v, int dtype,
   a.items = w.items;
   a.kc = w.kc;
   a.kc_marker = kc_plan_marker(flags, (int)head_dim);
+  a.narrow = narrow_tiles((flags & LSRM_PLAN_KEY_CENTRIC) != 0, hkv, g, n_q, n_k, n_blocks, topk);
   return LSRM_OK;
 }
 
