@@ -686,6 +686,9 @@ __global__ __launch_bounds__(256) void pool_pieces_small(
     int64_t nb, float* __restrict__ partial_a, const void* __restrict__ xb,
     float* __restrict__ partial_b) {
   constexpr int E = DT == LSRM_F32 ? 1 : 2;  // channels per word
+  constexpr int SKIP = 8;                    // rows passed over at once
+  constexpr int FEW = 4;                     // rows taken by register number
+  typedef uint32_t u32x32 __attribute__((ext_vector_type(32)));
   const int lane = threadIdx.x & 63;
   const uint32_t wpc = (uint32_t)(ch / (64 * E));  // waves per chunk
   const uint32_t n_waves = (uint32_t)((n + POOL_CHUNK - 1) / POOL_CHUNK) * wpc;
@@ -699,10 +702,11 @@ __global__ __launch_bounds__(256) void pool_pieces_small(
   const int64_t r1 = r0 + POOL_CHUNK < n ? r0 + POOL_CHUNK : n;
   const uint32_t* xp = reinterpret_cast<const uint32_t*>(second ? xb : xa) + (r0 * ch + c0) / E;
   float* partial = second ? partial_b : partial_a;
-  uint32_t w[POOL_CHUNK];
+  static_assert(POOL_CHUNK == 64, "two vectors of 32 rows");
+  u32x32 w[2];
 #pragma unroll
   for (int u = 0; u < POOL_CHUNK; ++u)
-    w[u] = __builtin_nontemporal_load(xp + (r0 + u < r1 ? u : r1 - 1 - r0) * (ch / E));
+    w[u / 32][u % 32] = __builtin_nontemporal_load(xp + (r0 + u < r1 ? u : r1 - 1 - r0) * (ch / E));
   // b = last block whose start is <= r0 (-1: before the first block, nb: past
   // the last): a two-level count of the nondecreasing offsets.
   const int64_t S = (nb + 64) / 64;
@@ -719,54 +723,78 @@ __global__ __launch_bounds__(256) void pool_pieces_small(
     }
     b = base + cnt - 1;
   }
-  // Lane l holds the end of block wb + l (the start of the next one).
+  // Lane l holds the end of block wb + l (the start of the next one; none past
+  // the last).
   int64_t wb = b;
-  int32_t ends = cu[b + 1 + lane < nb ? b + 1 + lane : nb];
-  auto end_of = [&](int64_t blk) __attribute__((always_inline)) -> int64_t {
-    if (blk >= nb) return INT64_MAX;
-    if (blk - wb >= 64) {
-      wb = blk;
-      ends = cu[blk + 1 + lane < nb ? blk + 1 + lane : nb];
-    }
-    return __builtin_amdgcn_readlane(ends, (int)(blk - wb));
+  auto load_ends = [&]() __attribute__((always_inline)) -> int32_t {
+    return wb + 1 + lane <= nb ? cu[wb + 1 + lane] : INT32_MAX;
   };
+  int32_t ends = load_ends();
   // Block by block: the rows [lo, hi) of the chunk that block b owns, added in
   // order (the row tests are scalar; one copy of the adds keeps the kernel
-  // small, since its instructions are fetched anew by every launch).
+  // small, since its instructions are fetched anew by every launch).  A few rows
+  // are taken by their register's number, of others SKIP are passed over at
+  // once, and blocks without rows all together.  4096 x 256 bf16 rows in blocks
+  // of 1 / 2 / 8 / 64 rows: 31 / 20 / 12 / 8.7 us, with a test per row and block
+  // 84 / 45 / 17 / 8.4, in the 256-channel kernel 39 / 27 / 16 / 11; with 50000
+  // empty blocks 27, taken one by one 313, in the 256-channel kernel 342.
   int64_t lo = 0;
   for (;; ++b) {
-    const int64_t be = end_of(b);
-    const int64_t hi = (be < r1 ? be : r1) - r0;
-    if (b >= nb) break;
-    if (hi > lo) {
-      if (b >= 0) {
-        const int l = (int)lo, e = (int)hi;
-        float acc[E];
-#pragma unroll
-        for (int i = 0; i < E; ++i) acc[i] = 0.0f;
-#pragma unroll
-        for (int u = 0; u < POOL_CHUNK; ++u) {
-          if (u < l || u >= e) continue;
-          if constexpr (E == 1) {
-            acc[0] = acc[0] + __uint_as_float(w[u]);
-          } else {
-            acc[0] = acc[0] + to_f32<DT>((uint16_t)(w[u] & 0xffffu));
-            acc[E - 1] = acc[E - 1] + to_f32<DT>((uint16_t)(w[u] >> 16));
-          }
-        }
-        float* dst = partial + (b + j) * ch + c0;
-#pragma unroll
-        for (int i = 0; i < E; ++i) dst[i] = acc[i];
+    // the first block that ends behind row lo
+    for (;;) {
+      if (b - wb >= 64) {
+        wb = b;
+        ends = load_ends();
       }
-      lo = hi;
+      const uint64_t behind = __ballot(ends > (int32_t)(r0 + lo)) >> (b - wb);
+      if (behind) {
+        b += __builtin_ctzll(behind);
+        break;
+      }
+      b = wb + 64;
     }
+    if (b >= nb) break;
+    const int64_t be = __builtin_amdgcn_readlane(ends, (int)(b - wb));
+    const int64_t hi = (be < r1 ? be : r1) - r0;
+    if (b >= 0) {
+      const int l = (int)lo, e = (int)hi;
+      float acc[E];
+#pragma unroll
+      for (int i = 0; i < E; ++i) acc[i] = 0.0f;
+      auto add = [&](uint32_t x) __attribute__((always_inline)) {
+        if constexpr (E == 1) {
+          acc[0] = acc[0] + __uint_as_float(x);
+        } else {
+          acc[0] = acc[0] + to_f32<DT>((uint16_t)(x & 0xffffu));
+          acc[E - 1] = acc[E - 1] + to_f32<DT>((uint16_t)(x >> 16));
+        }
+      };
+      if (e - l <= FEW) {  // rows by their register's number
+        for (int u = l; u < e; ++u) add(u < 32 ? w[0][u] : w[1][u - 32]);
+      } else {
+        const uint64_t rows = (~0ull >> (64 - (e - l))) << l;  // e > l
+#pragma unroll
+        for (int u0 = 0; u0 < POOL_CHUNK; u0 += SKIP) {
+          if (((rows >> u0) & ((1u << SKIP) - 1)) == 0) continue;
+#pragma unroll
+          for (int u = u0; u < u0 + SKIP; ++u)
+            if ((rows >> u) & 1) add(w[u / 32][u % 32]);
+        }
+      }
+      float* dst = partial + (b + j) * ch + c0;
+#pragma unroll
+      for (int i = 0; i < E; ++i) dst[i] = acc[i];
+    }
+    lo = hi;
     if (be >= r1) break;
   }
 }
 
 // Whether pool_pieces_small takes NT tensors of these rows: whole 256-byte
-// pieces and at most POOL_SMALL_WAVES waves.  Beyond that the byte rate decides
-// and the wider kernels are faster (8 bytes in flight per lane and byte read).
+// pieces and at most POOL_SMALL_WAVES waves.  At that line it is still ahead:
+// blocks of 283 rows, 65536 x 256 bf16 18.3 -> 11.8 us, 16384 x 1024 fp16 21.7 ->
+// 12.1, 131072 x 64 fp32 38.7 -> 10.8; the wider kernels keep the launches of
+// more than one round of its waves.
 bool small_pool(const void* x, int x_dtype, int64_t n, int64_t ch, int nt) {
   const int64_t row_bytes = ch * (x_dtype == LSRM_F32 ? 4 : 2);
   return n > 0 && row_bytes % 256 == 0 && ((uintptr_t)x % 4) == 0 &&
