@@ -546,8 +546,8 @@ __global__ __launch_bounds__(256) void topk_wave_kernel(
 // scan of the row per pick); 4 x 8192 rows, top-64, 1.38 and 1.57 (2.45, 34.8).
 // Bound by reading the scores once (the row's arithmetic is a third of that):
 // 4 x 4881 rows of 4881 scores, top-32, 465 us with four waves per row that
-// each listed their quarter's best, 286 us here (763 MB of scores read and 268 MB of
-// token rows written: 3.6 TB/s).
+// each listed their quarter's best, 306 us here (763 MB of scores read and 268 MB of
+// token rows written: 3.4 TB/s).
 constexpr int BOUND_CAP = 1024;
 
 template <int NM>

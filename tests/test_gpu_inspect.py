@@ -25,13 +25,11 @@ def _expected(rows, cu_q, cu_sb):
     return bits, int((rows[:, 1:] != rows[:, :-1]).any(-1).sum())
 
 
-@pytest.mark.parametrize("k", [1, 3, 4, 8, 12, 16, 32, 64, 128, 256])
-@pytest.mark.parametrize("n", [1, 2, 65, 513, 1030, 25037])
+# (25037 rows of 256 ids: more than one pass of the bounded grid)
+@pytest.mark.parametrize("k,n", [(k, n) for k in (1, 3, 4, 8, 12, 16, 32, 64, 128, 256)
+                                 for n in (1, 2, 65, 513, 1030)] + [(256, 25037)])
 @pytest.mark.parametrize("bad", ["none", "prefix", "empty", "unaligned"])
 def test_inspect_matches_row_by_row(k, n, bad):
-    # 25037 rows of 256 ids: more than one pass of the bounded grid
-    if n == 25037 and k != 256:
-        pytest.skip("one pass of the grid")
     gen = torch.Generator().manual_seed(k * 10007 + n)
     hkv, nb = 2, 300
     split = n // 3  # two batch elements, the boundary inside a wave's rows

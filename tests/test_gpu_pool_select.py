@@ -250,8 +250,8 @@ def test_select_ties_lowest_index():
         assert compact[:, b].tolist() == [expect, expect]
 
 
-def test_select_split_path_bitexact():
-    # More than 2048 blocks per batch element: the four-wave split selection
+def test_select_bounded_path_bitexact():
+    # More than 2048 blocks: rows selected behind a bound from class maxima
     # (cfg5's heavy-tailed blocks with near-tie scores, forced ids).
     w = W.config(5, n=262144, heads=2)
     assert 2048 < w.n_blocks <= 8192
@@ -260,7 +260,7 @@ def test_select_split_path_bitexact():
     np.testing.assert_array_equal(topk_idx, expand_per_token(ref, w.cu_block_tokens.numpy(), w.n))
 
 
-def test_select_split_path_ties_and_nan():
+def test_select_bounded_path_ties_and_nan():
     # 2200 one-token blocks whose keys are equal (every score ties: the
     # lowest ids win) except one NaN block (ranked last).
     n, d, topk = 2200, 64, 5
@@ -285,7 +285,7 @@ def test_select_split_path_ties_and_nan():
 def test_select_threshold_pass_and_fallback(nb, topk, pattern):
     # One-token blocks, so the pooled queries are the queries themselves, and
     # pooled keys given directly: 1500 blocks take the one-wave top-k, 4881
-    # the four-wave split.  "lane_periodic" scores depend on id % 64 only
+    # the one behind a bound.  "lane_periodic" scores depend on id % 64 only
     # (eight tie classes), so each lane holds candidates of one score and the
     # threshold pass has far more than 64 survivors (the exact fallback runs);
     # "sorted" scores grow with the id; topk 64 leaves no lane-best threshold.
@@ -335,7 +335,7 @@ def test_select_blocks_outside_every_batch_element(n_blocks, topk):
     # cu_seqblocks[-1] < n_blocks: the trailing blocks belong to no batch
     # element, so their tokens' rows must be -1 (the output is allocated
     # uninitialised, over memory pre-filled with valid-looking ids).  The
-    # three sizes take the wave, split and workgroup top-k kernels.
+    # three sizes take the wave, bounded and workgroup top-k kernels.
     rng = np.random.default_rng(n_blocks + topk)
     sizes = rng.integers(1, 6, size=n_blocks)
     cu_np = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
